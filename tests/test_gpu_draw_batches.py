@@ -1,0 +1,50 @@
+"""Draws in large batches against the same requests in small ones.
+
+A request's accepted point, candidate count and J f follow from its process,
+energy and stream id alone, so a batch of any size must return bit for bit what
+calls of a few requests return (those are compared with the oracle in
+test_gpu_draw.py).
+"""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+from petite_amd.constants import all_process_code
+from petite_amd.device import DeviceContext
+from petite_amd.tables import MaterialTables
+
+SEED = 77
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    return DeviceContext(MaterialTables("lead"), 0.010)
+
+
+def _draw(ctx, proc, E, sid, noalloc=False):
+    x, t, w, _ = ctx.draw(proc, E, sid, SEED, noalloc=noalloc)
+    return x.cpu().numpy(), t.cpu().numpy(), w.cpu().numpy()
+
+
+def _pieces(ctx, proc, E, sid, size):
+    parts = [_draw(ctx, proc[i:i + size], E[i:i + size], sid[i:i + size]) for i in range(0, len(E), size)]
+    return [np.concatenate(c) for c in zip(*parts)]
+
+
+# a block hands out the slots of 2,048 requests: its edges, and codes without a map
+@pytest.mark.parametrize("noalloc", [False, True])
+@pytest.mark.parametrize("n", [1, 255, 257, 2047, 2048, 2049, 6145])
+def test_request_slots(ctx, n, noalloc):
+    rng = np.random.default_rng(n)
+    proc = rng.choice([0, 0, 0, 1, 2, 2, 3, 4, 5, 9, -1, 12], size=n).astype(np.int32)  # 9: no dark map here
+    E = np.exp(rng.uniform(np.log(0.02), np.log(80.0), n))
+    sid = rng.integers(0, 2 ** 62, n)
+    x, t, w = _draw(ctx, proc, E, sid, noalloc)
+    has = (proc >= 0) & (proc <= 5)
+    assert np.all(t[has] > 0) and np.all(t[~has] == 0) and np.all(w[~has] == 0.0)
+    xs, ts, ws = _pieces(ctx, proc, E, sid, 97)
+    assert np.array_equal(t, ts)
+    assert np.array_equal(w, ws)
+    assert np.array_equal(x[has], xs[has])
