@@ -158,9 +158,10 @@ __device__ inline void block_stat_add(const unsigned long long (&v)[N], unsigned
 }
 
 // Hands out request indices to the lanes in ``need`` from wave-private
-// chunks of CH consecutive indices (one atomic per chunk).
-template <int CH>
+// chunks of ``chunk`` consecutive indices (one atomic per chunk); a take asks
+// for at most ``chunk`` of them.
 struct WaveQueue {
+  int chunk = 64;
   int64_t cur = 0, end = 0;
   __device__ inline int64_t take(unsigned long long need_mask, bool need, unsigned long long* counter) {
     const int lane = threadIdx.x & 63;
@@ -168,7 +169,7 @@ struct WaveQueue {
     const int64_t avail = end - cur;
     unsigned long long nb = 0;
     if (avail < n) {
-      if (lane == 0) nb = atomicAdd(counter, (unsigned long long)CH);
+      if (lane == 0) nb = atomicAdd(counter, (unsigned long long)chunk);
       nb = shfl_u64(nb, 0);
     }
     int64_t r = -1;
@@ -178,7 +179,7 @@ struct WaveQueue {
     }
     if (avail < n) {
       cur = (int64_t)nb + (n - avail);
-      end = (int64_t)nb + CH;
+      end = (int64_t)nb + chunk;
     } else {
       cur += n;
     }
@@ -256,19 +257,24 @@ __device__ inline double candidate_w(const DevTables& T, double E, const float* 
 // refills less often than a single lane, and larger G cuts the latency of
 // sweeps with fewer requests than lanes.
 template <int p>
-__device__ void draw_loop(const DevTables& T, const DrawLaunch& io, uint64_t seed, const int64_t count, const int lgG) {
+__device__ void draw_loop(const DevTables& T, const DrawLaunch& io, uint64_t seed, const int64_t count, int lgG, int blocks) {
   constexpr int ND = proc_ndim<p>();
   const int lane = threadIdx.x & 63;
-  const int G = 1 << lgG;
-  const int gl = lane & (G - 1);
-  const int g0 = lane - gl;
-  const unsigned long long gmask = (G == 64) ? ~0ull : (((1ull << G) - 1ull) << g0);
+  int G = 1 << lgG;
+  int gl = lane & (G - 1);
+  int g0 = lane - gl;
   const PetiteGridDesc& gd = T.d->grid[p];
   const int32_t ninc[4] = {gd.ninc[0], gd.ninc[1], gd.ninc[2], gd.ninc[3]};
   const uint32_t max_trials = (uint32_t)(T.d->max_trials < (int64_t)0x7FFFFFF0 ? (T.d->max_trials > 0 ? T.d->max_trials : 1)
                                                                                : (int64_t)0x7FFFFFF0);
-  WaveQueue<64> q;
+  // Requests per queue access: a quarter of a wave's share, so that the waves
+  // end together, from one per group up to 64.  With 64 whatever the count, a
+  // launch of 64 requests at 64 lanes each ran them one after another in its
+  // first wave: 130 us for a handful of one-candidate draws.
+  WaveQueue q;
+  q.chunk = (int)min((int64_t)64, max((int64_t)(64 >> lgG), count / (16 * (int64_t)blocks)));
   bool have = false, done = false;
+  bool drained = false;  // wave-uniform: the request queue is empty
   double E = 0.0, mf = 0.0;
   uint64_t sid = 0;
   const float* base = T.f32;
@@ -280,7 +286,7 @@ __device__ void draw_loop(const DevTables& T, const DrawLaunch& io, uint64_t see
     // refill's loads and table searches cost a whole-wave pass each time
     const bool need = (gl == 0) && !have && !done;
     const unsigned long long nm = __ballot(need);
-    if (nm && (__popcll(nm) >= (32 >> lgG) || __ballot(have) == 0ull)) {
+    if (nm && !drained && (__popcll(nm) >= (32 >> lgG) || __ballot(have) == 0ull)) {
       const int64_t r = q.take(nm, need, io.counters + refill_ctr(p));
       if (need) {
         if (r < count) {
@@ -311,8 +317,41 @@ __device__ void draw_loop(const DevTables& T, const DrawLaunch& io, uint64_t see
         base = (const float*)shfl_u64((unsigned long long)base, g0);
         j = __shfl(j, g0);
       }
+      drained = __ballot(done) != 0ull;
     }
-    if (__ballot(have) == 0ull) break;
+    const unsigned long long hm = __ballot(have);
+    if (hm == 0ull) break;
+    if (drained) {
+      // no request waits: the lanes of the groups that are through join the
+      // requests still open.  With n of them left, each gets the largest
+      // power of two of lanes that fits n times into the wave; the k-th open
+      // group's state moves to the k-th run of lanes.  Candidate j stays
+      // Philox counter j, so the accepted one is the same.
+      const int n_open = __popcll(hm) >> lgG;
+      int lg2 = lgG;
+      while ((n_open << (lg2 + 1)) <= 64) ++lg2;
+      if (lg2 > lgG) {
+        const int k = lane >> lg2;  // the run's open group
+        unsigned long long rest = hm;
+        for (int i = 0; i < k && rest; ++i) {
+          const int first = __ffsll((long long)rest) - 1;  // leader of the i-th open group
+          rest &= ~(((1ull << G) - 1ull) << first);                  // G < 64: lg2 > lgG
+        }
+        const int src = rest ? __ffsll((long long)rest) - 1 : 0;
+        E = shfl_f64(E, src);
+        mf = shfl_f64(mf, src);
+        sid = shfl_u64(sid, src);
+        oidx = (int64_t)shfl_u64((unsigned long long)oidx, src);
+        base = (const float*)shfl_u64((unsigned long long)base, src);
+        j = __shfl(j, src);
+        have = rest != 0ull;
+        lgG = lg2;
+        G = 1 << lgG;
+        gl = lane & (G - 1);
+        g0 = lane - gl;
+      }
+    }
+    const unsigned long long gmask = (G == 64) ? ~0ull : (((1ull << G) - 1ull) << g0);
     double x[4] = {0.0, 0.0, 0.0, 0.0};
     double w = 0.0, ua = 1.0, J = 0.0;
     const uint32_t jc = j + (uint32_t)gl;
@@ -381,10 +420,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     int lg, blocks;
     draw_plan((double)cnt, io.full_blocks, io.min_lg, io.group_requests, lg, blocks);
     if ((int)blockIdx.x >= blocks) return;
-    draw_loop<P>(T, io, seed, cnt, lg);
+    draw_loop<P>(T, io, seed, cnt, lg, blocks);
   } else {
     if (io.count[P] <= 0) return;
-    draw_loop<P>(T, io, seed, io.count[P], io.lgG[P]);
+    draw_loop<P>(T, io, seed, io.count[P], io.lgG[P], (int)gridDim.x);
   }
 }
 
@@ -490,14 +529,14 @@ __global__ __launch_bounds__(256) void k_draw_small(DevTables T, DrawLaunch io, 
   draw_plan((double)cnt, per, io.min_lg, io.group_requests, lg, blocks);
   if (b >= blocks) return;
   switch (p) {
-    case 0: draw_loop<0>(T, io, seed, cnt, lg); break;
-    case 1: draw_loop<1>(T, io, seed, cnt, lg); break;
-    case 2: draw_loop<2>(T, io, seed, cnt, lg); break;
-    case 3: draw_loop<3>(T, io, seed, cnt, lg); break;
-    case 4: draw_loop<4>(T, io, seed, cnt, lg); break;
-    case 5: draw_loop<5>(T, io, seed, cnt, lg); break;
-    case 6: draw_loop<6>(T, io, seed, cnt, lg); break;
-    default: draw_loop<7>(T, io, seed, cnt, lg); break;
+    case 0: draw_loop<0>(T, io, seed, cnt, lg, blocks); break;
+    case 1: draw_loop<1>(T, io, seed, cnt, lg, blocks); break;
+    case 2: draw_loop<2>(T, io, seed, cnt, lg, blocks); break;
+    case 3: draw_loop<3>(T, io, seed, cnt, lg, blocks); break;
+    case 4: draw_loop<4>(T, io, seed, cnt, lg, blocks); break;
+    case 5: draw_loop<5>(T, io, seed, cnt, lg, blocks); break;
+    case 6: draw_loop<6>(T, io, seed, cnt, lg, blocks); break;
+    default: draw_loop<7>(T, io, seed, cnt, lg, blocks); break;
   }
 }
 
@@ -907,7 +946,7 @@ __global__ __launch_bounds__(256) void k_transport(DevTables T, DevStore S, int6
   __syncthreads();
   const LdsSigma L{s_sig};
   const int lane = threadIdx.x & 63;
-  WaveQueue<64> q;
+  WaveQueue q;
   // lane states: stepping (act), finished and parked (wait), empty (neither), no work left (done)
   bool act = false, wait = false, done = false;
   int64_t slot = 0;

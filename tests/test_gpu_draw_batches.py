@@ -48,3 +48,23 @@ def test_request_slots(ctx, n, noalloc):
     assert np.array_equal(t, ts)
     assert np.array_equal(w, ws)
     assert np.array_equal(x[has], xs[has])
+
+
+# a batch whose groups start at 2 to 32 lanes: once no request waits, a wave's
+# idle lanes join the open ones (Ann at 60 MeV takes up to 1,000 candidates)
+@pytest.mark.parametrize("P, E", [("Ann", 0.06), ("Ann", 95.0), ("Brem", 50.0), ("PairProd", 10.0), ("MuonBrem", 20.0),
+                                  ("Comp", 1.0)])
+@pytest.mark.parametrize("n", [9001, 40000, 300001])
+def test_groups_that_grow(ctx, P, E, n):
+    m = min(n, 6000)
+    proc = np.full(n, all_process_code[P], dtype=np.int32)
+    e = np.full(n, E)
+    sid = np.arange(n)
+    x, t, w = _draw(ctx, proc, e, sid)
+    assert np.all(t > 0)
+    for lo in (0, n - m):
+        s = slice(lo, lo + m)
+        xs, ts, ws = _pieces(ctx, proc[s], e[s], sid[s], 500)  # 64 lanes per request throughout
+        assert np.array_equal(t[s], ts)
+        assert np.array_equal(w[s], ws)
+        assert np.array_equal(x[s], xs)
