@@ -159,15 +159,16 @@ typedef struct {
                               * is 4 ms per step slower on the 100k lead workload] */
   int32_t graph;             /* 1: a sweep group with per-process draw streams is captured once per
                               * run as a HIP graph and replayed; 2: direct launches [2] */
-  int32_t tail_sweep;        /* once fewer particles than this wait for the next sweep (seen at a host
-                              * check), each remaining particle's subtree is walked depth-first by one
-                              * wave (transport, draw and children in one kernel) [16384]; 1: never */
-  int32_t tail_waves;        /* depth-first walk waves per CU [8] */
-  int32_t tail_depth;        /* depth-first walk: stack entries per wave (1..128); a child past a full
-                              * stack waits for the next launch [128] */
-  int32_t tail_budget;       /* depth-first walk: particles a wave walks from one claimed particle before
-                              * it leaves the rest of its stack to the next launch [16]; a value above
-                              * 2^30 never leaves it */
+  int32_t tail_sweep;        /* once fewer particles than this wait for the next sweep (the primaries,
+                              * or as seen at a host check), the remaining particles and their subtrees
+                              * are walked by waves, a particle per lane (transport, draw and children
+                              * in one kernel) [16384]; 1: never */
+  int32_t tail_waves;        /* walk: waves per CU [8] */
+  int32_t tail_depth;        /* walk: stack entries per wave (1..128); a child past a full stack waits for
+                              * the next launch [128] */
+  int32_t tail_budget;       /* walk: particles per lane after which a wave leaves the rest of its stack
+                              * to the next launch, in the first launch; twice as many in each later one
+                              * [16]; a value above 2^30 never leaves it */
 } PetiteTuning;
 
 /* Set (tuning != NULL) or reset to the defaults (NULL) the context's launch

@@ -125,6 +125,16 @@ __device__ inline double shfl_f64(double v, int src) {
   return __longlong_as_double((long long)shfl_u64((unsigned long long)__double_as_longlong(v), src));
 }
 
+// Lane of the k-th set bit of mask (any lane when mask has fewer): the set
+// bits' lanes pushed to the front, one permutation.  Every lane of the wave
+// calls it.
+__device__ inline int nth_lane(unsigned long long mask, int k) {
+  const int lane = threadIdx.x & 63;
+  const int before = __popcll(mask & ((1ull << lane) - 1ull));
+  const int to = (mask >> lane) & 1ull ? before : __popcll(mask) + lane - before;
+  return __shfl(__builtin_amdgcn_ds_permute(to << 2, lane), k);
+}
+
 __device__ inline unsigned long long wave_sum(unsigned long long v) {
   for (int off = 32; off > 0; off >>= 1) v += shfl_u64(v, (threadIdx.x & 63) ^ off);
   return v;
@@ -331,20 +341,14 @@ __device__ void draw_loop(const DevTables& T, const DrawLaunch& io, uint64_t see
       int lg2 = lgG;
       while ((n_open << (lg2 + 1)) <= 64) ++lg2;
       if (lg2 > lgG) {
-        const int k = lane >> lg2;  // the run's open group
-        unsigned long long rest = hm;
-        for (int i = 0; i < k && rest; ++i) {
-          const int first = __ffsll((long long)rest) - 1;  // leader of the i-th open group
-          rest &= ~(((1ull << G) - 1ull) << first);                  // G < 64: lg2 > lgG
-        }
-        const int src = rest ? __ffsll((long long)rest) - 1 : 0;
+        const int src = nth_lane(__ballot(have && gl == 0), lane >> lg2);
         E = shfl_f64(E, src);
         mf = shfl_f64(mf, src);
         sid = shfl_u64(sid, src);
         oidx = (int64_t)shfl_u64((unsigned long long)oidx, src);
         base = (const float*)shfl_u64((unsigned long long)base, src);
         j = __shfl(j, src);
-        have = rest != 0ull;
+        have = (lane >> lg2) < n_open;
         lgG = lg2;
         G = 1 << lgG;
         gl = lane & (G - 1);
@@ -2357,10 +2361,13 @@ int petite_run_showers(PetiteCtx* c, const PetitePrimary* prim, int64_t n, uint6
   for (int p = 0; p < 8; ++p)
     if (c->desc.grid[p].n_E > 0 && (muons || (p != MUONE && p != MUONBREM))) small_procs |= 1u << p;
   const size_t lds = (size_t)c->dev.lds_doubles * sizeof(double);
-  // the depth-first walk of the last particles (k_tail): entered once fewer
-  // than tn.tail_sweep particles wait at a host check, then one launch per
-  // check until no spill is left
-  bool tail = false;
+  // the walk (k_tail): entered once fewer than tn.tail_sweep particles wait at
+  // a host check, the primaries included, then launched until no spill is
+  // left.  Small batches are all walk: every sweep costs 0.3-0.4 ms whatever it
+  // holds, and a run needs one per generation (measured, sweeps first / walk
+  // only: 1,000 x 10 GeV graphite 14.7 / 6.6 ms, 10,000 primaries of 0.1-100 GeV
+  // in lead 61 / 27 ms)
+  bool tail = n < (int64_t)tn.tail_sweep;
   int tpar = 0;  // spill list the next walk reads
   int64_t tail_launches = 0;
   double t_tail = 0.0;
@@ -2433,7 +2440,7 @@ int petite_run_showers(PetiteCtx* c, const PetitePrimary* prim, int64_t n, uint6
         if (c->timing) HIP_TRY(hipEventRecord(c->tev[4 * group + 2 * g], s));
         const TailParams tp{c->tail_spill + (int64_t)tpar * kTailSpill, ctr + C_SPILL + tpar,
                             c->tail_spill + (int64_t)(tpar ^ 1) * kTailSpill, ctr + C_SPILL + (tpar ^ 1), kTailSpill,
-                            tn.tail_depth, tn.tail_budget};
+                            tn.tail_depth, tail_limit(tn.tail_budget, tail_launches)};
         hipLaunchKernelGGL(k_tail, dim3(tail_blocks), dim3(256), lds, s, c->dev, S, seed, shower_energy, ctr,
                            c->dsig_lds, (const int64_t*)c->drange, ResumeBuf{c->dresume, rcap}, tp);
         HIP_TRY(hipGetLastError());

@@ -1,107 +1,130 @@
-// The last generations of a run as depth-first walks (k_tail).
+// The last generations of a run as walks (k_tail).
 //
 // Sweeps advance a batch one generation at a time, so a run takes as many
 // sweeps as its deepest chain of generations, and every sweep costs a fixed
 // latency however few particles it holds: a transport launch whose slowest
 // particle takes its substeps one after another, a draw launch whose slowest
 // request takes its candidate rounds, an emission launch.  A 400 GeV muon's
-// ~2,000 MuonE vertices are 2,000 generations.  Once few particles remain, a
-// wave instead takes one particle and walks its whole subtree: transport to
-// the next hard interaction (propagate_particle, shower.py:509-601), the
-// process choice (665-698), the accept/reject draw with the wave's 64 lanes
-// on candidates j .. j + 63 (draw_sample, 401-465; the lowest accepted index
-// is the sequential loop's candidate), and the children (sample_scattering,
-// 467-507) appended to the store.  The kept children go on the wave's stack,
-// the lower-energy one on top, so it is walked first: its energy is at most
-// half the parent's (plus m_e), so the stack never holds more than about
-// log2(E_primary / min_energy) + 1 entries.  A full stack (a depth limit
-// below that) passes the child to a spill list, which the next launch walks.
-// Every random number comes from the particle's own Philox stream, as in the
-// sweeps, so the records are the sweeps' records, bit for bit.
+// ~2,000 MuonE vertices are 2,000 generations.  Once few particles remain,
+// each wave instead walks particles and their subtrees by itself, one particle
+// per lane: substeps to the next hard interaction (propagate_particle,
+// shower.py:509-601) and the process choice (665-698); when two thirds of the
+// live lanes have got there, their accept/reject draws (draw_sample, 401-465),
+// the wave's 64 lanes shared among them, process by process (the lowest
+// accepted index is the sequential loop's candidate); and the children
+// (sample_scattering, 467-507), appended to the store.  A lane goes on with its
+// higher-energy child, so the chain that sets the run's length never waits; the
+// lower-energy one goes on the wave's stack, from which free lanes take.  A
+// full stack passes children to a spill list, and after its share of
+// iterations a wave starts nothing more and leaves its stack there, so the
+// next launch spreads the particles over all waves again.  Every random number
+// comes from the particle's own Philox stream, as in the sweeps, so the records
+// are the sweeps' records, bit for bit.
 //
-// The walk is wave-uniform: every lane computes the same transport (the
-// loads are the same addresses) and lane 0 writes; only the draw spreads the
-// candidates over the lanes.
+// What bounds it: the latency of a substep (~600 dependent instructions) and of
+// a draw phase, at 2 waves per SIMD.  Its predecessor walked one particle per
+// wave, every lane computing the same transport, with two atomics per draw on
+// one line of per-process counters; 400 GeV beam of 2,000 in lead: 264 ms per
+// run with it (170 ms of that in the walk), 166 ms now, all of it walk.
 #pragma once
 
-constexpr int kTailMaxDepth = 128;  // two stack entries per lane
-constexpr int kTailGroup = 8;       // walk launches queued per host check after the first
-constexpr int64_t kTailSpill = 1 << 20;  // entries per spill list
+constexpr int kTailMaxDepth = 128;  // stack entries per wave
+constexpr int kTailGroup = 4;       // walk launches queued per host check after the first
+constexpr int64_t kTailSpill = 1 << 22;  // entries per spill list
+constexpr int kTailStepsPerParticle = 8;  // iterations of a wave per particle of its lanes' budget
+constexpr int kTailPhaseSteps = 4;        // iterations a draw phase counts for
 
 struct TailParams {
   const int32_t* spill_in;            // slots left by the previous launch
   const unsigned long long* n_spill_in;
-  int32_t* spill_out;                 // slots past a full stack
+  int32_t* spill_out;                 // slots past a full stack or the launch's share
   unsigned long long* n_spill_out;
   int64_t spill_cap;
   int32_t depth;   // stack entries per wave (1..kTailMaxDepth)
-  int32_t budget;  // particles a wave walks from one claimed particle before it passes its stack on
+  int64_t limit;   // iterations after which a wave starts no more particles
 };
 
-// The wave's stack in registers: entry e sits in lane e % 64, in `lo` for
-// e < 64 and in `hi` above; sp is wave-uniform.
-struct WaveStack {
-  int32_t lo = 0, hi = 0;
-  int sp = 0;
-  __device__ inline void push(int32_t v, int lane) {
-    if (sp < 64) {
-      if (lane == sp) lo = v;
-    } else if (lane == sp - 64) {
-      hi = v;
-    }
-    ++sp;
-  }
-  __device__ inline int32_t pop() {
-    --sp;
-    return sp < 64 ? __shfl(lo, sp) : __shfl(hi, sp - 64);
-  }
+// A wave's buffers in LDS.
+struct WalkLds {
+  int32_t stack[kTailMaxDepth];
+  double x0[64];     // a lane's accepted point: the 1-D variable in float64,
+  float4 xs[64];     //   the 4-D point as the draw kernels store it,
+  int32_t tr[64];    //   the candidate count (negative: none in max_trials)
+};
+// Per-process draw statistics of a block.
+struct WalkStats {
+  unsigned long long trials[8], draws[8], viol[8];
 };
 
-// One accept/reject draw of process P by the whole wave (results uniform):
-// the candidate count as the draw stores it (negative when max_trials passed
-// without an acceptance), the accepted point and its J*f, and max_F.
+// The draws of process P that the lanes in `mine` ask for (at least one), by
+// the whole wave: results in W, indexed by the asking lane.  ie, mf: the asking
+// lane's map energy and max_F.
 template <int P>
-__device__ inline int32_t wave_draw(const DevTables& T, double E, uint64_t seed, uint64_t sid, float* xs, double& w_acc,
-                                    double& mf) {
+__device__ inline void walk_draws(const DevTables& T, uint64_t seed, bool mine, double E_own, uint64_t sid_own,
+                                  int ie, double mf, WalkLds& W, WalkStats& B) {
   constexpr int ND = proc_ndim<P>();
   const int lane = threadIdx.x & 63;
   const PetiteGridDesc& gd = T.d->grid[P];
   const int32_t ninc[4] = {gd.ninc[0], gd.ninc[1], gd.ninc[2], gd.ninc[3]};
   const uint32_t max_trials = (uint32_t)(T.d->max_trials < (int64_t)0x7FFFFFF0 ? (T.d->max_trials > 0 ? T.d->max_trials : 1)
                                                                                : (int64_t)0x7FFFFFF0);
-  const int ie = lu_key(T, P, E);
+  unsigned long long om = __ballot(mine);
+  int lg = 0, n_open = __popcll(om);
+  while ((n_open << (lg + 1)) <= 64) ++lg;
+  int G = 1 << lg, gl = lane & (G - 1), g0 = lane - gl;
+  int owner = nth_lane(om, lane >> lg);
+  bool have = (lane >> lg) < n_open;
+  double E = shfl_f64(E_own, owner);
+  mf = shfl_f64(mf, owner);
+  uint64_t sid = shfl_u64(sid_own, owner);
+  ie = __shfl(ie, owner);
   const float* base = T.f32 + gd.node_off + (int64_t)ie * gd.stride;
-  mf = T.maxf[P * T.maxE + ie] * T.d->maxF_fudge;
-  for (uint32_t j = draw_possible<P>(T) ? 0u : max_trials; j < max_trials; j += 64u) {
-    const uint32_t jc = j + (uint32_t)lane;
+  uint32_t j = draw_possible<P>(T) ? 0u : max_trials;
+  while (true) {
     double x[4] = {0.0, 0.0, 0.0, 0.0};
-    double ua = 1.0, J = 0.0;
-    double w = candidate_w<P, ND>(T, E, base, ninc, seed, sid, jc, x, ua, J);
-    if (ND == 4 && fabs(mf * ua - w) <= kRefBand * w) w = J * integrand_ref<P>(T, E, x);
-    const bool acc = (jc < max_trials) && (mf * ua < w);
-    const unsigned long long am = __ballot(acc);
-    if (am) {
-      const int win = __ffsll((long long)am) - 1;
-      for (int d = 0; d < 4; ++d) xs[d] = (float)shfl_f64(x[d], win);
-      w_acc = shfl_f64(w, win);
-      return (int32_t)(j + (uint32_t)win + 1u);
+    double w = 0.0, ua = 1.0, J = 0.0;
+    const uint32_t jc = j + (uint32_t)gl;
+    if (have) {
+      w = candidate_w<P, ND>(T, E, base, ninc, seed, sid, jc, x, ua, J);
+      if (ND == 4 && fabs(mf * ua - w) <= kRefBand * w) w = J * integrand_ref<P>(T, E, x);
     }
-  }
-  w_acc = 0.0;
-  return -(int32_t)max_trials;
-}
-
-__device__ inline int32_t wave_draw_any(int p, const DevTables& T, double E, uint64_t seed, uint64_t sid, float* xs,
-                                        double& w_acc, double& mf) {
-  switch (p) {
-    case 0: return wave_draw<0>(T, E, seed, sid, xs, w_acc, mf);
-    case 1: return wave_draw<1>(T, E, seed, sid, xs, w_acc, mf);
-    case 2: return wave_draw<2>(T, E, seed, sid, xs, w_acc, mf);
-    case 3: return wave_draw<3>(T, E, seed, sid, xs, w_acc, mf);
-    case 4: return wave_draw<4>(T, E, seed, sid, xs, w_acc, mf);
-    case 5: return wave_draw<5>(T, E, seed, sid, xs, w_acc, mf);
-    case 6: return wave_draw<6>(T, E, seed, sid, xs, w_acc, mf);
-    default: return wave_draw<7>(T, E, seed, sid, xs, w_acc, mf);
+    const bool acc = have && (jc < max_trials) && (mf * ua < w);
+    const unsigned long long gmask = (G == 64) ? ~0ull : (((1ull << G) - 1ull) << g0);
+    const unsigned long long am = __ballot(acc) & gmask;
+    if (have) {
+      const bool over = !am && j + (uint32_t)G >= max_trials;
+      if (am ? lane == __ffsll((long long)am) - 1 : (over && gl == 0)) {
+        const uint32_t n = am ? jc + 1u : max_trials;
+        W.tr[owner] = am ? (int32_t)n : -(int32_t)n;
+        W.x0[owner] = x[0];
+        W.xs[owner] = make_float4((float)x[0], (float)x[1], (float)x[2], (float)x[3]);
+        atomicAdd(&B.trials[P], (unsigned long long)n);
+        atomicAdd(&B.draws[P], 1ull);
+        if (am && w > mf) atomicAdd(&B.viol[P], 1ull);
+      }
+      if (am || over) have = false;
+      j += (uint32_t)G;
+    }
+    const unsigned long long lead = __ballot(have && gl == 0);
+    if (lead == 0ull) break;
+    n_open = __popcll(lead);
+    int lg2 = lg;
+    while ((n_open << (lg2 + 1)) <= 64) ++lg2;
+    if (lg2 > lg) {
+      // the lanes of the draws that are through join the open ones (draw_loop)
+      const int src = nth_lane(lead, lane >> lg2);
+      have = (lane >> lg2) < n_open;
+      E = shfl_f64(E, src);
+      mf = shfl_f64(mf, src);
+      sid = shfl_u64(sid, src);
+      base = (const float*)shfl_u64((unsigned long long)base, src);
+      owner = __shfl(owner, src);
+      j = __shfl(j, src);
+      lg = lg2;
+      G = 1 << lg;
+      gl = lane & (G - 1);
+      g0 = lane - gl;
+    }
   }
 }
 
@@ -109,9 +132,10 @@ __device__ inline int32_t wave_draw_any(int p, const DevTables& T, double E, uin
 // sweep handed on (live state in its resume records), the store slots
 // [first, first + n), then the previous launch's spills.  range: the tail
 // setup's {first, n, end, nres}.
-__global__ __launch_bounds__(256) void k_tail(DevTables T, DevStore S, uint64_t seed, double* shower_energy,
-                                              unsigned long long* counters, const double* sig_lds_src,
-                                              const int64_t* range, ResumeBuf RB, TailParams TPm) {
+constexpr int kWalkWaves = 4;  // waves per block
+__global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu(2))) void k_tail(DevTables T, DevStore S, uint64_t seed, double* shower_energy,
+                                                          unsigned long long* counters, const double* sig_lds_src,
+                                                          const int64_t* range, ResumeBuf RB, TailParams TPm) {
   const int64_t first = range[0], n = range[1];
   const int64_t nres = RB.rec ? range[3] : 0;
   const ResumeRec* rin = RB.rec ? RB.rec + (int64_t)(counters[C_RPARITY] & 1ull) * RB.cap : nullptr;
@@ -119,276 +143,393 @@ __global__ __launch_bounds__(256) void k_tail(DevTables T, DevStore S, uint64_t 
   // run reports) is cut to the list
   const int64_t n_in = (int64_t)*TPm.n_spill_in;
   const int64_t total = nres + n + (n_in < TPm.spill_cap ? n_in : TPm.spill_cap);
-  if ((int64_t)blockIdx.x * 4 >= total) return;
+  // items per claim: an even share of every wave of the launch, at most a lane's each
+  const int64_t waves = (int64_t)gridDim.x * kWalkWaves;
+  const int share = (int)min((int64_t)64, max((int64_t)1, (total + waves - 1) / waves));
+  if ((int64_t)blockIdx.x * kWalkWaves * share >= total) return;
   HIP_DYNAMIC_SHARED(double, s_sig)
+  __shared__ WalkLds s_walk[kWalkWaves];
+  __shared__ WalkStats s_stat;
   for (int i = threadIdx.x; i < T.lds_doubles; i += blockDim.x) s_sig[i] = sig_lds_src[i];
+  if (threadIdx.x < 8) s_stat.trials[threadIdx.x] = s_stat.draws[threadIdx.x] = s_stat.viol[threadIdx.x] = 0ull;
   __syncthreads();
   const LdsSigma L{s_sig};
   const int lane = threadIdx.x & 63;
+  const unsigned long long below = (1ull << lane) - 1ull;
+  WalkLds& W = s_walk[threadIdx.x >> 6];
   const int depth = TPm.depth < 1 ? 1 : (TPm.depth > kTailMaxDepth ? kTailMaxDepth : TPm.depth);
-  WaveStack st;
-  unsigned long long steps = 0, n_trials = 0, n_draws = 0, n_viol = 0, n_fail = 0, n_drop = 0, n_ovf = 0, n_lost = 0;
-  int walked = 0;  // particles walked since the wave's last claim
+  // more items than half a spill list holds are all walked in this launch
+  const int64_t limit = total > TPm.spill_cap / 2 ? (int64_t)1 << 62 : TPm.limit;
+  // lane states: empty, stepping, at its end (parked)
+  enum { EMPTY = 0, STEP = 1, PARKED = 2 };
+  int mode = EMPTY;
+  int sp = 0;              // stack entries (wave-uniform, as the next four)
+  int64_t iters = 0;
+  bool exhausted = false, fresh = true;
+  int32_t slot = 0;
+  int pid = 0, shower = 0, gen = 0;
+  uint32_t ch = 0xFFFu;
+  uint64_t sid = 0;
+  double m = 0.0, pme = 0.0, E = 0.0, p = 0.0, dep = 0.0, dz = 0.0;
+  float nx = 0.0f, ny = 0.0f, nz = 0.0f, rx = 0.0f, ry = 0.0f, rz = 0.0f, wgt = 0.0f;
+  uint32_t k = 0;
+  bool closing = false;
+  unsigned long long steps = 0, n_fail = 0, n_drop = 0, n_ovf = 0, n_lost = 0;
+  // puts the lane on a particle of species pid at its start (k_transport's refill)
+  auto start = [&](float4 p0, float4 r0) {
+    ch = sum_channels(pid);
+    m = pid_mass(pid);
+    pme = fmax(fmax(min_calc(T, pid), T.d->min_energy), m);
+    E = (double)p0.x;
+    nx = p0.y;
+    ny = p0.z;
+    nz = p0.w;
+    const float pn2 = nx * nx + ny * ny + nz * nz;
+    if (pn2 > 0.0f) {
+      const float inv = rsqrtf(pn2);
+      nx *= inv;
+      ny *= inv;
+      nz *= inv;
+    }
+    const bool still = ch == 0xFFFu && pid != 22;
+    p = still ? sqrt((double)pn2) : 0.0;  // the others' |p| is formed when they finish
+    rx = r0.x;
+    ry = r0.y;
+    rz = r0.z;
+    wgt = r0.w;
+    dep = 0.0;
+    k = 0;
+    closing = false;
+    mode = STEP;
+    if (E < pme || still) {
+      mode = PARKED;  // ends where it starts (shower.py:532-536, 640-653)
+    } else if (pid == 22) {
+      // one exponential flight, no MCS (shower.py:538-553)
+      const double mfp = L.mfp(22, E);
+      const double dist = -mfp * (double)log1p_f32(-u01f(draw_block(seed, sid, 0, PURPOSE_STEP).x));
+      rx += (float)(nx * dist);
+      ry += (float)(ny * dist);
+      rz += (float)(nz * dist);
+      k = 1;
+      mode = PARKED;
+    }
+  };
   while (true) {
-    // a claimed particle's subtree beyond `budget` particles is left to the
-    // next launch, which spreads the stack's entries over all of its waves:
-    // one large subtree no longer holds a single wave while the others idle
-    if (TPm.budget > 0 && walked >= TPm.budget && st.sp > 0) {
-      unsigned long long o = 0;
-      if (lane == 0) o = atomicAdd(TPm.n_spill_out, (unsigned long long)st.sp);
-      o = shfl_u64(o, 0);
-      if (lane < st.sp && (int64_t)(o + lane) < TPm.spill_cap) TPm.spill_out[o + lane] = st.lo;
-      if (lane + 64 < st.sp && (int64_t)(o + lane + 64) < TPm.spill_cap) TPm.spill_out[o + lane + 64] = st.hi;
-      const int64_t past = (int64_t)o + st.sp - TPm.spill_cap;
-      if (past > 0) n_lost += (unsigned long long)(past < st.sp ? past : st.sp);  // reported as an internal error
-      st.sp = 0;
-    }
-    int64_t slot;
-    int64_t rr = -1;  // the claimed item (-1: popped from the stack)
-    if (st.sp > 0) {
-      slot = st.pop();
-    } else {
-      walked = 0;
-      unsigned long long c = 0;
-      if (lane == 0) c = atomicAdd(counters + C_TRANSPORT, 1ull);
-      rr = (int64_t)shfl_u64(c, 0);
-      if (rr >= total) break;
-      if (rr < nres) slot = rin[rr].slot;
-      else if (rr < nres + n) slot = first + (rr - nres);
-      else slot = TPm.spill_in[rr - nres - n];
-    }
-    ++walked;
-    const bool resumed = rr >= 0 && rr < nres;
-    // ---- the particle: constants from the store, the start state from the
-    // store or the resume record (k_transport's refill)
-    const int pid = S.pid[slot];
-    const uint64_t sid = S.sid[slot];
-    const int shower = S.shower[slot];
-    const int gen = S.meta[slot] & 0xFFFF;
-    const float wgt = S.r0[slot].w;
-    const uint32_t ch = sum_channels(pid);
-    const double m = pid_mass(pid);
-    const double pme = fmax(fmax(min_calc(T, pid), T.d->min_energy), m);
-    double E, p = 0.0, dep = 0.0, dz = 0.0;
-    float nx, ny, nz, rx, ry, rz;
-    uint32_t k = 0;
-    bool act = false;
-    if (resumed) {
-      const ResumeRec& R0 = rin[rr];
-      E = R0.E;
-      dep = R0.dep;
-      dz = R0.dz;
-      nx = R0.nx;
-      ny = R0.ny;
-      nz = R0.nz;
-      rx = R0.rx;
-      ry = R0.ry;
-      rz = R0.rz;
-      k = R0.k;
-      act = true;
-    } else {
-      const float4 p0 = S.p0[slot];
-      const float4 r0 = S.r0[slot];
-      E = (double)p0.x;
-      nx = p0.y;
-      ny = p0.z;
-      nz = p0.w;
-      const float pn2 = nx * nx + ny * ny + nz * nz;
-      if (pn2 > 0.0f) {
-        const float inv = rsqrtf(pn2);
-        nx *= inv;
-        ny *= inv;
-        nz *= inv;
+    // past its share the wave starts no more: the next launch spreads what it
+    // leaves.  A wave whose particles all have lanes and include a muon goes on:
+    // a muon's chain of thousands of vertices sets the run's length, and
+    // would go slower among a spread's other particles
+    const bool stop = iters >= limit && (sp > 0 || __ballot(mode != EMPTY && (pid == 13 || pid == -13)) == 0ull);
+    // ---- free lanes take from the stack, then claim items (after a draw
+    // phase, or when no lane is stepping)
+    const unsigned long long im = __ballot(mode == EMPTY);
+    if (im && !stop && (fresh || __ballot(mode == STEP) == 0ull)) {
+      const int rank = __popcll(im & below);
+      const int take = min(__popcll(im), sp);
+      bool got = false;
+      int64_t rr = -1;
+      if (mode == EMPTY && rank < take) {
+        slot = W.stack[sp - 1 - rank];
+        got = true;
       }
-      const bool still = ch == 0xFFFu && pid != 22;
-      p = still ? sqrt((double)pn2) : 0.0;  // the others' |p| is formed when they finish
-      rx = r0.x;
-      ry = r0.y;
-      rz = r0.z;
-      if (E < pme || still) {
-        // ends where it starts (shower.py:532-536, 640-653)
-      } else if (pid == 22) {
-        // one exponential flight, no MCS (shower.py:538-553)
-        const double mfp = L.mfp(22, E);
-        const double dist = -mfp * (double)log1p_f32(-u01f(draw_block(seed, sid, 0, PURPOSE_STEP).x));
-        rx += (float)(nx * dist);
-        ry += (float)(ny * dist);
-        rz += (float)(nz * dist);
-        k = 1;
-      } else {
-        act = true;
-      }
-    }
-    // ---- substeps, then the closing increment (k_transport's advance)
-    bool closing = false;
-    while (act) {
-      const bool in_close = closing;
-      const double Ssum = L.nsigma_sum_ch(ch, E);
-      const double mfp = Ssum > 0.0 ? kCmToM / Ssum : 1.0e12;
-      const U4 u = draw_block(seed, sid, in_close ? 0u : k, in_close ? PURPOSE_CLOSE : PURPOSE_STEP);
-      bool adv = true;
-      double dist;
-      uint32_t w_r, w_a;
-      double m_lep = m;
-      if (!in_close) {
-        const double div = 6.0 + 14.0 * u01d(u.y);
-        dz = mfp / div;
-        dist = dz;
-        w_r = u.z;
-        w_a = u.w;
-        const double ux = u01d(u.x);
-        double thr = (double)__expf(-__builtin_amdgcn_rcpf((float)div));
-        if (fabs(ux - thr) < 1.0e-5) thr = exp(-(dz / mfp));
-        if (ux > thr) {
-          adv = false;
-          closing = true;
+      sp -= take;
+      const int need = min(__popcll(im) - take, share);
+      if (need > 0 && !exhausted) {
+        unsigned long long c = 0;
+        if (lane == 0) c = atomicAdd(counters + C_TRANSPORT, (unsigned long long)need);
+        c = shfl_u64(c, 0);
+        if (mode == EMPTY && !got && rank - take < need) {
+          rr = (int64_t)c + (rank - take);
+          got = rr < total;
+          if (got) slot = rr < nres ? rin[rr].slot
+                                    : (rr < nres + n ? (int32_t)(first + (rr - nres)) : TPm.spill_in[rr - nres - n]);
         }
-      } else {
-        const double distC = u01d(u.x);
-        if (E < pme) {
-          dist = distC * dz;
+        exhausted = (int64_t)c + need >= total;
+      }
+      if (got) {
+        pid = S.pid[slot];
+        sid = S.sid[slot];
+        shower = S.shower[slot];
+        gen = S.meta[slot] & 0xFFFF;
+        const float4 r0 = S.r0[slot];
+        start(S.p0[slot], r0);
+        if (rr >= 0 && rr < nres) {
+          // handed on by the last sweep: its live state
+          const ResumeRec& R0 = rin[rr];
+          E = R0.E;
+          dep = R0.dep;
+          dz = R0.dz;
+          nx = R0.nx;
+          ny = R0.ny;
+          nz = R0.nz;
+          rx = R0.rx;
+          ry = R0.ry;
+          rz = R0.rz;
+          k = R0.k;
+          mode = STEP;
+        }
+      }
+    }
+    fresh = false;
+    const unsigned long long am = __ballot(mode == STEP), wm = __ballot(mode == PARKED);
+    if (am == 0ull && wm == 0ull) break;
+    // a draw phase costs several substeps (loads, a round of candidates per
+    // process, the kinematics): run at two thirds of the live lanes parked it
+    // measures 15 % faster than at a third over the showers of 1 to 100,000
+    // primaries, and a half or four fifths are in between
+    if (am != 0ull && __popcll(wm) < 2 * __popcll(am)) {
+      // ---- one advance of every stepping lane (k_transport's)
+      ++iters;
+      if (mode == STEP) {
+        const bool in_close = closing;
+        const double Ssum = L.nsigma_sum_ch(ch, E);
+        const double mfp = Ssum > 0.0 ? kCmToM / Ssum : 1.0e12;
+        const U4 u = draw_block(seed, sid, in_close ? 0u : k, in_close ? PURPOSE_CLOSE : PURPOSE_STEP);
+        bool adv = true;
+        double dist;
+        uint32_t w_r, w_a;
+        double m_lep = m;
+        if (!in_close) {
+          const double div = 6.0 + 14.0 * u01d(u.y);
+          dz = mfp / div;
+          dist = dz;
+          w_r = u.z;
+          w_a = u.w;
+          const double ux = u01d(u.x);
+          double thr = (double)__expf(-__builtin_amdgcn_rcpf((float)div));
+          if (fabs(ux - thr) < 1.0e-5) thr = exp(-(dz / mfp));
+          if (ux > thr) {
+            adv = false;
+            closing = true;
+          }
         } else {
-          const float r2 = Ssum > 0.0 ? (float)(dz * Ssum * (1.0 / kCmToM)) : (float)(dz * 1.0e-12);
-          dist = -mfp * (double)log1p_f32(expm1f(-r2) * (float)distC);
+          const double distC = u01d(u.x);
+          if (E < pme) {
+            dist = distC * dz;
+          } else {
+            const float r2 = Ssum > 0.0 ? (float)(dz * Ssum * (1.0 / kCmToM)) : (float)(dz * 1.0e-12);
+            dist = -mfp * (double)log1p_f32(expm1f(-r2) * (float)distC);
+          }
+          w_r = u.y;
+          w_a = u.z;
+          m_lep = kMe;
         }
-        w_r = u.y;
-        w_a = u.z;
-        m_lep = kMe;
+        if (adv) charged_advance(T, dist, m, m_lep, w_r, w_a, E, nx, ny, nz, rx, ry, rz, dep);
+        ++k;
+        if (in_close) mode = PARKED;
+        else if (E < pme) closing = true;
       }
-      if (adv) charged_advance(T, dist, m, m_lep, w_r, w_a, E, nx, ny, nz, rx, ry, rz, dep);
-      ++k;
-      if (in_close) act = false;
-      else if (E < pme) closing = true;
-    }
-    // ---- the final state and the process choice (k_transport's finish)
-    steps += k;
-    if (!(ch == 0xFFFu && pid != 22)) p = momentum(E, m);
-    const float4 pf = make_float4((float)E, (float)(p * nx), (float)(p * ny), (float)(p * nz));
-    if (lane == 0) {
-      S.pf[slot] = pf;
-      S.rf[slot] = make_float4(rx, ry, rz, (float)k);
-    }
-    int want = -1;
-    if (E > pme) {
-      int c0 = -1, c1 = -1, c2 = -1;
-      switch (pid) {
-        case 11: c0 = BREM; c1 = MOLLER; break;
-        case -11: c0 = BREM; c1 = ANN; c2 = BHABHA; break;
-        case 22: c0 = PAIRPROD; c1 = COMP; break;
-        case 13: case -13: c0 = MUONE; c1 = MUONBREM; break;
-        default: break;
-      }
-      if (c0 >= 0) {
-        const float lf = __log2f((float)E);
-        const double w0 = L.nsigma(c0, E, lf), w1 = L.nsigma(c1, E, lf);
-        const double w2 = c2 >= 0 ? L.nsigma(c2, E, lf) : 0.0;
-        const double SC = c2 >= 0 ? w0 + w1 + w2 : w0 + w1;
-        if (SC > 0.0 && !isnan(SC)) {
-          const double uu = u01d(draw_block(seed, sid, 0, PURPOSE_INTERACT).x) * SC;
-          if (uu < w0) want = c0;
-          else if (c2 < 0 || uu < w0 + w1) want = c1;
-          else want = c2;
-        }
-      }
-    }
-    if (shower_energy && lane == 0) {
-      unsafeAtomicAdd(shower_energy + 4 * shower + 0, dep);
-      if (want < 0) unsafeAtomicAdd(shower_energy + 4 * shower + 1, E);
-    }
-    if (want < 0) continue;
-    // ---- the draw
-    float xs[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    double w_acc = 0.0, mf = 0.0;
-    const int32_t tr = wave_draw_any(want, T, E, seed, sid, xs, w_acc, mf);
-    const unsigned long long ntr = tr > 0 ? (unsigned long long)tr : (unsigned long long)(-(int64_t)tr);
-    const bool viol = tr > 0 && w_acc > mf;
-    n_draws += 1;
-    n_trials += ntr;
-    n_viol += viol ? 1ull : 0ull;
-    n_fail += tr > 0 ? 0ull : 1ull;
-    if (lane == 0) {
-      atomicAdd(counters + C_PTRIALS + want, ntr);
-      atomicAdd(counters + C_PDRAWS + want, 1ull);
-      if (viol) atomicAdd(counters + C_PVIOL + want, 1ull);
-    }
-    if (tr <= 0) {
-      if (shower_energy && lane == 0) unsafeAtomicAdd(shower_energy + 4 * shower + 1, E);
       continue;
     }
-    // ---- the children (k_emit)
-    const double az = u01d(draw_block(seed, sid, 0, PURPOSE_INTERACT).y);
-    const double x0 = accepted_x1(T, want, E, seed, sid, tr, xs[0]);
-    V4 lab[2];
-    int cpid[2];
-    vertex_children(want, pid, E, xs, x0, az, pf.y, pf.z, pf.w, lab, cpid);
-    bool keep[2];
-    for (int c = 0; c < 2; ++c) {
-      keep[c] = lab[c].e > T.d->min_energy;
-      if (!keep[c] && shower_energy && lane == 0) unsafeAtomicAdd(shower_energy + 4 * shower + 2, lab[c].e);
+    // ---- the parked lanes' final states and process choices (k_transport's finish)
+    iters += kTailPhaseSteps;
+    fresh = true;
+    int want = -1;
+    float4 pf = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (mode == PARKED) {
+      steps += k;
+      if (!(ch == 0xFFFu && pid != 22)) p = momentum(E, m);
+      pf = make_float4((float)E, (float)(p * nx), (float)(p * ny), (float)(p * nz));
+      S.pf[slot] = pf;
+      S.rf[slot] = make_float4(rx, ry, rz, (float)k);
+      if (E > pme) {
+        int c0 = -1, c1 = -1, c2 = -1;
+        switch (pid) {
+          case 11: c0 = BREM; c1 = MOLLER; break;
+          case -11: c0 = BREM; c1 = ANN; c2 = BHABHA; break;
+          case 22: c0 = PAIRPROD; c1 = COMP; break;
+          case 13: case -13: c0 = MUONE; c1 = MUONBREM; break;
+          default: break;
+        }
+        if (c0 >= 0) {
+          const float lf = __log2f((float)E);
+          const double w0 = L.nsigma(c0, E, lf), w1 = L.nsigma(c1, E, lf);
+          const double w2 = c2 >= 0 ? L.nsigma(c2, E, lf) : 0.0;
+          const double SC = c2 >= 0 ? w0 + w1 + w2 : w0 + w1;
+          if (SC > 0.0 && !isnan(SC)) {
+            const double uu = u01d(draw_block(seed, sid, 0, PURPOSE_INTERACT).x) * SC;
+            if (uu < w0) want = c0;
+            else if (c2 < 0 || uu < w0 + w1) want = c1;
+            else want = c2;
+          }
+        }
+      }
+      if (shower_energy) {
+        unsafeAtomicAdd(shower_energy + 4 * shower + 0, dep);
+        if (want < 0) unsafeAtomicAdd(shower_energy + 4 * shower + 1, E);
+      }
+      mode = EMPTY;
     }
-    if (shower_energy && lane == 0 &&
-        (want == COMP || want == ANN || want == MOLLER || want == BHABHA || want == MUONE))
-      unsafeAtomicAdd(shower_energy + 4 * shower + 3, 1.0);
-    n_drop += (unsigned long long)(!keep[0]) + (unsigned long long)(!keep[1]);
-    const int nk = (int)keep[0] + (int)keep[1];
-    if (nk == 0) continue;
+    // ---- the draws, process by process (the map energies and max_F of all
+    // of them first: one round of dependent loads)
+    int ie = 0;
+    double mf = 0.0;
+    if (want >= 0) {
+      ie = lu_key(T, want, E);
+      mf = T.maxf[want * T.maxE + ie] * T.d->maxF_fudge;
+    }
+    for (unsigned long long todo = __ballot(want >= 0); todo;) {
+      const int q = __shfl(want, __ffsll((long long)todo) - 1);
+      const bool mine = want == q;
+      switch (q) {
+        case 0: walk_draws<0>(T, seed, mine, E, sid, ie, mf, W, s_stat); break;
+        case 1: walk_draws<1>(T, seed, mine, E, sid, ie, mf, W, s_stat); break;
+        case 2: walk_draws<2>(T, seed, mine, E, sid, ie, mf, W, s_stat); break;
+        case 3: walk_draws<3>(T, seed, mine, E, sid, ie, mf, W, s_stat); break;
+        case 4: walk_draws<4>(T, seed, mine, E, sid, ie, mf, W, s_stat); break;
+        case 5: walk_draws<5>(T, seed, mine, E, sid, ie, mf, W, s_stat); break;
+        case 6: walk_draws<6>(T, seed, mine, E, sid, ie, mf, W, s_stat); break;
+        default: walk_draws<7>(T, seed, mine, E, sid, ie, mf, W, s_stat); break;
+      }
+      todo &= ~__ballot(mine);
+    }
+    // results written by other lanes of the wave
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    // ---- the children (k_emit)
+    V4 lab[2];
+    int cpid[2] = {0, 0};
+    bool keep[2] = {false, false};
+    if (want >= 0) {
+      if (W.tr[lane] <= 0) {
+        ++n_fail;
+        if (shower_energy) unsafeAtomicAdd(shower_energy + 4 * shower + 1, E);
+      } else {
+        const double az = u01d(draw_block(seed, sid, 0, PURPOSE_INTERACT).y);
+        const float4 xv = W.xs[lane];
+        const float xs[4] = {xv.x, xv.y, xv.z, xv.w};
+        vertex_children(want, pid, E, xs, W.x0[lane], az, pf.y, pf.z, pf.w, lab, cpid);
+        for (int c = 0; c < 2; ++c) {
+          keep[c] = lab[c].e > T.d->min_energy;
+          if (!keep[c]) {
+            ++n_drop;
+            if (shower_energy) unsafeAtomicAdd(shower_energy + 4 * shower + 2, lab[c].e);
+          }
+        }
+        if (shower_energy && (want == COMP || want == ANN || want == MOLLER || want == BHABHA || want == MUONE))
+          unsafeAtomicAdd(shower_energy + 4 * shower + 3, 1.0);
+      }
+    }
+    // store slots: one atomic per wave and phase
+    const unsigned long long k0 = __ballot(keep[0]), k1 = __ballot(keep[1]);
+    if ((k0 | k1) == 0ull) continue;
     unsigned long long cb = 0;
-    if (lane == 0) cb = atomicAdd(counters + C_STORE, (unsigned long long)nk);
-    cb = shfl_u64(cb, 0);
+    if (lane == 0) cb = atomicAdd(counters + C_STORE, (unsigned long long)(__popcll(k0) + __popcll(k1)));
+    cb = shfl_u64(cb, 0) + (unsigned long long)(__popcll(k0 & below) + __popcll(k1 & below));
     int32_t cslot[2] = {-1, -1};
+    uint64_t csid[2] = {0, 0};
+    float4 cp[2];
     for (int c = 0; c < 2; ++c) {
       if (!keep[c]) continue;
       if ((int64_t)cb < S.capacity) {
-        const int64_t cs = (int64_t)cb;
-        if (lane == 0) {
-          S.p0[cs] = make_float4((float)lab[c].e, (float)lab[c].x, (float)lab[c].y, (float)lab[c].z);
-          S.r0[cs] = make_float4(rx, ry, rz, wgt);
-          S.pid[cs] = cpid[c];
-          S.parent[cs] = (int32_t)slot;
-          S.meta[cs] = ((gen + 1) & 0xFFFF) | ((want + 1) << 16) | (c << 24);
-          S.shower[cs] = shower;
-          S.sid[cs] = derive_sid(seed, sid, (uint32_t)c, PURPOSE_CHILD);
-        }
-        cslot[c] = (int32_t)cs;
+        cslot[c] = (int32_t)cb;
+        cp[c] = make_float4((float)lab[c].e, (float)lab[c].x, (float)lab[c].y, (float)lab[c].z);
+        csid[c] = derive_sid(seed, sid, (uint32_t)c, PURPOSE_CHILD);
+        S.p0[cb] = cp[c];
+        S.r0[cb] = make_float4(rx, ry, rz, wgt);
+        S.pid[cb] = cpid[c];
+        S.parent[cb] = slot;
+        S.meta[cb] = ((gen + 1) & 0xFFFF) | ((want + 1) << 16) | (c << 24);
+        S.shower[cb] = shower;
+        S.sid[cb] = csid[c];
       } else {
         ++n_ovf;
       }
       ++cb;
     }
-    // lane 0's writes above are read by the whole wave when a child is popped
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    // the higher-energy child below, the lower-energy one on top
-    const int lower = (cslot[0] >= 0 && cslot[1] >= 0 && lab[1].e < lab[0].e) ? 1 : 0;
+    // the stores above are read by other lanes of the wave
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    // the lane goes on with its higher-energy child, unless the wave stops
+    const int lower = (cslot[0] >= 0 && cslot[1] >= 0) ? (lab[1].e < lab[0].e ? 1 : 0) : (cslot[0] >= 0 ? 1 : 0);
+    const int higher = 1 - lower;
+    const int32_t hs = higher ? cslot[1] : cslot[0], ls = higher ? cslot[0] : cslot[1];
+    const bool go_on = hs >= 0 && !stop;
     for (int t = 0; t < 2; ++t) {
-      const int c = t == 0 ? 1 - lower : lower;
-      if (cslot[c] < 0) continue;
-      if (st.sp < depth) {
-        st.push(cslot[c], lane);
-      } else {
+      const int32_t v = t == 0 ? (go_on ? -1 : hs) : ls;
+      const unsigned long long pm = __ballot(v >= 0);
+      if (!pm) continue;
+      const int at = sp + __popcll(pm & below);
+      if (v >= 0 && at < depth) W.stack[at] = v;
+      const unsigned long long om = __ballot(v >= 0 && at >= depth);
+      if (om) {
         unsigned long long o = 0;
-        if (lane == 0) o = atomicAdd(TPm.n_spill_out, 1ull);
-        o = shfl_u64(o, 0);
-        if ((int64_t)o < TPm.spill_cap) {
-          if (lane == 0) TPm.spill_out[o] = cslot[c];
-        } else {
-          ++n_lost;  // reported by the run as an internal error
+        if (lane == 0) o = atomicAdd(TPm.n_spill_out, (unsigned long long)__popcll(om));
+        o = shfl_u64(o, 0) + (unsigned long long)__popcll(om & below);
+        if (v >= 0 && at >= depth) {
+          if ((int64_t)o < TPm.spill_cap) TPm.spill_out[o] = v;
+          else ++n_lost;  // reported by the run as an internal error
         }
+      }
+      sp = min(depth, sp + __popcll(pm));
+    }
+    if (go_on) {
+      slot = hs;
+      pid = higher ? cpid[1] : cpid[0];
+      sid = higher ? csid[1] : csid[0];
+      gen = (gen + 1) & 0xFFFF;
+      start(higher ? cp[1] : cp[0], make_float4(rx, ry, rz, wgt));
+    }
+  }
+  // ---- what the wave did not start goes to the next launch, and so do the
+  // items no wave claimed (a handed-on one starts over there: its random
+  // numbers are indexed by its substeps, so it ends the same)
+  while (!exhausted) {
+    unsigned long long c = 0;
+    if (lane == 0) c = atomicAdd(counters + C_TRANSPORT, 64ull);
+    c = shfl_u64(c, 0);
+    exhausted = (int64_t)c + 64 >= total;
+    const int64_t have = min((int64_t)64, max((int64_t)0, total - (int64_t)c));
+    if (have == 0) break;
+    unsigned long long o = 0;
+    if (lane == 0) o = atomicAdd(TPm.n_spill_out, (unsigned long long)have);
+    o = shfl_u64(o, 0);
+    if (lane < have) {
+      const int64_t rr = (int64_t)c + lane;
+      const int32_t v = rr < nres ? rin[rr].slot
+                                  : (rr < nres + n ? (int32_t)(first + (rr - nres)) : TPm.spill_in[rr - nres - n]);
+      if ((int64_t)(o + lane) < TPm.spill_cap) TPm.spill_out[o + lane] = v;
+      else ++n_lost;
+    }
+  }
+  if (sp > 0) {
+    unsigned long long o = 0;
+    if (lane == 0) o = atomicAdd(TPm.n_spill_out, (unsigned long long)sp);
+    o = shfl_u64(o, 0);
+    for (int e = lane; e < sp; e += 64) {
+      if ((int64_t)(o + e) < TPm.spill_cap) TPm.spill_out[o + e] = W.stack[e];
+      else ++n_lost;
+    }
+  }
+  {
+    unsigned long long* const st = counters + C_STATS;
+    const unsigned long long v[7] = {steps, steps, n_fail, n_drop, n_ovf, n_lost, 0ull};
+    unsigned long long* const dst[7] = {st + ST_STEPS, counters + C_TAIL_STEPS, st + ST_NOSAMPLE, st + ST_DROPPED,
+                                        st + ST_OVERFLOW, st + ST_REQ_OVERFLOW, st};
+    block_stat_add<7>(v, dst);
+  }
+  if (threadIdx.x < 8) {
+    const int q = threadIdx.x;
+    if (s_stat.draws[q]) {
+      atomicAdd(counters + C_STATS + ST_TRIALS, s_stat.trials[q]);
+      atomicAdd(counters + C_STATS + ST_DRAWS, s_stat.draws[q]);
+      atomicAdd(counters + C_PTRIALS + q, s_stat.trials[q]);
+      atomicAdd(counters + C_PDRAWS + q, s_stat.draws[q]);
+      if (s_stat.viol[q]) {
+        atomicAdd(counters + C_STATS + ST_VIOL, s_stat.viol[q]);
+        atomicAdd(counters + C_PVIOL + q, s_stat.viol[q]);
       }
     }
   }
-  if (lane == 0) {
-    if (steps) {
-      atomicAdd(counters + C_STATS + ST_STEPS, steps);
-      atomicAdd(counters + C_TAIL_STEPS, steps);
-    }
-    if (n_draws) atomicAdd(counters + C_STATS + ST_DRAWS, n_draws);
-    if (n_trials) atomicAdd(counters + C_STATS + ST_TRIALS, n_trials);
-    if (n_viol) atomicAdd(counters + C_STATS + ST_VIOL, n_viol);
-    if (n_fail) atomicAdd(counters + C_STATS + ST_NOSAMPLE, n_fail);
-    if (n_drop) atomicAdd(counters + C_STATS + ST_DROPPED, n_drop);
-    if (n_ovf) atomicAdd(counters + C_STATS + ST_OVERFLOW, n_ovf);
-    if (n_lost) atomicAdd(counters + C_STATS + ST_REQ_OVERFLOW, n_lost);
-  }
+}
+
+// Iterations of a wave in walk launch number i (from 0): `budget` particles per
+// lane in the first, twice as many in each later one, so that particles are
+// spread often while their number grows and seldom once a few long chains
+// remain (a spread costs a launch, and leaves a chain among other particles);
+// budgets above 2^30 never stop a wave.
+static int64_t tail_limit(int32_t budget, int64_t i) {
+  if (budget > (1 << 30)) return (int64_t)1 << 62;
+  return (int64_t)std::max(budget, 1) * kTailStepsPerParticle << std::min<int64_t>(i, 20);
 }
 
 // Start of a tail launch: the items are the particles handed on by the last
