@@ -58,6 +58,7 @@ enum CounterIdx {
   C_DARK_N = 20,              // dark entries written in the current pass
   C_DARK_STATS = 21,          // [3] drate rows summing to zero, vectors written, bound-electron momentum failures
   C_MESON_N = 24,             // meson-decay entries written in the current pass
+  C_LONG = 25,                // draws handed to k_draw_long
   C_YIELD_OUT = 26,           // particles the current sweep's transport handed on to the next sweep
   C_RPARITY = 27,             // which half of the resume buffer the current sweep reads
   C_SPILL = 28,               // [2] depth-first walk: entries in each spill list
@@ -70,6 +71,19 @@ enum CounterIdx {
   C_N = C_REFILL + kCtrLine * PETITE_NPROC
 };
 __host__ __device__ constexpr int refill_ctr(int p) { return C_REFILL + kCtrLine * p; }
+
+// A request whose draw outlasts its launch's queue (see k_draw_long).
+struct LongDraw {
+  double E, mf;
+  uint64_t sid;
+  const float* base;  // its map slice
+  int64_t oidx;       // result index
+  uint32_t next;      // candidates below next are rejected or being tested
+  uint32_t win;       // the lowest accepted candidate found so far
+};
+constexpr int64_t kLongCap = 1 << 16;  // one per lane group of a whole-GPU launch
+constexpr int kLongRounds = 16;        // rounds after the queue is empty
+constexpr int kFreeRounds = 32;        // rounds a lane group waits for others to refill with
 
 // One launch of the accept/reject kernel.  Requests sit in per-process
 // regions (region p holds count[p] entries from p * req_cap); each block
@@ -93,6 +107,7 @@ struct DrawLaunch {
   int32_t full_blocks;         // blocks of a whole-GPU launch (device plan)
   int32_t min_lg;              // log2 of the fewest lanes per request
   int32_t group_requests;      // requests a lane group is sized to serve (small counts)
+  LongDraw* longs;             // non-null: list of kLongCap draws handed to k_draw_long
 };
 
 // Launch plan of one process's draw kernel: groups of 2^lg lanes share a
@@ -209,7 +224,7 @@ __device__ inline double integrand_p(const DevTables& T, double E, const double*
   if (P == MUONE) return f_muone(E, T.d->Ee_min, x[0]);
   if (P == DARKBREM) return f_dark_brem(E, kMe, T.d->mV, T.d->mT, T.d->Z, T.d->A, x);
   if (P == DARKMUONBREM) return f_dark_brem(E, kMmu, T.d->mV, T.d->mT, T.d->Z, T.d->A, x);
-  if (P == DARKANN) return f_dark_ann(E, T.d->mV, x[0]);
+  if (P == DARKANN) return (double)f_dark_ann_f32(E, T.d->mV, x[0]);
   if (P == DARKCOMP) return f_compton(E, T.d->mV, x[0]);
   return 0.0;
 }
@@ -228,19 +243,22 @@ __device__ inline bool draw_possible(const DevTables& T) {
   return true;
 }
 
-// The float64 reference-order integrand of a 4-D process (see f_brem_ref).
+// The float64 reference-order integrand of a process whose candidates are
+// judged in float32 first (see f_brem_ref, f_dark_ann_f32).
 template <int P>
 __device__ inline double integrand_ref(const DevTables& T, double E, const double* x) {
   if (P == BREM) return f_brem_ref(T, E, kMe, x[0], x[1], x[2], x[3]);
   if (P == MUONBREM) return f_brem_ref(T, E, kMmu, x[0], x[1], x[2], x[3]);
   if (P == PAIRPROD) return f_pairprod_ref(T, E, x[0], x[1], x[2], x[3]);
+  if (P == DARKANN) return f_dark_ann_ref(E, T.d->mV, x[0]);
   return integrand_p<P>(T, E, x);
 }
 
 // Relative band around the accept threshold max_F * u in which a float32
-// J*f of a 4-D process is re-evaluated in float64: the float32 bodies agree
-// with the float64 reference formula to 5e-6 (99th percentile) and 2e-5
-// (99.9th), so outside the band the two make the same decision.
+// J*f of a 4-D process or of DarkAnn is re-evaluated in float64: the float32
+// bodies agree with the float64 reference formula to 5e-6 (99th percentile) and
+// 2e-5 (99.9th; DarkAnn 5e-5 at most), so outside the band the two make the
+// same decision.
 constexpr double kRefBand = 4.0e-4;
 
 template <int P, int ND>
@@ -285,6 +303,8 @@ __device__ void draw_loop(const DevTables& T, const DrawLaunch& io, uint64_t see
   q.chunk = (int)min((int64_t)64, max((int64_t)(64 >> lgG), count / (16 * (int64_t)blocks)));
   bool have = false, done = false;
   bool drained = false;  // wave-uniform: the request queue is empty
+  int late = 0;          // rounds since
+  int idle = 0;          // rounds with a group free and less than half of them
   double E = 0.0, mf = 0.0;
   uint64_t sid = 0;
   const float* base = T.f32;
@@ -292,11 +312,13 @@ __device__ void draw_loop(const DevTables& T, const DrawLaunch& io, uint64_t see
   int64_t oidx = 0;
   unsigned long long n_trials = 0, n_viol = 0, n_fail = 0, n_draw = 0;
   while (true) {
-    // refill once half of the groups are free (or none has a request): the
-    // refill's loads and table searches cost a whole-wave pass each time
+    // refill once half of the groups are free (or none has a request, or one
+    // has been free for kFreeRounds rounds): the refill's loads and table
+    // searches cost a whole-wave pass each time
     const bool need = (gl == 0) && !have && !done;
     const unsigned long long nm = __ballot(need);
-    if (nm && !drained && (__popcll(nm) >= (32 >> lgG) || __ballot(have) == 0ull)) {
+    if (nm && !drained && (__popcll(nm) >= (32 >> lgG) || ++idle >= kFreeRounds || __ballot(have) == 0ull)) {
+      idle = 0;
       const int64_t r = q.take(nm, need, io.counters + refill_ctr(p));
       if (need) {
         if (r < count) {
@@ -354,15 +376,32 @@ __device__ void draw_loop(const DevTables& T, const DrawLaunch& io, uint64_t see
         gl = lane & (G - 1);
         g0 = lane - gl;
       }
+      if (p == DARKANN && io.longs && ++late > kLongRounds) {
+        // what is left may take a million candidates: to all the waves of
+        // k_draw_long
+        unsigned long long at = kLongCap;
+        if (have && gl == 0) {
+          at = atomicAdd(io.counters + C_LONG, 1ull);
+          if (at < (unsigned long long)kLongCap) io.longs[at] = LongDraw{E, mf, sid, base, oidx, j, 0xFFFFFFFFu};
+        }
+        if (shfl_u64(at, g0) < (unsigned long long)kLongCap) have = false;
+        if (__ballot(have) == 0ull) break;
+      }
     }
     const unsigned long long gmask = (G == 64) ? ~0ull : (((1ull << G) - 1ull) << g0);
     double x[4] = {0.0, 0.0, 0.0, 0.0};
     double w = 0.0, ua = 1.0, J = 0.0;
+    bool exact = true;
     const uint32_t jc = j + (uint32_t)gl;
     if (have) {
       w = candidate_w<p, ND>(T, E, base, ninc, seed, sid, jc, x, ua, J);
       // near the threshold the decision is the float64 reference formula's
+      // (DarkAnn: also where the float32 body has no value)
       if (ND == 4 && fabs(mf * ua - w) <= kRefBand * w) w = J * integrand_ref<p>(T, E, x);
+      if (p == DARKANN) {
+        exact = !(fabs(mf * ua - w) > kRefBand * w);
+        if (exact) w = J * integrand_ref<p>(T, E, x);
+      }
     }
     const bool acc = have && (jc < max_trials) && (mf * ua < w);
     const unsigned long long am = __ballot(acc) & gmask;
@@ -370,6 +409,7 @@ __device__ void draw_loop(const DevTables& T, const DrawLaunch& io, uint64_t see
       if (am) {
         const int win = __ffsll((long long)am) - 1;
         if (lane == win) {
+          if (p == DARKANN && !exact) w = J * integrand_ref<p>(T, E, x);  // the J f that is handed out
           float* xo = io.x_out + 4 * oidx;
           xo[0] = (float)x[0];
           xo[1] = (float)x[1];
@@ -429,6 +469,110 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     if (io.count[P] <= 0) return;
     draw_loop<P>(T, io, seed, io.count[P], io.lgG[P], (int)gridDim.x);
   }
+}
+
+// The draws that outlast their launch: DarkAnn's maps leave acceptances down to
+// 1e-6 at some energies, so a few thousand requests of a batch take up to a
+// million candidates each after the others are through, and their waves would
+// work them alone.  Here every wave takes the next kLongRun x 64 candidates of
+// an open request, again and again, and the lowest accepted candidate is the
+// one draw_sample's sequential loop accepts: a request is open until one is
+// found, and every run below it has been taken by then.  The waves spread over
+// the open requests of a window of 64 each; no wave waits for another, and
+// every look either takes a run or passes on to the next window, so all end.
+// Dark vectors of 2,000 showers of 5-12 GeV at m_V = 30 MeV: 18.5 ms a call
+// without it (and the float64 integrand throughout), 3.8 with both steps; at
+// 10 MeV 145 -> 15 ms.
+constexpr int kLongRun = 8;
+template <int P>
+__global__ __launch_bounds__(256) void k_draw_long(DevTables T, DrawLaunch io, uint64_t seed) {
+  constexpr int ND = proc_ndim<P>();
+  const int64_t n = (int64_t)min(io.counters[C_LONG], (unsigned long long)kLongCap);
+  if (n == 0) return;
+  const int lane = threadIdx.x & 63;
+  const int64_t wave = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int64_t windows = (n + 63) / 64;
+  const PetiteGridDesc& gd = T.d->grid[P];
+  const int32_t ninc[4] = {gd.ninc[0], gd.ninc[1], gd.ninc[2], gd.ninc[3]};
+  const uint32_t max_trials = (uint32_t)(T.d->max_trials < (int64_t)0x7FFFFFF0 ? (T.d->max_trials > 0 ? T.d->max_trials : 1)
+                                                                               : (int64_t)0x7FFFFFF0);
+  int64_t w0 = wave % windows;
+  int pick = (int)(wave / windows);
+  for (int64_t empty = 0; empty < windows;) {
+    bool open = false;
+    if (w0 * 64 + lane < n) {
+      LongDraw& q = io.longs[w0 * 64 + lane];
+      open = __hip_atomic_load(&q.win, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0xFFFFFFFFu &&
+             __hip_atomic_load(&q.next, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < max_trials;
+    }
+    const unsigned long long om = __ballot(open);
+    if (om == 0ull) {
+      w0 = w0 + 1 < windows ? w0 + 1 : 0;
+      ++empty;
+      continue;
+    }
+    empty = 0;
+    LongDraw& R = io.longs[w0 * 64 + nth_lane(om, pick++ % __popcll(om))];
+    const double E = R.E, mf = R.mf;
+    const uint64_t sid = R.sid;
+    const float* base = R.base;
+    uint32_t j = 0;
+    if (lane == 0) j = atomicAdd(&R.next, 64u * kLongRun);
+    j = __shfl(j, 0);
+    for (int k = 0; k < kLongRun && j < max_trials; ++k, j += 64u) {
+      const uint32_t jc = j + (uint32_t)lane;
+      double x[4] = {0.0, 0.0, 0.0, 0.0};
+      double ua = 1.0, J = 0.0;
+      double w = candidate_w<P, ND>(T, E, base, ninc, seed, sid, jc, x, ua, J);
+      if (!(fabs(mf * ua - w) > kRefBand * w)) w = J * integrand_ref<P>(T, E, x);
+      const unsigned long long am = __ballot(jc < max_trials && mf * ua < w);
+      if (am) {
+        if (lane == __ffsll((long long)am) - 1) atomicMin(&R.win, jc);
+        break;
+      }
+    }
+  }
+}
+
+template <int P>
+__global__ __launch_bounds__(256) void k_draw_long_finish(DevTables T, DrawLaunch io, uint64_t seed) {
+  constexpr int ND = proc_ndim<P>();
+  const int64_t n = (int64_t)min(io.counters[C_LONG], (unsigned long long)kLongCap);
+  const int64_t q0 = (int64_t)blockIdx.x * blockDim.x;
+  if (q0 >= n) return;
+  const int64_t q = q0 + threadIdx.x;
+  unsigned long long n_trials = 0, n_draw = 0, n_viol = 0, n_fail = 0;
+  if (q < n) {
+    const LongDraw R = io.longs[q];
+    const PetiteGridDesc& gd = T.d->grid[P];
+    const int32_t ninc[4] = {gd.ninc[0], gd.ninc[1], gd.ninc[2], gd.ninc[3]};
+    const uint32_t max_trials = (uint32_t)(T.d->max_trials < (int64_t)0x7FFFFFF0
+                                               ? (T.d->max_trials > 0 ? T.d->max_trials : 1) : (int64_t)0x7FFFFFF0);
+    n_draw = 1;
+    if (R.win < max_trials) {
+      double x[4] = {0.0, 0.0, 0.0, 0.0};
+      double ua = 1.0, J = 0.0;
+      (void)candidate_w<P, ND>(T, R.E, R.base, ninc, seed, R.sid, R.win, x, ua, J);
+      const double w = J * integrand_ref<P>(T, R.E, x);
+      float* xo = io.x_out + 4 * R.oidx;
+      for (int d = 0; d < 4; ++d) xo[d] = (float)x[d];
+      io.trials_out[R.oidx] = (int32_t)(R.win + 1u);
+      io.w_out[R.oidx] = (float)w;
+      n_trials = R.win + 1u;
+      n_viol = w > R.mf ? 1 : 0;
+    } else {
+      io.trials_out[R.oidx] = -(int32_t)max_trials;
+      io.w_out[R.oidx] = 0.0f;
+      n_trials = max_trials;
+      n_fail = 1;
+    }
+  }
+  unsigned long long* const ctr = io.counters;
+  const unsigned long long v[7] = {n_trials, n_draw, n_viol, n_fail, n_trials, n_draw, n_viol};
+  unsigned long long* const dst[7] = {ctr + C_STATS + ST_TRIALS, ctr + C_STATS + ST_DRAWS, ctr + C_STATS + ST_VIOL,
+                                      ctr + C_STATS + ST_NOSAMPLE, ctr + C_PTRIALS + P, ctr + C_PDRAWS + P,
+                                      ctr + C_PVIOL + P};
+  block_stat_add<7>(v, dst);
 }
 
 typedef void (*DrawKernel)(DevTables, DrawLaunch, uint64_t);
@@ -1656,6 +1800,7 @@ struct PetiteCtx {
   ResumeRec* dresume = nullptr;  // [2][resume_cap]
   int64_t resume_cap = 0;
   int32_t* tail_spill = nullptr;  // [2][kTailSpill]: depth-first walk spill lists
+  LongDraw* longs = nullptr;      // [kLongCap], contexts with a DarkAnn map
   std::vector<hipEvent_t> tev;
   int n_cu = 256;
   PetiteTuning tune{};  // launch and queue sizes in effect (defaults filled in)
@@ -1818,6 +1963,11 @@ static void plan_draw(PetiteCtx* c, const unsigned int* rq, DrawLaunch& io, int6
 
 static int ensure_draw_streams(PetiteCtx* c);
 
+static int ensure_longs(PetiteCtx* c) {
+  if (!c->longs && c->desc.grid[DARKANN].n_E > 0) HIP_TRY(hipMalloc(&c->longs, kLongCap * sizeof(LongDraw)));
+  return PETITE_OK;
+}
+
 // The per-process kernels are independent: with more than one, each runs on
 // its own stream so small processes overlap the large ones.
 static int launch_draws(PetiteCtx* c, const DrawLaunch& io, uint64_t seed, hipStream_t s) {
@@ -1841,6 +1991,13 @@ static int launch_draws(PetiteCtx* c, const DrawLaunch& io, uint64_t seed, hipSt
     }
     hipLaunchKernelGGL(kDrawKernels[p], dim3((unsigned)b), dim3(256), 0, sp, c->dev, io, seed);
     HIP_TRY(hipGetLastError());
+    if (p == DARKANN && io.longs) {
+      hipLaunchKernelGGL(k_draw_long<DARKANN>, dim3((unsigned)c->n_cu * 4), dim3(256), 0, sp, c->dev, io, seed);
+      HIP_TRY(hipGetLastError());
+      hipLaunchKernelGGL(k_draw_long_finish<DARKANN>, dim3((unsigned)(kLongCap / 256)), dim3(256), 0, sp, c->dev, io,
+                         seed);
+      HIP_TRY(hipGetLastError());
+    }
     if (na > 1) HIP_TRY(hipEventRecord(c->djoin[p], sp));
   }
   for (int i = 0; na > 1 && i < na; ++i) HIP_TRY(hipStreamWaitEvent(s, c->djoin[active[i]], 0));
@@ -2067,7 +2224,7 @@ void petite_ctx_destroy(PetiteCtx* c) {
                   (void*)c->res_trials, (void*)c->res_w, (void*)c->req_count, (void*)c->counters, (void*)c->ddesc,
                   (void*)c->dsig_lds, (void*)c->dark_blob, (void*)c->dyield, (void*)c->yield_blob, (void*)c->yacc, (void*)c->ylist, (void*)c->ylist_cnt, (void*)c->ytab_dev,
                   (void*)c->bnd_blob, (void*)c->bnd_tab, (void*)c->bnd_slots, (void*)c->bnd_jobs, (void*)c->bnd_bad,
-                  (void*)c->par.sid, (void*)c->par.pf, (void*)c->par.pos, (void*)c->par.info, (void*)c->tail_spill})
+                  (void*)c->par.sid, (void*)c->par.pf, (void*)c->par.pos, (void*)c->par.info, (void*)c->tail_spill, (void*)c->longs})
     if (p) (void)hipFree(p);
   free_entries(c);
   delete c;
@@ -2191,6 +2348,7 @@ int petite_vegas_draw(PetiteCtx* c, const int32_t* proc, const double* E, const 
   if (n > INT32_MAX) return fail(PETITE_ERR_ARG, "petite_vegas_draw: more than 2^31-1 requests");
   hipStream_t s = (hipStream_t)stream;
   int rc = ensure_requests(c, n);
+  if (!rc) rc = ensure_longs(c);
   if (rc) return rc;
   HIP_TRY(hipMemsetAsync(c->counters, 0, C_N * sizeof(unsigned long long), s));
   HIP_TRY(hipMemsetAsync(c->req_count, 0, PETITE_NPROC * sizeof(unsigned int), s));
@@ -2210,6 +2368,7 @@ int petite_vegas_draw(PetiteCtx* c, const int32_t* proc, const double* E, const 
   io.trials_out = trials_out;
   io.w_out = w_out;
   io.counters = c->counters;
+  io.longs = c->longs;
   int64_t blocks = 0;
   plan_draw(c, rq, io, blocks);
   rc = launch_draws(c, io, seed, s);
@@ -2855,6 +3014,7 @@ int petite_dark_reweight(PetiteCtx* c, const PetiteStore* sm, int64_t n_sm, uint
   int rc = ensure_entries(c, chunk * na);
   if (rc) return rc;
   rc = ensure_requests(c, chunk * na);
+  if (!rc) rc = ensure_longs(c);
   if (rc) return rc;
   unsigned long long* ctr = c->counters;
   HIP_TRY(hipMemsetAsync(c->dyield, 0, 5 * sizeof(double), s));
@@ -2873,6 +3033,7 @@ int petite_dark_reweight(PetiteCtx* c, const PetiteStore* sm, int64_t n_sm, uint
     if (sm_dark) {
       HIP_TRY(hipMemsetAsync(c->req_count, 0, PETITE_NPROC * sizeof(unsigned int), s));
       HIP_TRY(hipMemsetAsync(ctr + C_DARK_N, 0, sizeof(unsigned long long), s));
+      HIP_TRY(hipMemsetAsync(ctr + C_LONG, 0, sizeof(unsigned long long), s));
       HIP_TRY(hipMemsetAsync(ctr + C_REFILL, 0, kCtrLine * PETITE_NPROC * sizeof(unsigned long long), s));  // draw refill
       Requests R{c->req_slot, c->req_E, c->req_cap, c->req_count};
       if (c->timing) HIP_TRY(hipEventRecord(c->ev[0], s));
@@ -2899,6 +3060,7 @@ int petite_dark_reweight(PetiteCtx* c, const PetiteStore* sm, int64_t n_sm, uint
       io.trials_out = c->dres_trials;
       io.w_out = c->dres_w;
       io.counters = ctr;
+      io.longs = c->longs;
       int64_t blocks = 0;
       plan_draw(c, rq, io, blocks);
       if (c->timing) HIP_TRY(hipEventRecord(c->ev[2], s));
