@@ -970,6 +970,37 @@ struct LdsSigma {
       default: return 0.0;
     }
   }
+  // One channel's header in registers, and its value when the table has a node
+  // index: nsigma's arithmetic without branches, so that the lookups of a sum
+  // and the work beside them overlap.  (A lane whose E lies outside the table,
+  // or whose channel is empty, reads records inside the tables and gets 0.)
+  struct Channel {
+    float log2E0, per;
+    int rec, nm1;
+    double lo, hi;
+  };
+  __device__ inline Channel channel(uint32_t p) const {
+    const double* h = base + kLdsHeader * (p == 0xFu ? 0u : p);
+    const long long w0 = __double_as_longlong(h[0]), w1 = __double_as_longlong(h[1]);
+    Channel c;
+    c.log2E0 = __int_as_float((int)w0);
+    c.per = __int_as_float((int)(w0 >> 32));
+    const int n1 = (int)(w1 >> 32);
+    c.rec = n1 < 0 ? (int)(h - base) : (int)w1;  // no table: its own header
+    c.nm1 = max(n1, 0);
+    c.lo = p == 0xFu ? 1.0 : h[2];
+    c.hi = p == 0xFu ? 0.0 : h[3];
+    return c;
+  }
+  __device__ inline double indexed(const Channel& c, double E, float l2) const {
+    int j = (int)((l2 - c.log2E0) * c.per + 0.5f);
+    j = min(max(j, 0), c.nm1);
+    const double* r = base + c.rec + 4 * j;
+    const double va = r[3] * (E - r[0]) + r[2];
+    const double vb = r[7] * (E - r[4]) + r[6];
+    const double v = E >= r[4] ? vb : va;
+    return (E >= c.lo) & (E <= c.hi) ? v : 0.0;
+  }
   // The same sums for a lane's charged species from its channel word (see
   // sum_channels): every lane runs the same two lookups, positrons a third,
   // so a wave that mixes species does not run each species' sum in turn.
@@ -1008,16 +1039,17 @@ __device__ inline void mcs_rotate(const DevTables& T, float& nx, float& ny, floa
   const Frame f = frame_of(nx, ny, nz);
   float ox, oy, oz;
   frame_apply(f, sph * sth, -cph * sth, cth, ox, oy, oz);
-  const float inv = rsqrtf(ox * ox + oy * oy + oz * oz);
+  const float inv = rsqrtf(norm2(ox, oy, oz));
   nx = ox * inv;
   ny = oy * inv;
   nz = oz * inv;
 }
 
-// |p| of energy E and mass m.  fmax: contracted to fma(E, E, -(m*m)), E*E -
-// m*m at E == m is minus the rounding error of m*m, which can be negative (the
-// reference's p is 0 there).
-__device__ inline double momentum(double E, double m) { return sqrt(fmax(E * E - m * m, 0.0)); }
+// |p|^2 and |p| of energy E and mass m.  fmax: as an fma, E*E - m*m at E == m is
+// minus the rounding error of m*m, which can be negative (the reference's p is
+// 0 there).
+__device__ inline double momentum2(double E, double m) { return fmax(__fma_rn(E, E, -(m * m)), 0.0); }
+__device__ inline double momentum(double E, double m) { return sqrt(momentum2(E, m)); }
 
 // Moves a charged particle by ``dist`` after losing dEdx*dist (lose_energy,
 // particle.py:143-153) and scatters it (shower.py:569-581, 589-598).  The
@@ -1027,9 +1059,9 @@ __device__ inline void charged_advance(const DevTables& T, double dist, double m
                                        uint32_t w_a, double& E, float& nx, float& ny, float& nz, float& rx,
                                        float& ry, float& rz, double& dep) {
   const double Eb = E;
-  E = E - T.d->dEdx * dist;
+  E = __fma_rn(-T.d->dEdx, dist, E);
   if (E <= m) E = m;
-  const double q = fmax(E * E - m * m, 0.0);  // p^2, as momentum() forms it
+  const double q = momentum2(E, m);
   dep += Eb - E;
   if (q > 0.0) {
     rx += (float)(nx * dist);
@@ -1158,7 +1190,7 @@ __global__ __launch_bounds__(256) void k_transport(DevTables T, DevStore S, int6
           nx = p0.y;
           ny = p0.z;
           nz = p0.w;
-          const float pn2 = nx * nx + ny * ny + nz * nz;
+          const float pn2 = norm2(nx, ny, nz);
           if (pn2 > 0.0f) {
             const float inv = rsqrtf(pn2);
             nx *= inv;
@@ -2150,6 +2182,7 @@ int petite_ctx_create(const PetiteTableDesc* desc, const double* blob64, int64_t
       return u;
     };
     std::vector<double> lds(kLdsHeader * PETITE_NPROC, 0.0);
+    T.sig_indexed = 1;
     for (int p = 0; p < PETITE_NPROC; ++p) {
       const PetiteSigmaDesc& sd = desc->sigma[p];
       const int n = sd.n > 0 ? sd.n : 0;
@@ -2164,7 +2197,10 @@ int petite_ctx_create(const PetiteTableDesc* desc, const double* blob64, int64_t
       h[2] = x[0];
       h[3] = x[n - 1];
       h[4] = y[0];
-      if (n == 1) continue;
+      if (n == 1) {
+        if (p < kNprocSM) T.sig_indexed = 0;
+        continue;
+      }
       // records -1 .. n-1: record -1 and n-1 repeat records 0 and n-2
       const size_t rec_m1 = lds.size();
       for (int i = -1; i <= n - 1; ++i) {
@@ -2183,6 +2219,7 @@ int petite_ctx_create(const PetiteTableDesc* desc, const double* blob64, int64_t
         for (int k = 0; k < n && per > 0.0f; ++k)
           if (!(x[k] > 0.0) || !(std::fabs((std::log2(x[k]) - (double)log2E0) * (double)per - k) < 0.4)) per = 0.0f;
       }
+      if (p < kNprocSM && !(per > 0.0f)) T.sig_indexed = 0;
       // (the appends above may have moved the vector: index it afresh)
       lds[kLdsHeader * p + 0] = pack(fbits(log2E0), fbits(per));
       lds[kLdsHeader * p + 1] = pack((uint32_t)rec_m1, (uint32_t)(n - 1));

@@ -41,6 +41,7 @@ struct DevTables {
   float mcs_cB;        //   2.007e-5 Z^(2/3),
   float mcs_cC;        //   3.34 (Z alpha)^2  (moliere.py:196-219)
   int32_t lds_doubles; // size of the n*sigma tables staged in LDS by the transport kernel
+  int32_t sig_indexed; // every SM n*sigma table is empty or has a node index (LdsSigma::indexed)
   const PetiteTableDesc* d;  // device copy of the descriptor (read through the scalar cache)
 };
 

@@ -160,8 +160,9 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
   const int depth = TPm.depth < 1 ? 1 : (TPm.depth > kTailMaxDepth ? kTailMaxDepth : TPm.depth);
   // more items than half a spill list holds are all walked in this launch
   const int64_t limit = total > TPm.spill_cap / 2 ? (int64_t)1 << 62 : TPm.limit;
-  // lane states: empty, stepping, at its end (parked)
-  enum { EMPTY = 0, STEP = 1, PARKED = 2 };
+  // lane states: empty, stepping, at its end (parked), given a particle that
+  // has not started
+  enum { EMPTY = 0, STEP = 1, PARKED = 2, GIVEN = 3 };
   int mode = EMPTY;
   int sp = 0;              // stack entries (wave-uniform, as the next four)
   int64_t iters = 0;
@@ -175,45 +176,6 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
   uint32_t k = 0;
   bool closing = false;
   unsigned long long steps = 0, n_fail = 0, n_drop = 0, n_ovf = 0, n_lost = 0;
-  // puts the lane on a particle of species pid at its start (k_transport's refill)
-  auto start = [&](float4 p0, float4 r0) {
-    ch = sum_channels(pid);
-    m = pid_mass(pid);
-    pme = fmax(fmax(min_calc(T, pid), T.d->min_energy), m);
-    E = (double)p0.x;
-    nx = p0.y;
-    ny = p0.z;
-    nz = p0.w;
-    const float pn2 = nx * nx + ny * ny + nz * nz;
-    if (pn2 > 0.0f) {
-      const float inv = rsqrtf(pn2);
-      nx *= inv;
-      ny *= inv;
-      nz *= inv;
-    }
-    const bool still = ch == 0xFFFu && pid != 22;
-    p = still ? sqrt((double)pn2) : 0.0;  // the others' |p| is formed when they finish
-    rx = r0.x;
-    ry = r0.y;
-    rz = r0.z;
-    wgt = r0.w;
-    dep = 0.0;
-    k = 0;
-    closing = false;
-    mode = STEP;
-    if (E < pme || still) {
-      mode = PARKED;  // ends where it starts (shower.py:532-536, 640-653)
-    } else if (pid == 22) {
-      // one exponential flight, no MCS (shower.py:538-553)
-      const double mfp = L.mfp(22, E);
-      const double dist = -mfp * (double)log1p_f32(-u01f(draw_block(seed, sid, 0, PURPOSE_STEP).x));
-      rx += (float)(nx * dist);
-      ry += (float)(ny * dist);
-      rz += (float)(nz * dist);
-      k = 1;
-      mode = PARKED;
-    }
-  };
   while (true) {
     // past its share the wave starts no more: the next launch spreads what it
     // leaves.  A wave whose particles all have lanes and include a muon goes on:
@@ -223,11 +185,11 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
     // ---- free lanes take from the stack, then claim items (after a draw
     // phase, or when no lane is stepping)
     const unsigned long long im = __ballot(mode == EMPTY);
+    int64_t rr = -1;
     if (im && !stop && (fresh || __ballot(mode == STEP) == 0ull)) {
       const int rank = __popcll(im & below);
       const int take = min(__popcll(im), sp);
       bool got = false;
-      int64_t rr = -1;
       if (mode == EMPTY && rank < take) {
         slot = W.stack[sp - 1 - rank];
         got = true;
@@ -247,79 +209,130 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
         exhausted = (int64_t)c + need >= total;
       }
       if (got) {
+        const float4 p0 = S.p0[slot], r0 = S.r0[slot];
         pid = S.pid[slot];
         sid = S.sid[slot];
         shower = S.shower[slot];
         gen = S.meta[slot] & 0xFFFF;
-        const float4 r0 = S.r0[slot];
-        start(S.p0[slot], r0);
-        if (rr >= 0 && rr < nres) {
-          // handed on by the last sweep: its live state
-          const ResumeRec& R0 = rin[rr];
-          E = R0.E;
-          dep = R0.dep;
-          dz = R0.dz;
-          nx = R0.nx;
-          ny = R0.ny;
-          nz = R0.nz;
-          rx = R0.rx;
-          ry = R0.ry;
-          rz = R0.rz;
-          k = R0.k;
-          mode = STEP;
-        }
+        E = (double)p0.x;
+        nx = p0.y;
+        ny = p0.z;
+        nz = p0.w;
+        rx = r0.x;
+        ry = r0.y;
+        rz = r0.z;
+        wgt = r0.w;
+        mode = GIVEN;
+      }
+    }
+    // ---- the given particles' starts (k_transport's refill)
+    if (mode == GIVEN) {
+      ch = sum_channels(pid);
+      m = pid_mass(pid);
+      pme = fmax(fmax(min_calc(T, pid), T.d->min_energy), m);
+      const float pn2 = norm2(nx, ny, nz);
+      if (pn2 > 0.0f) {
+        const float inv = rsqrtf(pn2);
+        nx *= inv;
+        ny *= inv;
+        nz *= inv;
+      }
+      const bool still = ch == 0xFFFu && pid != 22;
+      p = still ? sqrt((double)pn2) : 0.0;  // the others' |p| is formed when they finish
+      dep = 0.0;
+      k = 0;
+      closing = false;
+      mode = STEP;
+      if (rr >= 0 && rr < nres) {
+        // handed on by the last sweep: its live state
+        const ResumeRec& R0 = rin[rr];
+        E = R0.E;
+        dep = R0.dep;
+        dz = R0.dz;
+        nx = R0.nx;
+        ny = R0.ny;
+        nz = R0.nz;
+        rx = R0.rx;
+        ry = R0.ry;
+        rz = R0.rz;
+        k = R0.k;
+      } else if (E < pme || still) {
+        mode = PARKED;  // ends where it starts (shower.py:532-536, 640-653)
+      } else if (pid == 22) {
+        // one exponential flight, no MCS (shower.py:538-553)
+        const double mfp = L.mfp(22, E);
+        const double dist = -mfp * (double)log1p_f32(-u01f(draw_block(seed, sid, 0, PURPOSE_STEP).x));
+        rx += (float)(nx * dist);
+        ry += (float)(ny * dist);
+        rz += (float)(nz * dist);
+        k = 1;
+        mode = PARKED;
       }
     }
     fresh = false;
-    const unsigned long long am = __ballot(mode == STEP), wm = __ballot(mode == PARKED);
+    unsigned long long am = __ballot(mode == STEP), wm = __ballot(mode == PARKED);
     if (am == 0ull && wm == 0ull) break;
     // a draw phase costs several substeps (loads, a round of candidates per
     // process, the kinematics): run at two thirds of the live lanes parked it
     // measures 15 % faster than at a third over the showers of 1 to 100,000
     // primaries, and a half or four fifths are in between
     if (am != 0ull && __popcll(wm) < 2 * __popcll(am)) {
-      // ---- one advance of every stepping lane (k_transport's)
-      ++iters;
-      if (mode == STEP) {
-        const bool in_close = closing;
-        const double Ssum = L.nsigma_sum_ch(ch, E);
-        const double mfp = Ssum > 0.0 ? kCmToM / Ssum : 1.0e12;
-        const U4 u = draw_block(seed, sid, in_close ? 0u : k, in_close ? PURPOSE_CLOSE : PURPOSE_STEP);
-        bool adv = true;
-        double dist;
-        uint32_t w_r, w_a;
-        double m_lep = m;
-        if (!in_close) {
-          const double div = 6.0 + 14.0 * u01d(u.y);
-          dz = mfp / div;
-          dist = dz;
-          w_r = u.z;
-          w_a = u.w;
-          const double ux = u01d(u.x);
-          double thr = (double)__expf(-__builtin_amdgcn_rcpf((float)div));
-          if (fabs(ux - thr) < 1.0e-5) thr = exp(-(dz / mfp));
-          if (ux > thr) {
-            adv = false;
-            closing = true;
-          }
-        } else {
-          const double distC = u01d(u.x);
-          if (E < pme) {
-            dist = distC * dz;
+      // ---- advances of the stepping lanes (k_transport's) until a phase is due
+      const LdsSigma::Channel c0 = L.channel(ch & 0xFu), c1 = L.channel((ch >> 4) & 0xFu),
+                              c2 = L.channel((ch >> 8) & 0xFu);
+      do {
+        ++iters;
+        if (mode == STEP) {
+          const bool in_close = closing;
+          const U4 u = draw_block(seed, sid, in_close ? 0u : k, in_close ? PURPOSE_CLOSE : PURPOSE_STEP);
+          double Ssum;
+          if (T.sig_indexed) {
+            const float l2 = __log2f((float)E);
+            const double s01 = L.indexed(c0, E, l2) + L.indexed(c1, E, l2);
+            const double s2 = L.indexed(c2, E, l2);
+            Ssum = (ch >> 8) == 0xFu ? s01 : s01 + s2;
           } else {
-            const float r2 = Ssum > 0.0 ? (float)(dz * Ssum * (1.0 / kCmToM)) : (float)(dz * 1.0e-12);
-            dist = -mfp * (double)log1p_f32(expm1f(-r2) * (float)distC);
+            Ssum = L.nsigma_sum_ch(ch, E);
           }
-          w_r = u.y;
-          w_a = u.z;
-          m_lep = kMe;
+          const double mfp = Ssum > 0.0 ? kCmToM / Ssum : 1.0e12;
+          bool adv = true;
+          double dist;
+          uint32_t w_r, w_a;
+          double m_lep = m;
+          if (!in_close) {
+            const double div = 6.0 + 14.0 * u01d(u.y);
+            dz = mfp / div;
+            dist = dz;
+            w_r = u.z;
+            w_a = u.w;
+            const double ux = u01d(u.x);
+            double thr = (double)__expf(-__builtin_amdgcn_rcpf((float)div));
+            if (fabs(ux - thr) < 1.0e-5) thr = exp(-(dz / mfp));
+            if (ux > thr) {
+              adv = false;
+              closing = true;
+            }
+          } else {
+            const double distC = u01d(u.x);
+            if (E < pme) {
+              dist = distC * dz;
+            } else {
+              const float r2 = Ssum > 0.0 ? (float)(dz * Ssum * (1.0 / kCmToM)) : (float)(dz * 1.0e-12);
+              dist = -mfp * (double)log1p_f32(expm1f(-r2) * (float)distC);
+            }
+            w_r = u.y;
+            w_a = u.z;
+            m_lep = kMe;
+          }
+          if (adv) charged_advance(T, dist, m, m_lep, w_r, w_a, E, nx, ny, nz, rx, ry, rz, dep);
+          ++k;
+          if (in_close) mode = PARKED;
+          else if (E < pme) closing = true;
         }
-        if (adv) charged_advance(T, dist, m, m_lep, w_r, w_a, E, nx, ny, nz, rx, ry, rz, dep);
-        ++k;
-        if (in_close) mode = PARKED;
-        else if (E < pme) closing = true;
-      }
-      continue;
+        am = __ballot(mode == STEP);
+        wm = __ballot(mode == PARKED);
+      } while (am != 0ull && __popcll(wm) < 2 * __popcll(am));
+      if (wm == 0ull) continue;
     }
     // ---- the parked lanes' final states and process choices (k_transport's finish)
     iters += kTailPhaseSteps;
@@ -463,11 +476,16 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
       sp = min(depth, sp + __popcll(pm));
     }
     if (go_on) {
+      const float4 c = higher ? cp[1] : cp[0];
       slot = hs;
       pid = higher ? cpid[1] : cpid[0];
       sid = higher ? csid[1] : csid[0];
       gen = (gen + 1) & 0xFFFF;
-      start(higher ? cp[1] : cp[0], make_float4(rx, ry, rz, wgt));
+      E = (double)c.x;
+      nx = c.y;
+      ny = c.z;
+      nz = c.w;
+      mode = GIVEN;
     }
   }
   // ---- what the wave did not start goes to the next launch, and so do the

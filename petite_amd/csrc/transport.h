@@ -145,8 +145,12 @@ __device__ inline double pid_mass(int pid) {
 struct Frame {
   float c_t, s_t, c_p, s_p;
 };
+// The sums of products of the transport's float32 arithmetic are written as
+// explicit fmas: which product of a*b + c*d a compiler contracts can change
+// with the code around it, and a particle's records must not.
+__device__ inline float norm2(float x, float y, float z) { return __fmaf_rn(z, z, __fmaf_rn(x, x, y * y)); }
 __device__ inline Frame frame_of(float nx, float ny, float nz) {
-  const float rho = sqrtf(nx * nx + ny * ny);
+  const float rho = sqrtf(__fmaf_rn(nx, nx, ny * ny));
   Frame f;
   f.c_t = nz;
   f.s_t = rho;
@@ -161,9 +165,9 @@ __device__ inline Frame frame_of(float nx, float ny, float nz) {
   return f;
 }
 __device__ inline void frame_apply(const Frame& f, float lx, float ly, float lz, float& ox, float& oy, float& oz) {
-  ox = f.c_t * f.c_p * lx - f.s_p * ly + f.s_t * f.c_p * lz;
-  oy = f.c_t * f.s_p * lx + f.c_p * ly + f.s_t * f.s_p * lz;
-  oz = -f.s_t * lx + f.c_t * lz;
+  ox = __fmaf_rn(f.s_t * f.c_p, lz, __fmaf_rn(f.c_t * f.c_p, lx, -(f.s_p * ly)));
+  oy = __fmaf_rn(f.s_t * f.s_p, lz, __fmaf_rn(f.c_t * f.s_p, lx, f.c_p * ly));
+  oz = __fmaf_rn(f.c_t, lz, -(f.s_t * lx));
 }
 
 // Same rotation in float64 for the children of an interaction.
