@@ -105,7 +105,7 @@ __device__ inline double bsm_weight(const DevTables& T, const PetiteDarkDesc& D,
                                     const WeightArgs& a) {
   const double E0 = a.E0;
   if (code == DARKCOMP) {
-    if (pid != 22 || E0 < D.min_comp || E0 < T.d->min_calc[2]) return 0.0;
+    if (pid != 22 || E0 < D.min_comp || E0 < T.min_calc[2]) return 0.0;
     const double* lx = b + D.comp_off;
     const double num = loglog(lx, lx + D.comp_n, D.comp_n, a.l10, D.comp_l0, D.comp_inv_dl);
     return D.eps2 * (num / a.den);
@@ -234,7 +234,7 @@ __global__ __launch_bounds__(256) void k_dark_select(DevTables T, PetiteDarkDesc
           // scatter the initial momentum over the distance (m_lepton = m_e,
           // dark_shower.py:753-755), then lose E0 - E_int.  beta comes from the
           // on-shell |p| = sqrt(E0^2 - m^2): a float32 record's |p| can round to E0.
-          const double dist = (E0 - E_int) / T.d->dEdx;
+          const double dist = (E0 - E_int) / T.dEdx;
           const double px = p0.y, py = p0.z, pz = p0.w;
           const double pn = sqrt(px * px + py * py + pz * pz);
           const double pon = sqrt(fmax(E0 * E0 - m_part * m_part, 0.0));
@@ -379,7 +379,7 @@ __global__ __launch_bounds__(256) void k_dark_emit(DevTables T, PetiteDarkDesc D
     const int32_t slot = Q.parent[e];
     double w = Q.weight[e];
     const double E = Q.E[e];
-    const double mV = T.d->mV;
+    const double mV = T.mV;
     bool ok = state != S_NONE;
     V4 v{0.0, 0.0, 0.0, 0.0};
     if (ok && state == S_DIRECT) {
@@ -397,7 +397,7 @@ __global__ __launch_bounds__(256) void k_dark_emit(DevTables T, PetiteDarkDesc D
         if (code == DARKCOMP) {
           const U4 w1 = draw_block(seed, dsid, 1, PURPOSE_INTERACT);
           double pe = 0.0;
-          if (!draw_pe(seed, dsid, T.d->Zeff, pe)) {
+          if (!draw_pe(seed, dsid, T.Zeff, pe)) {
             ok = false;
             ++n_pe_fail;
           } else {
@@ -483,7 +483,7 @@ __global__ __launch_bounds__(kMesonBlock) void k_meson_decay(DevTables T, Petite
     const int pid = S.pid[i];
     const int k = pid == 111 ? 0 : (pid == 221 ? 1 : (pid == 331 ? 2 : -1));
     const double mM = k == 0 ? 0.1349768 : (k == 1 ? 0.547862 : 0.95778);
-    const double mV = T.d->mV;
+    const double mV = T.mV;
     if (k >= 0 && D.meson_w[k] > 0.0 && mV / mM < 1.0) {
       const double r = mV / mM;
       const double q = 1.0 - r * r;
@@ -596,7 +596,7 @@ __device__ inline double loglog10(const double* lx, const double* ly, int n, dou
 __device__ inline void yield_weight(const DevTables& T, const PetiteDarkDesc& D, const double* b, int pid, int code,
                                     const WeightArgs& a, double ln_eps2, double ln_den, double& wv, double& lam) {
   if (code == DARKCOMP) {
-    if (pid != 22 || a.E0 < D.min_comp || a.E0 < T.d->min_calc[2]) {
+    if (pid != 22 || a.E0 < D.min_comp || a.E0 < T.min_calc[2]) {
       wv = 0.0;
       lam = 0.0;
       return;
@@ -659,7 +659,7 @@ __device__ inline void bound_wd(const DevTables& T, const BoundView& B, int k, i
     }
     return;
   }
-  if (a.E0 < S.min_comp || a.E0 < T.d->min_calc[2]) return;
+  if (a.E0 < S.min_comp || a.E0 < T.min_calc[2]) return;
   const double* lx = t + 4 * n;
   const double* ly = t + 5 * n;
   const double l = a.l10;

@@ -218,14 +218,14 @@ __device__ inline double integrand_p(const DevTables& T, double E, const double*
   if (P == MUONBREM) return (double)f_brem(T, E, kMmu, T.brem_C_mu, x);
   if (P == PAIRPROD) return (double)f_pairprod(T, E, x);
   if (P == COMP) return f_compton(E, 0.0, x[0]);
-  if (P == ANN) return f_annihilation(E, 0.0, T.d->Eg_min, x[0]);
-  if (P == MOLLER) return f_moller(E, T.d->Ee_min, x[0]);
-  if (P == BHABHA) return f_bhabha(E, T.d->Ee_min, x[0]);
-  if (P == MUONE) return f_muone(E, T.d->Ee_min, x[0]);
-  if (P == DARKBREM) return f_dark_brem(E, kMe, T.d->mV, T.d->mT, T.d->Z, T.d->A, x);
-  if (P == DARKMUONBREM) return f_dark_brem(E, kMmu, T.d->mV, T.d->mT, T.d->Z, T.d->A, x);
-  if (P == DARKANN) return (double)f_dark_ann_f32(E, T.d->mV, x[0]);
-  if (P == DARKCOMP) return f_compton(E, T.d->mV, x[0]);
+  if (P == ANN) return f_annihilation(E, 0.0, T.Eg_min, x[0]);
+  if (P == MOLLER) return f_moller(E, T.Ee_min, x[0]);
+  if (P == BHABHA) return f_bhabha(E, T.Ee_min, x[0]);
+  if (P == MUONE) return f_muone(E, T.Ee_min, x[0]);
+  if (P == DARKBREM) return f_dark_brem(E, kMe, T.mV, T.mT, T.Z, T.A, x);
+  if (P == DARKMUONBREM) return f_dark_brem(E, kMmu, T.mV, T.mT, T.Z, T.A, x);
+  if (P == DARKANN) return (double)f_dark_ann_f32(E, T.mV, x[0]);
+  if (P == DARKCOMP) return f_compton(E, T.mV, x[0]);
   return 0.0;
 }
 
@@ -239,7 +239,7 @@ constexpr int proc_ndim() {
 // sqrt(1 - 4 m_e^2 / m_V^2) (all_processes.py:431) for m_V <= 2 m_e.
 template <int P>
 __device__ inline bool draw_possible(const DevTables& T) {
-  if (P == DARKANN) return T.d->mV > 2.0 * kMe;
+  if (P == DARKANN) return T.mV > 2.0 * kMe;
   return true;
 }
 
@@ -247,10 +247,10 @@ __device__ inline bool draw_possible(const DevTables& T) {
 // judged in float32 first (see f_brem_ref, f_dark_ann_f32).
 template <int P>
 __device__ inline double integrand_ref(const DevTables& T, double E, const double* x) {
-  if (P == BREM) return f_brem_ref(T, E, kMe, x[0], x[1], x[2], x[3]);
-  if (P == MUONBREM) return f_brem_ref(T, E, kMmu, x[0], x[1], x[2], x[3]);
-  if (P == PAIRPROD) return f_pairprod_ref(T, E, x[0], x[1], x[2], x[3]);
-  if (P == DARKANN) return f_dark_ann_ref(E, T.d->mV, x[0]);
+  if (P == BREM) return f_brem_ref(T.Eg_min, T.brem_a0, T.Z, E, kMe, x[0], x[1], x[2], x[3]);
+  if (P == MUONBREM) return f_brem_ref(T.Eg_min, T.brem_a0, T.Z, E, kMmu, x[0], x[1], x[2], x[3]);
+  if (P == PAIRPROD) return f_pairprod_ref(T.brem_a0, T.Z, E, x[0], x[1], x[2], x[3]);
+  if (P == DARKANN) return f_dark_ann_ref(E, T.mV, x[0]);
   return integrand_p<P>(T, E, x);
 }
 
@@ -293,8 +293,7 @@ __device__ void draw_loop(const DevTables& T, const DrawLaunch& io, uint64_t see
   int g0 = lane - gl;
   const PetiteGridDesc& gd = T.d->grid[p];
   const int32_t ninc[4] = {gd.ninc[0], gd.ninc[1], gd.ninc[2], gd.ninc[3]};
-  const uint32_t max_trials = (uint32_t)(T.d->max_trials < (int64_t)0x7FFFFFF0 ? (T.d->max_trials > 0 ? T.d->max_trials : 1)
-                                                                               : (int64_t)0x7FFFFFF0);
+  const uint32_t max_trials = T.max_trials;
   // Requests per queue access: a quarter of a wave's share, so that the waves
   // end together, from one per group up to 64.  With 64 whatever the count, a
   // launch of 64 requests at 64 lanes each ran them one after another in its
@@ -329,7 +328,7 @@ __device__ void draw_loop(const DevTables& T, const DrawLaunch& io, uint64_t see
           sid = io.req_sid ? io.req_sid[ridx] : io.sid_src[src];
           const int ie = lu_key(T, p, E);
           base = T.f32 + gd.node_off + (int64_t)ie * gd.stride;
-          mf = T.maxf[p * T.maxE + ie] * T.d->maxF_fudge;
+          mf = T.maxf[p * T.maxE + ie] * T.maxF_fudge;
           // a draw that cannot accept ends after its first round, as the
           // reference's loop would after max_trials candidates
           j = draw_possible<p>(T) ? 0u : max_trials;
@@ -494,8 +493,7 @@ __global__ __launch_bounds__(256) void k_draw_long(DevTables T, DrawLaunch io, u
   const int64_t windows = (n + 63) / 64;
   const PetiteGridDesc& gd = T.d->grid[P];
   const int32_t ninc[4] = {gd.ninc[0], gd.ninc[1], gd.ninc[2], gd.ninc[3]};
-  const uint32_t max_trials = (uint32_t)(T.d->max_trials < (int64_t)0x7FFFFFF0 ? (T.d->max_trials > 0 ? T.d->max_trials : 1)
-                                                                               : (int64_t)0x7FFFFFF0);
+  const uint32_t max_trials = T.max_trials;
   int64_t w0 = wave % windows;
   int pick = (int)(wave / windows);
   for (int64_t empty = 0; empty < windows;) {
@@ -546,8 +544,7 @@ __global__ __launch_bounds__(256) void k_draw_long_finish(DevTables T, DrawLaunc
     const LongDraw R = io.longs[q];
     const PetiteGridDesc& gd = T.d->grid[P];
     const int32_t ninc[4] = {gd.ninc[0], gd.ninc[1], gd.ninc[2], gd.ninc[3]};
-    const uint32_t max_trials = (uint32_t)(T.d->max_trials < (int64_t)0x7FFFFFF0
-                                               ? (T.d->max_trials > 0 ? T.d->max_trials : 1) : (int64_t)0x7FFFFFF0);
+    const uint32_t max_trials = T.max_trials;
     n_draw = 1;
     if (R.win < max_trials) {
       double x[4] = {0.0, 0.0, 0.0, 0.0};
@@ -592,8 +589,7 @@ __device__ void draw_block_one(const DevTables& T, const DrawLaunch& io, uint64_
   __shared__ uint32_t s_win;
   const PetiteGridDesc& gd = T.d->grid[p];
   const int32_t ninc[4] = {gd.ninc[0], gd.ninc[1], gd.ninc[2], gd.ninc[3]};
-  const uint32_t max_trials = (uint32_t)(T.d->max_trials < (int64_t)0x7FFFFFF0 ? (T.d->max_trials > 0 ? T.d->max_trials : 1)
-                                                                               : (int64_t)0x7FFFFFF0);
+  const uint32_t max_trials = T.max_trials;
   const int64_t ridx = (int64_t)p * io.req_cap + r;
   const int32_t src = io.req_slot[ridx];
   const int64_t oidx = io.explicit_out ? (int64_t)src : ridx;
@@ -601,7 +597,7 @@ __device__ void draw_block_one(const DevTables& T, const DrawLaunch& io, uint64_
   const uint64_t sid = io.req_sid ? io.req_sid[ridx] : io.sid_src[src];
   const int ie = lu_key(T, p, E);
   const float* base = T.f32 + gd.node_off + (int64_t)ie * gd.stride;
-  const double mf = T.maxf[p * T.maxE + ie] * T.d->maxF_fudge;
+  const double mf = T.maxf[p * T.maxE + ie] * T.maxF_fudge;
   for (uint32_t j = draw_possible<p>(T) ? 0u : max_trials; j < max_trials; j += blockDim.x) {
     if (threadIdx.x == 0) s_win = 0xFFFFFFFFu;
     __syncthreads();
@@ -864,11 +860,11 @@ __global__ void k_init_primaries(DevStore S, const PetitePrimary* prim, int64_t 
 
 __device__ inline double min_calc(const DevTables& T, int pid) {
   switch (pid) {
-    case 11: return T.d->min_calc[0];
-    case -11: return T.d->min_calc[1];
-    case 22: return T.d->min_calc[2];
-    case 13: return T.d->min_calc[3];
-    case -13: return T.d->min_calc[4];
+    case 11: return T.min_calc[0];
+    case -11: return T.min_calc[1];
+    case 22: return T.min_calc[2];
+    case 13: return T.min_calc[3];
+    case -13: return T.min_calc[4];
     default: return 0.0;
   }
 }
@@ -971,8 +967,8 @@ struct LdsSigma {
     }
   }
   // One channel's header in registers, and its value when the table has a node
-  // index: nsigma's arithmetic without branches, so that the lookups of a sum
-  // and the work beside them overlap.  (A lane whose E lies outside the table,
+  // index: nsigma's arithmetic without branches and with the reads apart from
+  // their use, so that the lookups of a sum and the work beside them overlap.  (A lane whose E lies outside the table,
   // or whose channel is empty, reads records inside the tables and gets 0.)
   struct Channel {
     float log2E0, per;
@@ -992,13 +988,20 @@ struct LdsSigma {
     c.hi = p == 0xFu ? 0.0 : h[3];
     return c;
   }
-  __device__ inline double indexed(const Channel& c, double E, float l2) const {
+  // The two records around E's node, read ahead of their use.
+  struct Pair {
+    double xa, ya, sa, xb, yb, sb;
+  };
+  __device__ inline Pair fetch(const Channel& c, float l2) const {
     int j = (int)((l2 - c.log2E0) * c.per + 0.5f);
     j = min(max(j, 0), c.nm1);
     const double* r = base + c.rec + 4 * j;
-    const double va = r[3] * (E - r[0]) + r[2];
-    const double vb = r[7] * (E - r[4]) + r[6];
-    const double v = E >= r[4] ? vb : va;
+    return Pair{r[0], r[2], r[3], r[4], r[6], r[7]};
+  }
+  __device__ inline double value(const Channel& c, const Pair& r, double E) const {
+    const double va = r.sa * (E - r.xa) + r.ya;
+    const double vb = r.sb * (E - r.xb) + r.yb;
+    const double v = E >= r.xb ? vb : va;
     return (E >= c.lo) & (E <= c.hi) ? v : 0.0;
   }
   // The same sums for a lane's charged species from its channel word (see
@@ -1027,10 +1030,10 @@ __device__ inline void mcs_rotate(const DevTables& T, float& nx, float& ny, floa
   // quantity (a float64 division per factor costs several times as much)
   const float beta = fp * __builtin_amdgcn_rcpf((float)E);
   const float pMeV = (float)(m_lep * 1.0e3) * fp * __builtin_amdgcn_rcpf((float)m_part);
-  const float t = (float)(T.d->rho * (dz * (1.0 / kCmToM)));
+  const float t = (float)(T.rho * (dz * (1.0 / kCmToM)));
   const float th0 = lynch_dahl_theta0(T.mcs_cA, T.mcs_cB, T.mcs_cC, t, pMeV, beta);
   const float r = sqrtf(-2.0f * logf(u01f(w_r)));
-  const float theta = ((w_a & 1u) ? r : -r) * th0 * (float)T.d->rescale_MCS;
+  const float theta = ((w_a & 1u) ? r : -r) * th0 * (float)T.rescale_MCS;
   float sth, cth;
   sincosf(theta, &sth, &cth);
   const float ua = u01f(w_a);
@@ -1059,7 +1062,7 @@ __device__ inline void charged_advance(const DevTables& T, double dist, double m
                                        uint32_t w_a, double& E, float& nx, float& ny, float& nz, float& rx,
                                        float& ry, float& rz, double& dep) {
   const double Eb = E;
-  E = __fma_rn(-T.d->dEdx, dist, E);
+  E = __fma_rn(-T.dEdx, dist, E);
   if (E <= m) E = m;
   const double q = momentum2(E, m);
   dep += Eb - E;
@@ -1067,7 +1070,7 @@ __device__ inline void charged_advance(const DevTables& T, double dist, double m
     rx += (float)(nx * dist);
     ry += (float)(ny * dist);
     rz += (float)(nz * dist);
-    if (T.d->MS) mcs_rotate(T, nx, ny, nz, E, sqrtf((float)q), m, m_lep, dist, w_r, w_a);
+    if (T.MS) mcs_rotate(T, nx, ny, nz, E, sqrtf((float)q), m, m_lep, dist, w_r, w_a);
   } else {
     nx = ny = nz = 0.0f;
   }
@@ -1159,7 +1162,7 @@ __global__ __launch_bounds__(256) void k_transport(DevTables T, DevStore S, int6
           wgt = S.r0[slot].w;
           ch = sum_channels(pid);
           m = pid_mass(pid);
-          pme = fmax(fmax(min_calc(T, pid), T.d->min_energy), m);
+          pme = fmax(fmax(min_calc(T, pid), T.min_energy), m);
           E = R0.E;
           dep = R0.dep;
           dz = R0.dz;
@@ -1185,7 +1188,7 @@ __global__ __launch_bounds__(256) void k_transport(DevTables T, DevStore S, int6
           wgt = r0.w;
           ch = sum_channels(pid);
           m = pid_mass(pid);
-          pme = fmax(fmax(min_calc(T, pid), T.d->min_energy), m);
+          pme = fmax(fmax(min_calc(T, pid), T.min_energy), m);
           E = (double)p0.x;
           nx = p0.y;
           ny = p0.z;
@@ -1514,7 +1517,7 @@ __global__ __launch_bounds__(64 * kEmitWaves) void k_emit(DevTables T, DevStore 
       const double x0 = accepted_x1(T, p, E, seed, sid, tr, xs[0]);
       vertex_children(p, pid, E, xs, x0, az, pf.y, pf.z, pf.w, lab, cpid);
       for (int k = 0; k < 2; ++k) {
-        keep[k] = lab[k].e > T.d->min_energy;
+        keep[k] = lab[k].e > T.min_energy;
         if (!keep[k] && shower_energy) unsafeAtomicAdd(shower_energy + 4 * shower + 2, lab[k].e);
       }
       if (shower_energy && (p == COMP || p == ANN || p == MOLLER || p == BHABHA || p == MUONE))
@@ -2155,6 +2158,21 @@ int petite_ctx_create(const PetiteTableDesc* desc, const double* blob64, int64_t
   T.maxf = c->dmaxf;
   T.maxE = maxE;
   T.d = c->ddesc;
+  T.dEdx = desc->dEdx;
+  T.rho = desc->rho;
+  T.min_energy = desc->min_energy;
+  T.Eg_min = desc->Eg_min;
+  T.Ee_min = desc->Ee_min;
+  T.mV = desc->mV;
+  T.mT = desc->mT;
+  T.Z = desc->Z;
+  T.A = desc->A;
+  T.Zeff = desc->Zeff;
+  T.maxF_fudge = desc->maxF_fudge;
+  for (int i = 0; i < 5; ++i) T.min_calc[i] = desc->min_calc[i];
+  T.rescale_MCS = desc->rescale_MCS;
+  T.MS = desc->MS;
+  T.max_trials = (uint32_t)std::min<int64_t>(std::max<int64_t>(desc->max_trials, 1), 0x7FFFFFF0);
   const double Z = desc->Z;
   const double a0 = 184.15 * pow(2.718, -0.5) * pow(Z, -1.0 / 3.0) / kMe;
   const double a04 = a0 * a0 * a0 * a0;

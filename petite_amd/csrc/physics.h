@@ -42,7 +42,15 @@ struct DevTables {
   float mcs_cC;        //   3.34 (Z alpha)^2  (moliere.py:196-219)
   int32_t lds_doubles; // size of the n*sigma tables staged in LDS by the transport kernel
   int32_t sig_indexed; // every SM n*sigma table is empty or has a node index (LdsSigma::indexed)
-  const PetiteTableDesc* d;  // device copy of the descriptor (read through the scalar cache)
+  // The descriptor's scalars, in the kernel arguments: read through `d` in a
+  // kernel that also writes memory, each use is a vector load and a wait (three
+  // of them held a third of a substep's latency in the walk).
+  double dEdx, rho, min_energy, Eg_min, Ee_min, mV, mT, Z, A, Zeff, maxF_fudge;
+  double min_calc[5];
+  double rescale_MCS;
+  int32_t MS;
+  uint32_t max_trials; // 1 .. 0x7FFFFFF0
+  const PetiteTableDesc* d;  // device copy of the descriptor: its grids and tables
 };
 
 // ---------------------------------------------------------------- tables ---
@@ -191,7 +199,7 @@ __device__ inline float rcp_f(float x) { return __builtin_amdgcn_rcpf(x); }
 
 // Brem / MuonBrem, all_processes.py:139-206.  PF*FF = C epp d dp /(w ep (1+a0^2 q^2)^2).
 __device__ inline float f_brem(const DevTables& T, double ep, double m, float C, const double* x) {
-  const double egmin = T.d->Eg_min;
+  const double egmin = T.Eg_min;
   const double range = ep - m - egmin;
   const double w = egmin + x[0] * range;
   const double epp = ep - w;
@@ -256,13 +264,12 @@ __device__ inline float f_pairprod(const DevTables& T, double w, const double* x
 // the form factor g2_elastic (99-103) applied as a separate factor.  The
 // draws take these only for a candidate whose float32 J*f lies within a
 // small band of the accept threshold, so the accept decision is the one a
-// float64 evaluation of the reference formula makes.  Not inlined (and the
-// point passed by value): the rare call keeps the draw loop's registers at
+// float64 evaluation of the reference formula makes.  Not inlined (and
+// everything passed by value): the rare call keeps the draw loop's registers at
 // the float32 body's count.
-__device__ __noinline__ double f_brem_ref(const DevTables& T, double ep, double m, double x0, double x1, double x2,
-                                          double x3) {
+__device__ __noinline__ double f_brem_ref(double egmin, double a0, double Z, double ep, double m, double x0, double x1,
+                                          double x2, double x3) {
   const double x[4] = {x0, x1, x2, x3};
-  const double egmin = T.d->Eg_min;
   const double w = egmin + x[0] * (ep - m - egmin);
   const double d = ep / (2.0 * m) * (x[1] + x[2]);
   const double dp = ep / (2.0 * m) * (x[1] - x[2]);
@@ -275,8 +282,6 @@ __device__ __noinline__ double f_brem_ref(const DevTables& T, double ep, double 
   const double a = kAlpha / m;
   const double PF = 8.0 / kPi * kAlpha * (a * a) * (epp * (m * m * m * m)) / (w * ep * (qsq * qsq)) * d * dp;
   const double jac = kPi * ep * ep * (ep - m - egmin) / (m * m);
-  const double a0 = T.brem_a0;
-  const double Z = T.d->Z;
   const double a0t = 1.0 + a0 * a0 * qsq;
   const double FF = Z * Z * (a0 * a0 * a0 * a0) * (qsq * qsq) / (a0t * a0t);
   const double A = 1.0 + d * d, B = 1.0 + dp * dp;
@@ -287,7 +292,7 @@ __device__ __noinline__ double f_brem_ref(const DevTables& T, double ep, double 
   return PF * (T1 + T2 + T3 + T4) * jac * FF;
 }
 
-__device__ __noinline__ double f_pairprod_ref(const DevTables& T, double w, double x0, double x1, double x2,
+__device__ __noinline__ double f_pairprod_ref(double a0, double Z, double w, double x0, double x1, double x2,
                                               double x3) {
   const double x[4] = {x0, x1, x2, x3};
   const double m = kMe;
@@ -303,8 +308,6 @@ __device__ __noinline__ double f_pairprod_ref(const DevTables& T, double w, doub
   const double a = kAlpha / m;
   const double PF = 8.0 / kPi * kAlpha * (a * a) * epp * epm / (w * w * w * (qq * qq)) * dp * dm;
   const double jac = kPi * w * w * (w - 2.0 * m) / (m * m);
-  const double a0 = T.brem_a0;
-  const double Z = T.d->Z;
   const double t = m * m * qq;
   const double a0t = 1.0 + a0 * a0 * t;
   const double FF = Z * Z * (a0 * a0 * a0 * a0) * (t * t) / (a0t * a0t);
@@ -538,14 +541,14 @@ __device__ inline double integrand(const DevTables& T, int proc, double E, const
     case MUONBREM: return (double)f_brem(T, E, kMmu, T.brem_C_mu, x);
     case PAIRPROD: return (double)f_pairprod(T, E, x);
     case COMP: return f_compton(E, 0.0, x[0]);
-    case ANN: return f_annihilation(E, 0.0, T.d->Eg_min, x[0]);
-    case MOLLER: return f_moller(E, T.d->Ee_min, x[0]);
-    case BHABHA: return f_bhabha(E, T.d->Ee_min, x[0]);
-    case MUONE: return f_muone(E, T.d->Ee_min, x[0]);
-    case DARKBREM: return f_dark_brem(E, kMe, T.d->mV, T.d->mT, T.d->Z, T.d->A, x);
-    case DARKMUONBREM: return f_dark_brem(E, kMmu, T.d->mV, T.d->mT, T.d->Z, T.d->A, x);
-    case DARKANN: return f_dark_ann(E, T.d->mV, x[0]);
-    case DARKCOMP: return f_compton(E, T.d->mV, x[0]);
+    case ANN: return f_annihilation(E, 0.0, T.Eg_min, x[0]);
+    case MOLLER: return f_moller(E, T.Ee_min, x[0]);
+    case BHABHA: return f_bhabha(E, T.Ee_min, x[0]);
+    case MUONE: return f_muone(E, T.Ee_min, x[0]);
+    case DARKBREM: return f_dark_brem(E, kMe, T.mV, T.mT, T.Z, T.A, x);
+    case DARKMUONBREM: return f_dark_brem(E, kMmu, T.mV, T.mT, T.Z, T.A, x);
+    case DARKANN: return f_dark_ann(E, T.mV, x[0]);
+    case DARKCOMP: return f_compton(E, T.mV, x[0]);
     default: return 0.0;
   }
 }

@@ -66,8 +66,7 @@ __device__ inline void walk_draws(const DevTables& T, uint64_t seed, bool mine, 
   const int lane = threadIdx.x & 63;
   const PetiteGridDesc& gd = T.d->grid[P];
   const int32_t ninc[4] = {gd.ninc[0], gd.ninc[1], gd.ninc[2], gd.ninc[3]};
-  const uint32_t max_trials = (uint32_t)(T.d->max_trials < (int64_t)0x7FFFFFF0 ? (T.d->max_trials > 0 ? T.d->max_trials : 1)
-                                                                               : (int64_t)0x7FFFFFF0);
+  const uint32_t max_trials = T.max_trials;
   unsigned long long om = __ballot(mine);
   int lg = 0, n_open = __popcll(om);
   while ((n_open << (lg + 1)) <= 64) ++lg;
@@ -229,7 +228,7 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
     if (mode == GIVEN) {
       ch = sum_channels(pid);
       m = pid_mass(pid);
-      pme = fmax(fmax(min_calc(T, pid), T.d->min_energy), m);
+      pme = fmax(fmax(min_calc(T, pid), T.min_energy), m);
       const float pn2 = norm2(nx, ny, nz);
       if (pn2 > 0.0f) {
         const float inv = rsqrtf(pn2);
@@ -284,12 +283,20 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
         ++iters;
         if (mode == STEP) {
           const bool in_close = closing;
+          // the channels' records are on their way while the Philox block is formed
+          LdsSigma::Pair r0{}, r1{}, r2{};
+          if (T.sig_indexed) {
+            const float l2 = __log2f((float)E);
+            r0 = L.fetch(c0, l2);
+            r1 = L.fetch(c1, l2);
+            r2 = L.fetch(c2, l2);
+            __builtin_amdgcn_sched_barrier(0);
+          }
           const U4 u = draw_block(seed, sid, in_close ? 0u : k, in_close ? PURPOSE_CLOSE : PURPOSE_STEP);
           double Ssum;
           if (T.sig_indexed) {
-            const float l2 = __log2f((float)E);
-            const double s01 = L.indexed(c0, E, l2) + L.indexed(c1, E, l2);
-            const double s2 = L.indexed(c2, E, l2);
+            const double s01 = L.value(c0, r0, E) + L.value(c1, r1, E);
+            const double s2 = L.value(c2, r2, E);
             Ssum = (ch >> 8) == 0xFu ? s01 : s01 + s2;
           } else {
             Ssum = L.nsigma_sum_ch(ch, E);
@@ -379,7 +386,7 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
     double mf = 0.0;
     if (want >= 0) {
       ie = lu_key(T, want, E);
-      mf = T.maxf[want * T.maxE + ie] * T.d->maxF_fudge;
+      mf = T.maxf[want * T.maxE + ie] * T.maxF_fudge;
     }
     for (unsigned long long todo = __ballot(want >= 0); todo;) {
       const int q = __shfl(want, __ffsll((long long)todo) - 1);
@@ -413,7 +420,7 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
         const float xs[4] = {xv.x, xv.y, xv.z, xv.w};
         vertex_children(want, pid, E, xs, W.x0[lane], az, pf.y, pf.z, pf.w, lab, cpid);
         for (int c = 0; c < 2; ++c) {
-          keep[c] = lab[c].e > T.d->min_energy;
+          keep[c] = lab[c].e > T.min_energy;
           if (!keep[c]) {
             ++n_drop;
             if (shower_energy) unsafeAtomicAdd(shower_energy + 4 * shower + 2, lab[c].e);
