@@ -1834,7 +1834,8 @@ struct PetiteCtx {
   int64_t* drange = nullptr;
   ResumeRec* dresume = nullptr;  // [2][resume_cap]
   int64_t resume_cap = 0;
-  int32_t* tail_spill = nullptr;  // [2][kTailSpill]: depth-first walk spill lists
+  int32_t* tail_spill = nullptr;  // [2][tail_spill_cap]: depth-first walk spill lists
+  int64_t tail_spill_cap = 0;
   LongDraw* longs = nullptr;      // [kLongCap], contexts with a DarkAnn map
   std::vector<hipEvent_t> tev;
   int n_cu = 256;
@@ -2644,7 +2645,14 @@ int petite_run_showers(PetiteCtx* c, const PetitePrimary* prim, int64_t n, uint6
   }
   while (true) {
     if (tail) {
-      if (!c->tail_spill) HIP_TRY(hipMalloc(&c->tail_spill, 2 * kTailSpill * sizeof(int32_t)));
+      if (c->tail_spill_cap < store->capacity) {
+        if (c->tail_spill) HIP_TRY(hipFree(c->tail_spill));
+        c->tail_spill = nullptr;
+        c->tail_spill_cap = 0;
+        HIP_TRY(hipMalloc(&c->tail_spill, 2 * store->capacity * sizeof(int32_t)));
+        c->tail_spill_cap = store->capacity;
+      }
+      const int64_t scap = c->tail_spill_cap;
       // the first walk alone (it often leaves no spill), then kTailGroup per
       // host check: a launch whose inputs are empty ends at once
       const int ng = tail_launches == 0 ? 1 : kTailGroup;
@@ -2652,8 +2660,8 @@ int petite_run_showers(PetiteCtx* c, const PetitePrimary* prim, int64_t n, uint6
         hipLaunchKernelGGL(k_tail_setup, dim3(1), dim3(64), 0, s, ctr, c->drange, store->capacity, rcap, tpar);
         HIP_TRY(hipGetLastError());
         if (c->timing) HIP_TRY(hipEventRecord(c->tev[4 * group + 2 * g], s));
-        const TailParams tp{c->tail_spill + (int64_t)tpar * kTailSpill, ctr + C_SPILL + tpar,
-                            c->tail_spill + (int64_t)(tpar ^ 1) * kTailSpill, ctr + C_SPILL + (tpar ^ 1), kTailSpill,
+        const TailParams tp{c->tail_spill + (int64_t)tpar * scap, ctr + C_SPILL + tpar,
+                            c->tail_spill + (int64_t)(tpar ^ 1) * scap, ctr + C_SPILL + (tpar ^ 1), scap,
                             tn.tail_depth, tail_limit(tn.tail_budget, tail_launches)};
         hipLaunchKernelGGL(k_tail, dim3(tail_blocks), dim3(256), lds, s, c->dev, S, seed, shower_energy, ctr,
                            c->dsig_lds, (const int64_t*)c->drange, ResumeBuf{c->dresume, rcap}, tp);

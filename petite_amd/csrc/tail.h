@@ -30,7 +30,6 @@
 
 constexpr int kTailMaxDepth = 128;  // stack entries per wave
 constexpr int kTailGroup = 4;       // walk launches queued per host check after the first
-constexpr int64_t kTailSpill = 1 << 22;  // entries per spill list
 constexpr int kTailStepsPerParticle = 8;  // iterations of a wave per particle of its lanes' budget
 constexpr int kTailPhaseSteps = 4;        // iterations a draw phase counts for
 
@@ -39,7 +38,7 @@ struct TailParams {
   const unsigned long long* n_spill_in;
   int32_t* spill_out;                 // slots past a full stack or the launch's share
   unsigned long long* n_spill_out;
-  int64_t spill_cap;
+  int64_t spill_cap;  // the store's capacity: a list holds every particle there is room for
   int32_t depth;   // stack entries per wave (1..kTailMaxDepth)
   int64_t limit;   // iterations after which a wave starts no more particles
 };
@@ -157,8 +156,6 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
   const unsigned long long below = (1ull << lane) - 1ull;
   WalkLds& W = s_walk[threadIdx.x >> 6];
   const int depth = TPm.depth < 1 ? 1 : (TPm.depth > kTailMaxDepth ? kTailMaxDepth : TPm.depth);
-  // more items than half a spill list holds are all walked in this launch
-  const int64_t limit = total > TPm.spill_cap / 2 ? (int64_t)1 << 62 : TPm.limit;
   // lane states: empty, stepping, at its end (parked), given a particle that
   // has not started
   enum { EMPTY = 0, STEP = 1, PARKED = 2, GIVEN = 3 };
@@ -180,7 +177,7 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
     // leaves.  A wave whose particles all have lanes and include a muon goes on:
     // a muon's chain of thousands of vertices sets the run's length, and
     // would go slower among a spread's other particles
-    const bool stop = iters >= limit && (sp > 0 || __ballot(mode != EMPTY && (pid == 13 || pid == -13)) == 0ull);
+    const bool stop = iters >= TPm.limit && (sp > 0 || __ballot(mode != EMPTY && (pid == 13 || pid == -13)) == 0ull);
     // ---- free lanes take from the stack, then claim items (after a draw
     // phase, or when no lane is stepping)
     const unsigned long long im = __ballot(mode == EMPTY);
