@@ -575,341 +575,393 @@ __global__ __launch_bounds__(kMesonBlock) void k_meson_decay(DevTables T, Petite
 }
 
 // ------------------------------------------------------ m_V-continuous yield --
-constexpr int kYieldBatch = 16;
-constexpr int kYieldWindow = 8;  // trained masses a pass may use (consecutive)
+// Each mass point's sum over the record is a table lookup and (but for
+// DarkAnn) an exponential per particle, in float64.  The record's energies and
+// weights go to a list per species once, so that a wave works on one process;
+// a block holds several points' sums in registers, and the grid's y dimension
+// covers the rest, so that a particle's logarithms serve kYieldGroup points
+// and a short record still fills the chip.  The blocks' sums go to rows of
+// their own and one kernel adds those (atomics of every wave on the points'
+// sums, all in four cache lines, were served one after another).  19e6 records
+// x 32 points with gradients: 3.4 ms (interpolation 2.3, bound 0.74, lists
+// 0.32); two scans of mixed species with unpacked tables took 10.6 ms.
+constexpr int kYieldBatch = 32;   // points of a pass
+constexpr int kYieldGroup = 8;     // points of a block of k_dark_yield
+constexpr int kBoundGroup = 4;    // points of a block of k_bound_yield
+constexpr int kYieldComp = 4;     // table of DarkComp beside the four weight families
+constexpr int kYieldSpecies = 4;  // e-, e+, photons, mu-+
 constexpr double kLn10 = 2.302585092994045684;
 
-struct YieldTables {
-  PetiteDarkDesc d[PETITE_MAX_MASSES];
-  int32_t n_mass;
-  const double* b;
+// One grid interval: x .. xn, the value at x and the slope.  The last node has
+// xn = inf and slope 0.
+struct alignas(32) YieldRow {
+  double x, xn, y, slope;
 };
 
-// Mass points of one pass (ascending m_V): segment j0 + j[k] (trained masses
-// j0 + j[k] and the next), t and dt/dm_V; `need` marks which of the window's
-// trained masses j0 .. j0 + kYieldWindow - 1 the segments use.
+// One process' table at one trained mass: a weight in E (the linear families)
+// or log10 n sigma in log10 E (DarkComp).
+struct YieldTable {
+  double thr;       // lowest energy with a weight
+  double x0, x1;    // grid ends
+  double g0, inv;   // guess of the interval from ln E (log10 E for DarkComp); inv = 0: bisection
+  double eps2, ln_eps2;
+  int32_t n, off;   // rows
+};
+
+struct YieldTables {
+  YieldTable t[PETITE_MAX_MASSES][kYieldComp + 1];
+  const YieldRow* rows;
+  int32_t n_mass;
+};
+
+// Mass points of one pass (ascending m_V): segment j[k] (trained masses j[k]
+// and the next), t and dt/dm_V, and eps^2 for the bound-electron tables.
 struct YieldPoints {
   int32_t n;
-  int32_t j0;
-  uint32_t need;
   int32_t j[kYieldBatch];
   double t[kYieldBatch];
   double dtdm[kYieldBatch];
-  double ln_eps2[kYieldWindow];
+  double eps2[kYieldBatch];
 };
 
-// interpolate1d in log10-log10 (dark_shower.py:31-46), returning the log10 of
-// the value: -20 outside the table (the fill 1e-20); l = log10(E).
-__device__ inline double loglog10(const double* lx, const double* ly, int n, double l, double l0, double inv_dl) {
-  if (n <= 0 || l < lx[0] || l > lx[n - 1]) return -20.0;
-  if (l == lx[n - 1]) return ly[n - 1];
-  const int lo = find_interval(lx, n, l, (float)l, l0, inv_dl);
-  const double slope = (ly[lo + 1] - ly[lo]) / (lx[lo + 1] - lx[lo]);
-  return slope * (l - lx[lo]) + ly[lo];
-}
-
-// Weight of one trained mass for the yield, as (w, ln w): GetBSMWeights with
-// that mass's tables (dark_shower.py:595-647).  DarkComp's log-log table gives
-// ln w = ln eps^2 - ln(n sigma_PP + n sigma_Comp) + ln 10 * L directly (w
-// itself, eps^2 10^L / den, is formed only where the linear branch needs it;
-// here w = 1 marks it positive); the other families take the log of the
-// interpolated weight.
-__device__ inline void yield_weight(const DevTables& T, const PetiteDarkDesc& D, const double* b, int pid, int code,
-                                    const WeightArgs& a, double ln_eps2, double ln_den, double& wv, double& lam) {
-  if (code == DARKCOMP) {
-    if (pid != 22 || a.E0 < D.min_comp || a.E0 < T.min_calc[2]) {
-      wv = 0.0;
-      lam = 0.0;
-      return;
-    }
-    const double* lx = b + D.comp_off;
-    lam = ln_eps2 - ln_den + kLn10 * loglog10(lx, lx + D.comp_n, D.comp_n, a.l10, D.comp_l0, D.comp_inv_dl);
-    wv = 1.0;
-    return;
-  }
-  wv = bsm_weight(T, D, b, pid, code, a);
-  lam = wv > 0.0 ? log(wv) : 0.0;
-}
-
-// Bound-electron tables at the pass's masses (quad.h): slot k * nv + v holds
-// m_k (v = 0), m_k (1 + h) (v = 1) and m_k (1 - h) (v = 2, with the
-// derivative).  slot == nullptr: DarkAnn and DarkComp interpolate between the
-// trained masses like the other processes.
-struct BoundView {
-  const quad::BoundSlot* slot;
-  const double* tab;
-  int32_t stride;  // doubles per slot
-  int32_t nv;  // slots per point: 3 with the derivative (m_k, and its node derivatives after k_bound_deriv), else 1
-};
-
-// W and dW/dm_V of DarkAnn / DarkComp at point k: the interpolant of slot
-// k * nv at E0, and (GRAD) its derivative from the node derivatives in slot
-// k * nv + 1 (k_bound_deriv).  With s the interval weight,
-//   d/dm [y_lo + s (y_hi - y_lo)] = y'_lo + s (y'_hi - y'_lo) + (y_hi - y_lo) s',
-//   s' = -[x'_lo (1 - s) + x'_hi s] / (x_hi - x_lo);
-// DarkComp in log10 space: W = eps^2 10^L / den, dW = W ln 10 dL.  Below the
-// thresholds or outside the grid W = dW = 0.
-template <bool GRAD>
-__device__ inline void bound_wd(const DevTables& T, const BoundView& B, int k, int code, const WeightArgs& a,
-                                double ln_den, double ln_eps2, double& W, double& dW) {
-  const int s0 = k * B.nv;
-  const quad::BoundSlot& S = B.slot[s0];
-  const double* t = B.tab + (int64_t)s0 * B.stride;
-  const double* d = t + B.stride;
-  constexpr int n = quad::kBoundGrid;
-  W = dW = 0.0;
-  if (code == DARKANN) {
-    const double E0 = a.E0;
-    if (E0 < S.min_ann || !(E0 >= t[0]) || E0 > t[n - 1]) return;
-    const double* y = t + 3 * n;
-    const double e2 = exp(ln_eps2);
-    if (E0 == t[n - 1]) {
-      W = e2 * y[n - 1];
-      if (GRAD) dW = e2 * d[3 * n + n - 1];
-      return;
-    }
-    const int lo = find_interval(t, n, E0, a.lf, S.lnEa0, S.inv_dln_a);
-    const double xl = t[lo], xh = t[lo + 1], yl = y[lo], yh = y[lo + 1];
-    const double slope = (yh - yl) / (xh - xl);
-    W = e2 * (slope * (E0 - xl) + yl);
-    if (GRAD) {
-      const double sw = (E0 - xl) / (xh - xl);
-      const double sd = -(d[lo] * (1.0 - sw) + d[lo + 1] * sw) / (xh - xl);
-      const double dyl = d[3 * n + lo], dyh = d[3 * n + lo + 1];
-      dW = e2 * (dyl + sw * (dyh - dyl) + (yh - yl) * sd);
-    }
-    return;
-  }
-  if (a.E0 < S.min_comp || a.E0 < T.min_calc[2]) return;
-  const double* lx = t + 4 * n;
-  const double* ly = t + 5 * n;
-  const double l = a.l10;
-  if (l < lx[0] || l > lx[n - 1]) {
-    W = exp(ln_eps2 - ln_den - 20.0 * kLn10);  // the fill 1e-20
-    return;
-  }
-  double L, dL = 0.0;
-  if (l == lx[n - 1]) {
-    L = ly[n - 1];
-    if (GRAD) dL = d[5 * n + n - 1];
-  } else {
-    const int lo = find_interval(lx, n, l, (float)l, S.l0c, S.inv_dlc);
-    const double xl = lx[lo], xh = lx[lo + 1], yl = ly[lo], yh = ly[lo + 1];
-    L = (yh - yl) / (xh - xl) * (l - xl) + yl;
-    if (GRAD) {
-      const double sw = (l - xl) / (xh - xl);
-      const double sd = -(d[4 * n + lo] * (1.0 - sw) + d[4 * n + lo + 1] * sw) / (xh - xl);
-      const double dyl = d[5 * n + lo], dyh = d[5 * n + lo + 1];
-      dL = dyl + sw * (dyh - dyl) + (yh - yl) * sd;
-    }
-  }
-  W = exp(ln_eps2 - ln_den + kLn10 * L);
-  if (GRAD) dW = W * kLn10 * dL;
-}
-
-// Record indices one yield kernel visits (the rest contribute nothing to it).
-struct RecordList {
-  const int32_t* idx;
+// The particles of one species: entry i at Ew[i] or, for the list that fills
+// its array from the end, Ew[-i]; photons with log10 E and ln(n sigma_PP +
+// n sigma_Comp) beside.
+struct YieldList {
+  const float2* Ew;
+  const double2* ph;
+  int32_t dir;
   const unsigned long long* count;  // on the device
 };
 
-// Species bit of a record's pid (0 e-, 1 e+, 2 photon, 3 mu-, 4 mu+; 5 other).
-__device__ inline uint32_t species_bit(int pid) {
+// find_interval over rows.
+template <typename Row>
+__device__ inline int find_row(const Row* r, int n, double v, float guess_arg, double g0, double inv) {
+  int lo;
+  if (inv > 0.0) {
+    lo = (int)((guess_arg - (float)g0) * (float)inv);
+    lo = lo < 0 ? 0 : (lo > n - 1 ? n - 1 : lo);
+    while (lo > 0 && r[lo].x > v) --lo;
+    while (lo < n - 1 && r[lo].xn <= v) ++lo;
+  } else {
+    lo = 0;
+    int hi = n;
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (r[mid].x <= v) lo = mid; else hi = mid;
+    }
+  }
+  return lo;
+}
+
+struct YieldArgs {
+  double E0, l10, ln_den;  // (the last two of photons)
+  float lf;
+};
+
+// Weight of one trained mass, as (w, ln w): GetBSMWeights with that mass's
+// tables (dark_shower.py:595-647).  DarkComp's log-log table (fill -20) gives
+// ln w = ln eps^2 - ln(n sigma_PP + n sigma_Comp) + ln 10 * L directly (w
+// itself is formed only where the linear branch needs it; w = 1 marks it
+// positive); the other families take the log of the interpolated weight.
+template <bool COMP>
+__device__ inline void yield_weight(const YieldTable& t, const YieldRow* rows, const YieldArgs& a, double& wv,
+                                    double& lam) {
+  wv = lam = 0.0;
+  if (a.E0 < t.thr) return;
+  const YieldRow* r = rows + t.off;
+  if (COMP) {
+    double L = -20.0;
+    if (t.n > 0 && !(a.l10 < t.x0 || a.l10 > t.x1)) {
+      const YieldRow R = r[find_row(r, t.n, a.l10, (float)a.l10, t.g0, t.inv)];
+      L = R.slope * (a.l10 - R.x) + R.y;
+    }
+    wv = 1.0;
+    lam = t.ln_eps2 - a.ln_den + kLn10 * L;
+    return;
+  }
+  if (t.n <= 0 || !(a.E0 >= t.x0) || a.E0 > t.x1) return;
+  const YieldRow R = r[find_row(r, t.n, a.E0, a.lf, t.g0, t.inv)];
+  wv = t.eps2 * (R.slope * (a.E0 - R.x) + R.y);
+  lam = wv > 0.0 ? log(wv) : 0.0;
+}
+
+// Bound-electron tables at one point's m_V: the interval weights and, in the
+// derivative's terms, with u = x - x_lo and dots for d/dm_V of the nodes,
+//   d/dm [y_lo + u (y_hi - y_lo) / (x_hi - x_lo)] = c0 + c1 u.
+struct alignas(16) BoundRow {
+  double x, xn, y, slope, c0, c1;
+};
+
+// Species list (0 e-, 1 e+, 2 photon, 3 mu-+; -1 other) of a record's pid.
+__device__ inline int species_of(int pid) {
   switch (pid) {
-    case 11: return 1u;
-    case -11: return 2u;
-    case 22: return 4u;
-    case 13: return 8u;
-    case -13: return 16u;
-    default: return 32u;
+    case 11: return 0;
+    case -11: return 1;
+    case 22: return 2;
+    case 13:
+    case -13: return 3;
+    default: return -1;
   }
 }
 
-// The records of each yield kernel (species in mask_a / mask_b): the scans
-// then run over the records that carry weight only (in a lead shower about
-// half of them for each kernel) instead of masking the other lanes in every
-// pass.  Each wave lists a run of kListRun x 64 consecutive records in record
-// order: a first look counts its entries, one atomic per block and list
-// reserves the block's share (atomics on one address are served one after
-// another, so one per wave and 64 records cost more than the scans save), a
-// second look writes them.
+// The lists of the species in `mask`: e- from the front of Ew[0], e+ from its
+// end, photons from the front of Ew[1], muons from its end (cap entries each).
+// Each wave lists a run of kListRun x 64 consecutive records: a first look
+// counts its entries, one atomic per block and list reserves the block's
+// share, a second look writes them.
 constexpr int kListRun = 16;
-__global__ __launch_bounds__(256) void k_yield_lists(DevStore S, int64_t n, uint32_t mask_a, uint32_t mask_b,
-                                                     int32_t* list_a, int32_t* list_b, unsigned long long* counts) {
-  __shared__ unsigned long long s_cnt[2][4], s_base[2];
+__global__ __launch_bounds__(256) void k_yield_lists(DevStore S, int64_t first, int64_t n, uint32_t mask, float2* Ew,
+                                                     int64_t cap, unsigned long long* counts) {
+  __shared__ unsigned int s_cnt[kYieldSpecies][4];
+  __shared__ unsigned long long s_base[kYieldSpecies];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const unsigned long long below = (1ull << lane) - 1ull;
   constexpr int64_t kWaveRun = 64 * kListRun, kBlockRun = 4 * kWaveRun;
   for (int64_t b0 = (int64_t)blockIdx.x * kBlockRun; b0 < n; b0 += (int64_t)gridDim.x * kBlockRun) {
     const int64_t w0 = b0 + wid * kWaveRun;
-    unsigned long long ca = 0, cb = 0;
+    unsigned int c[kYieldSpecies] = {0u, 0u, 0u, 0u};
     for (int j = 0; j < kListRun; ++j) {
       const int64_t i = w0 + j * 64 + lane;
-      const uint32_t bit = i < n ? species_bit(S.pid[i]) : 0u;
-      ca += (unsigned long long)__popcll(__ballot((bit & mask_a) != 0u));
-      cb += (unsigned long long)__popcll(__ballot((bit & mask_b) != 0u));
+      const int sp = i < n ? species_of(S.pid[first + i]) : -1;
+#pragma unroll
+      for (int q = 0; q < kYieldSpecies; ++q) c[q] += (unsigned int)__popcll(__ballot(sp == q && ((mask >> q) & 1u)));
     }
-    if (lane == 0) {
-      s_cnt[0][wid] = ca;
-      s_cnt[1][wid] = cb;
+    if (lane == 0)
+      for (int q = 0; q < kYieldSpecies; ++q) s_cnt[q][wid] = c[q];
+    __syncthreads();
+    if (threadIdx.x < kYieldSpecies) {
+      const int q = threadIdx.x;
+      const unsigned int tot = s_cnt[q][0] + s_cnt[q][1] + s_cnt[q][2] + s_cnt[q][3];
+      s_base[q] = tot ? atomicAdd(counts + q, (unsigned long long)tot) : 0ull;
     }
     __syncthreads();
-    if (threadIdx.x < 2) {
-      const int l = threadIdx.x;
-      const unsigned long long tot = s_cnt[l][0] + s_cnt[l][1] + s_cnt[l][2] + s_cnt[l][3];
-      s_base[l] = tot ? atomicAdd(counts + l, tot) : 0ull;
-    }
-    __syncthreads();
-    unsigned long long oa = s_base[0], ob = s_base[1];
-    for (int w = 0; w < wid; ++w) {
-      oa += s_cnt[0][w];
-      ob += s_cnt[1][w];
+    unsigned long long o[kYieldSpecies];
+#pragma unroll
+    for (int q = 0; q < kYieldSpecies; ++q) {
+      o[q] = s_base[q];
+      for (int w = 0; w < wid; ++w) o[q] += s_cnt[q][w];
     }
     for (int j = 0; j < kListRun; ++j) {
       const int64_t i = w0 + j * 64 + lane;
-      const uint32_t bit = i < n ? species_bit(S.pid[i]) : 0u;
-      const bool in_a = (bit & mask_a) != 0u, in_b = (bit & mask_b) != 0u;
-      const unsigned long long ma = __ballot(in_a), mb = __ballot(in_b);
-      if (in_a) list_a[oa + __popcll(ma & below)] = (int32_t)i;
-      if (in_b) list_b[ob + __popcll(mb & below)] = (int32_t)i;
-      oa += (unsigned long long)__popcll(ma);
-      ob += (unsigned long long)__popcll(mb);
+      const int sp = i < n ? species_of(S.pid[first + i]) : -1;
+#pragma unroll
+      for (int q = 0; q < kYieldSpecies; ++q) {
+        const bool in = sp == q && ((mask >> q) & 1u);
+        const unsigned long long m = __ballot(in);
+        if (in) {
+          const int64_t at = (int64_t)(o[q] + __popcll(m & below));
+          float2* const A = Ew + (q >> 1) * cap;
+          A[(q & 1) ? cap - 1 - at : at] = make_float2(S.p0[first + i].x, S.r0[first + i].w);
+        }
+        o[q] += (unsigned long long)__popcll(m);
+      }
     }
     __syncthreads();  // s_cnt and s_base are read before the next run writes them
   }
 }
 
-// One float64 pass over the record: acc[2k] += w W(m_k), acc[2k+1] += w dW/dm(m_k)
-// (GRAD = false: the yield alone).  Between trained masses j and j+1 a
-// particle's weight is interpolated geometrically, W = exp(ln w_j + t ln(w_j+1 /
-// w_j)), where both are positive, linearly otherwise.
-template <bool GRAD>
-__global__ __launch_bounds__(256) void k_dark_yield(DevTables T, const YieldTables* __restrict__ Yp, DevStore S,
-                                                    RecordList L, YieldPoints P, bool bound_on, double* acc) {
-  const YieldTables& Y = *Yp;
-  double y[kYieldBatch], dy[kYieldBatch];
-#pragma unroll
-  for (int k = 0; k < kYieldBatch; ++k) y[k] = dy[k] = 0.0;
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  const PetiteDarkDesc& d0 = Y.d[0];
-  const int64_t n = (int64_t)*L.count;
-  for (int64_t ii = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; ii < n; ii += stride) {
-    const int64_t i = L.idx[ii];
-    const int pid = S.pid[i];
-    const double E0 = (double)S.p0[i].x;
-    const double w = (double)S.r0[i].w;
-    const WeightArgs wa = weight_args(T, pid, E0);
-    const double ln_den = pid == 22 ? log(wa.den) : 0.0;
-    for (int a = 0; a < d0.n_active; ++a) {
-      const int code = d0.active[a];
-      if (code == DARKCOMP ? pid != 22 : family_of(code, pid) < 0) continue;
-      if (bound_on && (code == DARKANN || code == DARKCOMP)) continue;  // k_bound_yield
-      double wv[kYieldWindow], lam[kYieldWindow];
-#pragma unroll
-      for (int q = 0; q < kYieldWindow; ++q) {
-        wv[q] = lam[q] = 0.0;
-        if (P.need & (1u << q))
-          yield_weight(T, Y.d[P.j0 + q], Y.b, pid, code, wa, P.ln_eps2[q], ln_den, wv[q], lam[q]);
-      }
-#pragma unroll
-      for (int k = 0; k < kYieldBatch; ++k) {
-        if (k >= P.n) break;
-        double lo = 0.0, hi = 0.0, llo = 0.0, lhi = 0.0;
-        // segment P.j[k] of the window (uniform over the grid); selects
-        // without indexing the register arrays
-#pragma unroll
-        for (int q = 0; q + 1 < kYieldWindow; ++q)
-          if (P.j[k] == q) {
-            lo = wv[q];
-            llo = lam[q];
-            hi = wv[q + 1];
-            lhi = lam[q + 1];
-          }
-        if (P.j[k] >= kYieldWindow - 1) {
-          lo = hi = wv[kYieldWindow - 1];
-          llo = lhi = lam[kYieldWindow - 1];
-        }
-        if (P.j0 + P.j[k] + 1 >= Y.n_mass) {
-          hi = lo;
-          lhi = llo;
-        }
-        const double t = P.t[k];
-        double W, dW;
-        if (lo > 0.0 && hi > 0.0) {
-          const double r = lhi - llo;
-          W = exp(llo + t * r);
-          dW = GRAD ? W * r * P.dtdm[k] : 0.0;
-        } else {
-          if (code == DARKCOMP) {
-            lo = lo > 0.0 ? exp(llo) : 0.0;
-            hi = hi > 0.0 ? exp(lhi) : 0.0;
-          }
-          W = lo + t * (hi - lo);
-          dW = GRAD ? (hi - lo) * P.dtdm[k] : 0.0;
-        }
-        y[k] += w * W;
-        if (GRAD) dy[k] += w * dW;
-      }
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < kYieldBatch; ++k) {
-    double a = y[k], b = dy[k];
-    for (int off = 32; off > 0; off >>= 1) {
-      a += shfl_f64(a, (threadIdx.x & 63) ^ off);
-      if (GRAD) b += shfl_f64(b, (threadIdx.x & 63) ^ off);
-    }
-    if ((threadIdx.x & 63) == 0 && k < P.n) {
-      unsafeAtomicAdd(acc + 2 * k, a);
-      if (GRAD) unsafeAtomicAdd(acc + 2 * k + 1, b);
-    }
+// log10 E and the log of the total rate of the listed photons.
+__global__ __launch_bounds__(256) void k_yield_photons(DevTables T, YieldList L, double2* out) {
+  const int64_t n = (int64_t)*L.count, stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+    const double E0 = (double)L.Ew[i].x;
+    out[i] = make_double2(log10(E0), log(nsigma(T, PAIRPROD, E0) + nsigma(T, COMP, E0)));
   }
 }
 
-// The bound-electron processes' part of the yield (DarkAnn of positrons,
-// DarkComp of photons) from the tables at the pass's masses: one float64 pass
-// over the record beside k_dark_yield, which leaves them out, into the same
-// accumulators.  A kernel of its own keeps the interpolation kernel's
-// registers (its three table lookups per mass would double them).
-template <bool GRAD>
-__global__ __launch_bounds__(256) void k_bound_yield(DevTables T, DevStore S, RecordList L, int32_t n_pts, int32_t ann,
-                                                     int32_t comp, double ln_eps2, BoundView Bv, double* acc) {
-  double y[kYieldBatch], dy[kYieldBatch];
+// The block's sums of its points k0 .. k0 + G - 1 into the block's row.
+template <bool GRAD, int G>
+__device__ inline void yield_row(const double* y, const double* dy, int k0, int n_pts, double* part) {
+  __shared__ double s_sum[4][2 * G];
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
 #pragma unroll
-  for (int k = 0; k < kYieldBatch; ++k) y[k] = dy[k] = 0.0;
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  const int64_t n = (int64_t)*L.count;
-  for (int64_t ii = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; ii < n; ii += stride) {
-    const int64_t i = L.idx[ii];
-    const int pid = S.pid[i];
-    const bool is_ann = ann && pid == -11, is_comp = comp && pid == 22;
-    if (!is_ann && !is_comp) continue;
-    const double E0 = (double)S.p0[i].x;
-    const double w = (double)S.r0[i].w;
-    const WeightArgs wa = weight_args(T, pid, E0);
-    const double ln_den = is_comp ? log(wa.den) : 0.0;
-    const int code = is_ann ? DARKANN : DARKCOMP;
+  for (int k = 0; k < G; ++k) {
+    double a = y[k], b = GRAD ? dy[k] : 0.0;
+    for (int off = 32; off > 0; off >>= 1) {
+      a += shfl_f64(a, lane ^ off);
+      if (GRAD) b += shfl_f64(b, lane ^ off);
+    }
+    if (lane == 0) {
+      s_sum[wid][2 * k] = a;
+      s_sum[wid][2 * k + 1] = b;
+    }
+  }
+  __syncthreads();
+  const int q = threadIdx.x;
+  if (q < 2 * G && k0 + (q >> 1) < n_pts)
+    part[(int64_t)blockIdx.x * (2 * kYieldBatch) + 2 * k0 + q] =
+        (s_sum[0][q] + s_sum[1][q]) + (s_sum[2][q] + s_sum[3][q]);
+}
+
+// Sums over the rows of every kernel of a pass, added to the points' totals.
+__global__ __launch_bounds__(256) void k_yield_sum(const double* part, int64_t rows, double* acc) {
+  __shared__ double s_sum[256];
+  const int q = blockIdx.x;  // 2 k: yield, 2 k + 1: derivative
+  double s = 0.0;
+  for (int64_t r = threadIdx.x; r < rows; r += 256) s += part[r * (2 * kYieldBatch) + q];
+  s_sum[threadIdx.x] = s;
+  __syncthreads();
+  for (int h = 128; h > 0; h >>= 1) {
+    if ((int)threadIdx.x < h) s_sum[threadIdx.x] += s_sum[threadIdx.x + h];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) acc[q] += s_sum[0];
+}
+
+// A process' sums over one species: w W(m_k) and w dW/dm(m_k) (GRAD = false:
+// the yield alone).  Between trained masses j and j+1 a particle's weight is
+// interpolated geometrically, W = exp(ln w_j + t ln(w_j+1 / w_j)), where both
+// are positive, linearly otherwise.  Points of one segment, and of the next,
+// share the trained masses' weights.
+template <bool GRAD, bool COMP>
+__global__ __launch_bounds__(256) void k_dark_yield(const YieldTables* __restrict__ Yp, int fam, YieldList L,
+                                                    YieldPoints P, double* __restrict__ part) {
+  constexpr int G = kYieldGroup;
+  const YieldTables& Y = *Yp;
+  const YieldRow* const rows = Y.rows;
+  const int k0 = blockIdx.y * G;
+  double y[G], dy[G];
 #pragma unroll
-    for (int k = 0; k < kYieldBatch; ++k) {
-      if (k >= n_pts) break;
+  for (int k = 0; k < G; ++k) y[k] = dy[k] = 0.0;
+  const int64_t n = (int64_t)*L.count, stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+    const float2 Ew = L.Ew[L.dir * i];
+    const double w = (double)Ew.y;
+    YieldArgs a{};
+    a.E0 = (double)Ew.x;
+    if (COMP) {
+      const double2 ph = L.ph[i];
+      a.l10 = ph.x;
+      a.ln_den = ph.y;
+    } else {
+      a.lf = __logf(Ew.x);
+    }
+    double lo = 0.0, hi = 0.0, llo = 0.0, lhi = 0.0;
+    int jc = -2;
+#pragma unroll
+    for (int k = 0; k < G; ++k) {
+      if (k0 + k >= P.n) break;
+      const int j = P.j[k0 + k];
+      if (j != jc) {
+        if (j == jc + 1) {
+          lo = hi;
+          llo = lhi;
+        } else {
+          yield_weight<COMP>(Y.t[j][fam], rows, a, lo, llo);
+        }
+        hi = lo;
+        lhi = llo;
+        if (j + 1 < Y.n_mass) yield_weight<COMP>(Y.t[j + 1][fam], rows, a, hi, lhi);
+        jc = j;
+      }
+      const double t = P.t[k0 + k];
       double W, dW;
-      bound_wd<GRAD>(T, Bv, k, code, wa, ln_den, ln_eps2, W, dW);
+      if (lo > 0.0 && hi > 0.0) {
+        const double r = lhi - llo;
+        W = exp(llo + t * r);
+        dW = GRAD ? W * r * P.dtdm[k0 + k] : 0.0;
+      } else {
+        const double l = COMP ? (lo > 0.0 ? exp(llo) : 0.0) : lo;
+        const double h = COMP ? (hi > 0.0 ? exp(lhi) : 0.0) : hi;
+        W = l + t * (h - l);
+        dW = GRAD ? (h - l) * P.dtdm[k0 + k] : 0.0;
+      }
       y[k] += w * W;
       if (GRAD) dy[k] += w * dW;
     }
   }
-#pragma unroll
-  for (int k = 0; k < kYieldBatch; ++k) {
-    double a = y[k], b = dy[k];
-    for (int off = 32; off > 0; off >>= 1) {
-      a += shfl_f64(a, (threadIdx.x & 63) ^ off);
-      if (GRAD) b += shfl_f64(b, (threadIdx.x & 63) ^ off);
-    }
-    if ((threadIdx.x & 63) == 0 && k < n_pts) {
-      unsafeAtomicAdd(acc + 2 * k, a);
-      if (GRAD) unsafeAtomicAdd(acc + 2 * k + 1, b);
+  yield_row<GRAD, G>(y, dy, k0, P.n, part);
+}
+
+// Rows of the bound-electron tables of point k from slot k * nv (m_k) and the
+// node derivatives in slot k * nv + 1 (quad::k_bound_deriv; nv = 1: none):
+// DarkAnn's W in E, then DarkComp's log10 n sigma in log10 E.
+__global__ __launch_bounds__(256) void k_bound_rows(const double* tab, int32_t stride, int32_t nv, BoundRow* rows) {
+  constexpr int n = quad::kBoundGrid;
+  const int i = threadIdx.x, comp = blockIdx.y;
+  if (i >= n) return;
+  const double* x = tab + (int64_t)blockIdx.x * nv * stride + (comp ? 4 * n : 0);
+  const double* y = x + (comp ? n : 3 * n);
+  const double* dx = x + stride;
+  const double* dy = y + stride;
+  const bool last = i == n - 1;
+  BoundRow R{x[i], last ? (double)INFINITY : x[i + 1], y[i], 0.0, nv == 3 ? dy[i] : 0.0, 0.0};
+  if (!last) {
+    const double inv = 1.0 / (R.xn - R.x), dv = y[i + 1] - R.y;
+    R.slope = dv / (R.xn - R.x);
+    if (nv == 3) {
+      R.c0 = dy[i] - dv * dx[i] * inv;
+      R.c1 = inv * ((dy[i + 1] - dy[i]) - dv * (dx[i + 1] - dx[i]) * inv);
     }
   }
+  rows[((int64_t)blockIdx.x * 2 + comp) * n + i] = R;
+}
+
+// The bound-electron processes' part of the yield (DarkAnn of positrons,
+// DarkComp of photons) from the tables at the points' masses, held in LDS:
+// W and dW/dm_V are the rows' interpolants, in log10 space for DarkComp (W =
+// eps^2 10^L / den, dW = W ln 10 dL).  Below the thresholds, and for DarkAnn
+// outside the grid, W = dW = 0; outside DarkComp's grid L = -20.
+template <bool GRAD, bool COMP>
+__global__ __launch_bounds__(256) void k_bound_yield(const quad::BoundSlot* __restrict__ slot,
+                                                     const BoundRow* __restrict__ rows, int32_t nv, double min_photon,
+                                                     YieldList L, YieldPoints P, double* __restrict__ part) {
+  constexpr int G = kBoundGroup, N = quad::kBoundGrid;
+  __shared__ BoundRow s_row[G][N];
+  const int k0 = blockIdx.y * G;
+  double thr[G], g0[G], inv[G], y[G], dy[G];
+#pragma unroll
+  for (int k = 0; k < G; ++k) {
+    y[k] = dy[k] = thr[k] = g0[k] = inv[k] = 0.0;
+    if (k0 + k >= P.n) continue;
+    const quad::BoundSlot& S = slot[(k0 + k) * nv];
+    thr[k] = COMP ? fmax(S.min_comp, min_photon) : S.min_ann;
+    g0[k] = COMP ? S.l0c : S.lnEa0;
+    inv[k] = COMP ? S.inv_dlc : S.inv_dln_a;
+    for (int i = threadIdx.x; i < N; i += 256) s_row[k][i] = rows[((int64_t)(k0 + k) * 2 + (COMP ? 1 : 0)) * N + i];
+  }
+  __syncthreads();
+  const int64_t n = (int64_t)*L.count, stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+    const float2 Ew = L.Ew[L.dir * i];
+    const double E0 = (double)Ew.x, w = (double)Ew.y;
+    double v = E0, ln_den = 0.0;
+    if (COMP) {
+      const double2 ph = L.ph[i];
+      v = ph.x;
+      ln_den = ph.y;
+    }
+    const float g = COMP ? (float)v : __logf(Ew.x);
+#pragma unroll
+    for (int k = 0; k < G; ++k) {
+      if (k0 + k >= P.n) break;
+      const BoundRow* const r = s_row[k];
+      if (E0 < thr[k]) continue;
+      const bool out = COMP ? (v < r[0].x || v > r[N - 1].x) : !(v >= r[0].x && v <= r[N - 1].x);
+      if (!COMP && out) continue;
+      double val = -20.0, d = 0.0;
+      if (!out) {
+        const int lo = find_row(r, N, v, g, g0[k], inv[k]);
+        const double u = v - r[lo].x;
+        val = r[lo].slope * u + r[lo].y;
+        if (GRAD) d = r[lo].c0 + r[lo].c1 * u;
+      }
+      if (COMP) {
+        val = exp(kLn10 * val - ln_den);
+        d = val * kLn10 * d;
+      }
+      y[k] += w * val;
+      if (GRAD) dy[k] += w * d;
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < G; ++k) {
+    const double e2 = k0 + k < P.n ? P.eps2[k0 + k] : 0.0;
+    y[k] *= e2;
+    dy[k] *= e2;
+  }
+  yield_row<GRAD, G>(y, dy, k0, P.n, part);
 }
 
 }  // namespace dark

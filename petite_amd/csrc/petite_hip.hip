@@ -1856,11 +1856,15 @@ struct PetiteCtx {
   double masses[PETITE_MAX_MASSES] = {};
   dark::YieldTables ytab{};
   dark::YieldTables* ytab_dev = nullptr;  // device copy read by the kernel
-  double* yield_blob = nullptr;
-  double* yacc = nullptr;
-  int32_t* ylist = nullptr;               // [2][ylist_cap]: the records of k_dark_yield, of k_bound_yield
+  std::vector<int> yactive;               // the model's processes
+  dark::YieldRow* yrows = nullptr;
+  double* yacc = nullptr;                 // the points' sums
+  int64_t yacc_cap = 0;
+  double* ypart = nullptr;                // the blocks' sums
+  int64_t ypart_cap = 0;
+  float2* ylist = nullptr;                // [2][ylist_cap]: species lists; double2[ylist_cap] of the photons behind
   int64_t ylist_cap = 0;
-  unsigned long long* ylist_cnt = nullptr;  // [2]
+  unsigned long long* ylist_cnt = nullptr;  // [kYieldSpecies]
   // bound-electron tables at each m_V of the yield (petite_yield_bound)
   bool bnd_on = false;
   quad::BoundParams bnd{};
@@ -1870,6 +1874,7 @@ struct PetiteCtx {
   double* bnd_blob = nullptr;          // survival and mean-free-path tables, running integrals, fixed nodes
   double* bnd_tab = nullptr;           // per slot: grids, log-log tables, weights, panel nodes
   quad::BoundSlot* bnd_slots = nullptr;
+  dark::BoundRow* bnd_rows = nullptr;  // per point: the packed intervals of DarkAnn and DarkComp
   quad::Job* bnd_jobs = nullptr;
   int* bnd_bad = nullptr;
   const double* bnd_fixed = nullptr;   // survival-grid panel nodes (in bnd_blob)
@@ -2278,8 +2283,8 @@ void petite_ctx_destroy(PetiteCtx* c) {
   }
   for (void* p : {(void*)c->d64, (void*)c->d32, (void*)c->dmaxf, (void*)c->req_slot, (void*)c->req_E, (void*)c->res_x,
                   (void*)c->res_trials, (void*)c->res_w, (void*)c->req_count, (void*)c->counters, (void*)c->ddesc,
-                  (void*)c->dsig_lds, (void*)c->dark_blob, (void*)c->dyield, (void*)c->yield_blob, (void*)c->yacc, (void*)c->ylist, (void*)c->ylist_cnt, (void*)c->ytab_dev,
-                  (void*)c->bnd_blob, (void*)c->bnd_tab, (void*)c->bnd_slots, (void*)c->bnd_jobs, (void*)c->bnd_bad,
+                  (void*)c->dsig_lds, (void*)c->dark_blob, (void*)c->dyield, (void*)c->yrows, (void*)c->yacc, (void*)c->ypart, (void*)c->ylist, (void*)c->ylist_cnt, (void*)c->ytab_dev,
+                  (void*)c->bnd_blob, (void*)c->bnd_tab, (void*)c->bnd_slots, (void*)c->bnd_jobs, (void*)c->bnd_bad, (void*)c->bnd_rows,
                   (void*)c->par.sid, (void*)c->par.pf, (void*)c->par.pos, (void*)c->par.info, (void*)c->tail_spill, (void*)c->longs})
     if (p) (void)hipFree(p);
   free_entries(c);
@@ -3206,20 +3211,48 @@ int petite_yield_setup(PetiteCtx* c, int32_t n_mass, const double* masses, const
         std::memcmp(descs[j].active, descs[0].active, sizeof(descs[0].active)) != 0)
       return fail(PETITE_ERR_ARG, "petite_yield_setup: the masses must share the active processes");
   }
-  if (c->yield_blob) {
-    (void)hipFree(c->yield_blob);
-    c->yield_blob = nullptr;
-  }
-  HIP_TRY(hipMalloc(&c->yield_blob, n * sizeof(double)));
-  HIP_TRY(hipMemcpy(c->yield_blob, blob, n * sizeof(double), hipMemcpyHostToDevice));
-  if (!c->yacc) HIP_TRY(hipMalloc(&c->yacc, 2 * dark::kYieldBatch * sizeof(double)));
-  c->n_mass = n_mass;
+  // the tables as rows of intervals
+  std::vector<dark::YieldRow> rows;
+  dark::YieldTables Y{};
   for (int j = 0; j < n_mass; ++j) {
-    c->masses[j] = masses[j];
-    c->ytab.d[j] = descs[j];
+    const PetiteDarkDesc& D = descs[j];
+    for (int f = 0; f <= dark::kYieldComp; ++f) {
+      const bool comp = f == dark::kYieldComp;
+      dark::YieldTable& t = Y.t[j][f];
+      const double* x = blob + (comp ? D.comp_off : D.w_off[f]);
+      t.n = comp ? D.comp_n : D.w_n[f];
+      t.off = (int32_t)rows.size();
+      t.g0 = comp ? D.comp_l0 : D.w_lnE0[f];
+      t.inv = comp ? D.comp_inv_dl : D.w_inv_dlog[f];
+      t.eps2 = D.eps2;
+      t.ln_eps2 = std::log(D.eps2);
+      t.thr = comp ? std::max(D.min_comp, c->dev.min_calc[2])
+                   : (f == dark::F_ANN ? D.min_ann : (f == dark::F_MUBREM ? D.min_muon_brem : D.min_brem));
+      if (t.n <= 0) continue;
+      t.x0 = x[0];
+      t.x1 = x[t.n - 1];
+      const double* y = x + t.n;
+      for (int i = 0; i < t.n; ++i) {
+        const bool last = i == t.n - 1;
+        rows.push_back({x[i], last ? (double)INFINITY : x[i + 1], y[i],
+                        last ? 0.0 : (y[i + 1] - y[i]) / (x[i + 1] - x[i])});
+      }
+    }
   }
-  c->ytab.n_mass = n_mass;
-  c->ytab.b = c->yield_blob;
+  if (c->yrows) {
+    (void)hipFree(c->yrows);
+    c->yrows = nullptr;
+  }
+  c->n_mass = 0;
+  HIP_TRY(hipMalloc(&c->yrows, std::max<size_t>(1, rows.size()) * sizeof(dark::YieldRow)));
+  if (!rows.empty())
+    HIP_TRY(hipMemcpy(c->yrows, rows.data(), rows.size() * sizeof(dark::YieldRow), hipMemcpyHostToDevice));
+  Y.rows = c->yrows;
+  Y.n_mass = n_mass;
+  c->ytab = Y;
+  c->yactive.assign(descs[0].active, descs[0].active + descs[0].n_active);
+  c->n_mass = n_mass;
+  for (int j = 0; j < n_mass; ++j) c->masses[j] = masses[j];
   c->bnd_on = false;  // a new model brings its own bound-electron inputs (petite_yield_bound)
   if (!c->ytab_dev) HIP_TRY(hipMalloc(&c->ytab_dev, sizeof(dark::YieldTables)));
   HIP_TRY(hipMemcpy(c->ytab_dev, &c->ytab, sizeof(dark::YieldTables), hipMemcpyHostToDevice));
@@ -3240,12 +3273,14 @@ int petite_yield_bound(PetiteCtx* c, const PetiteBoundDesc* d, const double* blo
   const double* nd = blob + d->nodes.off;
   for (int i = 1; i < d->nodes.n; ++i)
     if (!(nd[i] > nd[i - 1])) return fail(PETITE_ERR_ARG, "petite_yield_bound: nodes must ascend strictly");
-  for (void* p : {(void*)c->bnd_blob, (void*)c->bnd_tab, (void*)c->bnd_slots, (void*)c->bnd_jobs, (void*)c->bnd_bad})
+  for (void* p : {(void*)c->bnd_blob, (void*)c->bnd_tab, (void*)c->bnd_slots, (void*)c->bnd_jobs, (void*)c->bnd_bad,
+                  (void*)c->bnd_rows})
     if (p) (void)hipFree(p);
   c->bnd_blob = c->bnd_tab = nullptr;
   c->bnd_slots = nullptr;
   c->bnd_jobs = nullptr;
   c->bnd_bad = nullptr;
+  c->bnd_rows = nullptr;
   c->bnd_on = false;
   int64_t n_cum = 0;
   for (int q = 0; q < 3; ++q) n_cum += d->loss[q].n;
@@ -3255,6 +3290,7 @@ int petite_yield_bound(PetiteCtx* c, const PetiteBoundDesc* d, const double* blo
   HIP_TRY(hipMalloc(&c->bnd_slots, sizeof(quad::BoundSlot) * quad::kBoundMaxSlots));
   HIP_TRY(hipMalloc(&c->bnd_jobs, sizeof(quad::Job) * quad::kBoundMaxSlots));
   HIP_TRY(hipMalloc(&c->bnd_bad, sizeof(int)));
+  HIP_TRY(hipMalloc(&c->bnd_rows, sizeof(dark::BoundRow) * 2 * quad::kBoundGrid * dark::kYieldBatch));
   HIP_TRY(hipMemset(c->bnd_bad, 0, sizeof(int)));
   HIP_TRY(hipMemcpy(c->bnd_blob, blob, sizeof(double) * (size_t)n, hipMemcpyHostToDevice));
   // one job per slot; every slot shares the survival channels and their
@@ -3340,48 +3376,85 @@ int petite_dark_yield(PetiteCtx* c, const PetiteStore* sm, int64_t n_sm, int32_t
   DevStore S{(float4*)sm->p0, (float4*)sm->r0, (float4*)sm->pf, (float4*)sm->rf, sm->pid, sm->parent, sm->meta,
              sm->shower, sm->sid, sm->capacity};
   if (n_sm > INT32_MAX) return fail(PETITE_ERR_ARG, "petite_dark_yield: more than 2^31-1 records");
-  const int64_t blocks = std::max<int64_t>(1, std::min<int64_t>((n_sm + 255) / 256, (int64_t)c->n_cu * 8));
-  bool use_bound = false;
-  for (int a = 0; a < c->ytab.d[0].n_active; ++a)
-    use_bound |= c->ytab.d[0].active[a] == DARKANN || c->ytab.d[0].active[a] == DARKCOMP;
-  // the records each kernel visits, by species (bits: e-, e+, photon, mu-, mu+):
-  // k_dark_yield takes the interpolated processes' species, k_bound_yield
-  // positrons (DarkAnn) and photons (DarkComp) when the tables at each m_V
-  // carry those processes
-  const bool bound_all = c->bnd_on && use_bound;
-  uint32_t mask_a = 0u, mask_b = 0u;
-  for (int a = 0; a < c->ytab.d[0].n_active; ++a) {
-    const int code = c->ytab.d[0].active[a];
-    const bool bnd = code == DARKANN || code == DARKCOMP;
-    if (bound_all && bnd) {
-      mask_b |= code == DARKANN ? 2u : 4u;
+  if (n_points == 0) return PETITE_OK;
+  // the launches of a pass: the interpolated processes by species, and with
+  // the tables at each m_V positrons (DarkAnn) and photons (DarkComp)
+  struct Launch {
+    int species, fam;
+    bool bound;
+  };
+  std::vector<Launch> launches;
+  bool b_ann = false, b_comp = false, use_bound = false;
+  uint32_t mask = 0u;
+  for (const int code : c->yactive) {
+    if (code == DARKANN || code == DARKCOMP) use_bound = true;
+    if (c->bnd_on && (code == DARKANN || code == DARKCOMP)) {
+      (code == DARKANN ? b_ann : b_comp) = true;
       continue;
     }
-    if (code == DARKBREM) mask_a |= 1u | 2u;
-    else if (code == DARKANN) mask_a |= 2u;
-    else if (code == DARKMUONBREM) mask_a |= 8u | 16u;
-    else if (code == DARKCOMP) mask_a |= 4u;
-  }
-  if (n_sm > 0) {
-    if (c->ylist_cap < n_sm) {
-      if (c->ylist) HIP_TRY(hipFree(c->ylist));
-      c->ylist = nullptr;
-      c->ylist_cap = 0;
-      HIP_TRY(hipMalloc(&c->ylist, 2 * n_sm * sizeof(int32_t)));
-      c->ylist_cap = n_sm;
+    if (code == DARKBREM) {
+      launches.push_back({0, dark::F_BREM_E, false});
+      launches.push_back({1, dark::F_BREM_P, false});
+    } else if (code == DARKANN) {
+      launches.push_back({1, dark::F_ANN, false});
+    } else if (code == DARKMUONBREM) {
+      launches.push_back({3, dark::F_MUBREM, false});
+    } else if (code == DARKCOMP) {
+      launches.push_back({2, dark::kYieldComp, false});
     }
-    if (!c->ylist_cnt) HIP_TRY(hipMalloc(&c->ylist_cnt, 2 * sizeof(unsigned long long)));
-    HIP_TRY(hipMemsetAsync(c->ylist_cnt, 0, 2 * sizeof(unsigned long long), s));
-    hipLaunchKernelGGL(dark::k_yield_lists, dim3((unsigned)blocks), dim3(256), 0, s, S, n_sm, mask_a, mask_b, c->ylist,
-                       c->ylist + c->ylist_cap, c->ylist_cnt);
-    HIP_TRY(hipGetLastError());
   }
-  const dark::RecordList list_a{c->ylist, c->ylist_cnt}, list_b{c->ylist + c->ylist_cap, c->ylist_cnt + 1};
-  // passes over the points in ascending m_V, so that a pass needs few trained masses
+  use_bound = use_bound && c->bnd_on;
+  if (b_ann) launches.push_back({1, dark::F_ANN, true});
+  if (b_comp) launches.push_back({2, dark::kYieldComp, true});
+  for (const Launch& l : launches) mask |= 1u << l.species;
+  // the record in parts of at most kYieldChunk particles (32 B of lists each)
+  constexpr int64_t kYieldChunk = (int64_t)1 << 25;
+  const int64_t chunk = std::min(n_sm, kYieldChunk);
+  if (c->ylist_cap < chunk) {
+    if (c->ylist) HIP_TRY(hipFree(c->ylist));
+    c->ylist = nullptr;
+    c->ylist_cap = 0;
+    HIP_TRY(hipMalloc(&c->ylist, (size_t)chunk * 2 * (sizeof(float2) + sizeof(double))));
+    c->ylist_cap = chunk;
+  }
+  if (!c->ylist_cnt) HIP_TRY(hipMalloc(&c->ylist_cnt, dark::kYieldSpecies * sizeof(unsigned long long)));
+  const int64_t n_pass = (n_points + dark::kYieldBatch - 1) / dark::kYieldBatch;
+  const int64_t sums = n_pass * 2 * dark::kYieldBatch;
+  if (c->yacc_cap < sums) {
+    if (c->yacc) HIP_TRY(hipFree(c->yacc));
+    c->yacc = nullptr;
+    c->yacc_cap = 0;
+    HIP_TRY(hipMalloc(&c->yacc, sums * sizeof(double)));
+    c->yacc_cap = sums;
+  }
+  HIP_TRY(hipMemsetAsync(c->yacc, 0, sums * sizeof(double), s));
+  // blocks of each launch: the resident blocks of the chip over the groups of points
+  auto blocks_x = [&](bool bound, int n, int64_t records) {
+    const int g = bound ? dark::kBoundGroup : dark::kYieldGroup;
+    const int64_t groups = (n + g - 1) / g;
+    return std::max<int64_t>(1, std::min((records + 255) / 256, (int64_t)c->n_cu * (bound ? 4 : 8) / groups));
+  };
+  {
+    int64_t rows = 0;
+    for (const Launch& l : launches)
+      rows += std::max(blocks_x(l.bound, 1, chunk), blocks_x(l.bound, dark::kYieldBatch, chunk));
+    if (c->ypart_cap < rows) {
+      if (c->ypart) HIP_TRY(hipFree(c->ypart));
+      c->ypart = nullptr;
+      c->ypart_cap = 0;
+      HIP_TRY(hipMalloc(&c->ypart, rows * 2 * dark::kYieldBatch * sizeof(double)));
+      c->ypart_cap = rows;
+    }
+  }
+  double2* const ph = (double2*)(c->ylist + 2 * c->ylist_cap);
+  auto list_of = [&](int sp) {
+    const float2* base = c->ylist + (sp >> 1) * c->ylist_cap;
+    return dark::YieldList{(sp & 1) ? base + c->ylist_cap - 1 : base, ph, (sp & 1) ? -1 : 1, c->ylist_cnt + sp};
+  };
+  // the points in ascending m_V, with their segment and interpolation parameter
   std::vector<int> order(n_points);
   for (int k = 0; k < n_points; ++k) order[k] = k;
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return mV[a] < mV[b]; });
-  // segment and interpolation parameter of every point, ascending m_V
   std::vector<int> seg(n_points);
   std::vector<double> tt(n_points), dd(n_points);
   for (int q = 0; q < n_points; ++q) {
@@ -3400,28 +3473,20 @@ int petite_dark_yield(PetiteCtx* c, const PetiteStore* sm, int64_t n_sm, int32_t
     tt[q] = t;
     dd[q] = dtdm;
   }
-  // passes of at most kYieldBatch points whose segments fit one window of
-  // kYieldWindow consecutive trained masses
-  for (int k0 = 0; k0 < n_points;) {
+  for (int64_t pass = 0; pass < n_pass; ++pass) {
+    const int k0 = (int)pass * dark::kYieldBatch;
     dark::YieldPoints P{};
-    P.j0 = seg[k0];
-    P.n = 0;
-    while (P.n < dark::kYieldBatch && k0 + P.n < n_points && seg[k0 + P.n] + 1 < P.j0 + dark::kYieldWindow) ++P.n;
-    for (int q = 0; q < dark::kYieldWindow; ++q)
-      P.ln_eps2[q] = P.j0 + q < nm ? std::log(c->ytab.d[P.j0 + q].eps2) : 0.0;
+    P.n = std::min(n_points - k0, dark::kYieldBatch);
     for (int k = 0; k < P.n; ++k) {
-      const int j = seg[k0 + k] - P.j0;
-      P.j[k] = j;
+      P.j[k] = seg[k0 + k];
       P.t[k] = tt[k0 + k];
       P.dtdm[k] = dd[k0 + k];
-      P.need |= 1u << j;
-      if (P.j0 + j + 1 < nm) P.need |= 1u << (j + 1);
+      P.eps2[k] = c->ytab.t[seg[k0 + k]][0].eps2;
     }
-    dark::BoundView Bv{};
-    if (c->bnd_on && use_bound) {
+    const int nv = dyield_host ? 3 : 1;
+    if (use_bound) {
       // tables at each point's m_V (and m_V (1 +- h) for the derivative),
       // the grid tops of the trained mass at or below it
-      const int nv = dyield_host ? 3 : 1;
       quad::BoundPass BP{};
       BP.n_slots = P.n * nv;
       for (int k = 0; k < P.n; ++k) {
@@ -3435,11 +3500,12 @@ int petite_dark_yield(PetiteCtx* c, const PetiteStore* sm, int64_t n_sm, int32_t
           BP.top_comp[sl] = c->bnd_top_comp[j];
         }
       }
+      const int32_t stride = quad::kBoundTab + c->bnd.node_stride;
       hipLaunchKernelGGL(quad::k_bound_tables, dim3((unsigned)BP.n_slots), dim3(256), 0, s, c->bnd, BP, c->bnd_slots,
                          c->bnd_tab, c->bnd_jobs);
       HIP_TRY(hipGetLastError());
-      hipLaunchKernelGGL(quad::k_bound_nodes, dim3(1), dim3(64), 0, s, c->bnd, BP.n_slots, c->bnd_fixed, c->bnd_tab,
-                         c->bnd_jobs);
+      hipLaunchKernelGGL(quad::k_bound_nodes, dim3((unsigned)BP.n_slots), dim3(256), 0, s, c->bnd, c->bnd_fixed,
+                         c->bnd_tab, c->bnd_jobs);
       HIP_TRY(hipGetLastError());
       const int64_t n_int = (int64_t)BP.n_slots * quad::kBoundGrid;
       hipLaunchKernelGGL(quad::k_track_quad, dim3((unsigned)((n_int + quad::kWavesPerBlock - 1) / quad::kWavesPerBlock)),
@@ -3449,52 +3515,65 @@ int petite_dark_yield(PetiteCtx* c, const PetiteStore* sm, int64_t n_sm, int32_t
       if (nv == 3) {
         quad::BoundDeriv D{};
         D.n_pts = P.n;
-        D.stride = quad::kBoundTab + c->bnd.node_stride;
+        D.stride = stride;
         for (int k = 0; k < P.n; ++k) D.inv_2h[k] = 1.0 / (2.0 * c->bnd_h * mV[order[k0 + k]]);
         hipLaunchKernelGGL(quad::k_bound_deriv, dim3((unsigned)P.n), dim3(256), 0, s, D, c->bnd_tab);
         HIP_TRY(hipGetLastError());
       }
-      Bv.slot = c->bnd_slots;
-      Bv.tab = c->bnd_tab;
-      Bv.stride = quad::kBoundTab + c->bnd.node_stride;
-      Bv.nv = nv;
-    }
-    HIP_TRY(hipMemsetAsync(c->yacc, 0, 2 * dark::kYieldBatch * sizeof(double), s));
-    if (n_sm > 0) {
-      const bool bound_on = Bv.slot != nullptr;
-      if (dyield_host)
-        hipLaunchKernelGGL(dark::k_dark_yield<true>, dim3((unsigned)blocks), dim3(256), 0, s, c->dev,
-                           (const dark::YieldTables*)c->ytab_dev, S, list_a, P, bound_on, c->yacc);
-      else
-        hipLaunchKernelGGL(dark::k_dark_yield<false>, dim3((unsigned)blocks), dim3(256), 0, s, c->dev,
-                           (const dark::YieldTables*)c->ytab_dev, S, list_a, P, bound_on, c->yacc);
+      hipLaunchKernelGGL(dark::k_bound_rows, dim3((unsigned)P.n, 2), dim3(256), 0, s, (const double*)c->bnd_tab, stride,
+                         nv, c->bnd_rows);
       HIP_TRY(hipGetLastError());
-      if (bound_on) {
-        int ann = 0, comp = 0;
-        for (int a = 0; a < c->ytab.d[0].n_active; ++a) {
-          ann |= c->ytab.d[0].active[a] == DARKANN;
-          comp |= c->ytab.d[0].active[a] == DARKCOMP;
-        }
-        if (dyield_host)
-          hipLaunchKernelGGL(dark::k_bound_yield<true>, dim3((unsigned)blocks), dim3(256), 0, s, c->dev, S, list_b, P.n,
-                             ann, comp, P.ln_eps2[0], Bv, c->yacc);
-        else
-          hipLaunchKernelGGL(dark::k_bound_yield<false>, dim3((unsigned)blocks), dim3(256), 0, s, c->dev, S, list_b, P.n,
-                             ann, comp, P.ln_eps2[0], Bv, c->yacc);
+    }
+    for (int64_t first = 0; first < n_sm && mask; first += chunk) {
+      const int64_t n = std::min(chunk, n_sm - first);
+      if (pass == 0 || chunk < n_sm) {  // (one part: the lists serve every pass)
+        HIP_TRY(hipMemsetAsync(c->ylist_cnt, 0, dark::kYieldSpecies * sizeof(unsigned long long), s));
+        hipLaunchKernelGGL(dark::k_yield_lists,
+                           dim3((unsigned)std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, (int64_t)c->n_cu * 8))),
+                           dim3(256), 0, s, S, first, n, mask, c->ylist, c->ylist_cap, c->ylist_cnt);
         HIP_TRY(hipGetLastError());
+        if (mask & 4u) {
+          hipLaunchKernelGGL(dark::k_yield_photons,
+                             dim3((unsigned)std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, (int64_t)c->n_cu * 8))),
+                             dim3(256), 0, s, c->dev, list_of(2), ph);
+          HIP_TRY(hipGetLastError());
+        }
       }
+      int64_t rows = 0;
+      for (const Launch& l : launches) {
+        const int64_t bx = blocks_x(l.bound, P.n, n);
+        const int g = l.bound ? dark::kBoundGroup : dark::kYieldGroup;
+        const dim3 grid((unsigned)bx, (unsigned)((P.n + g - 1) / g));
+        double* const part = c->ypart + rows * 2 * dark::kYieldBatch;
+        const bool comp = l.fam == dark::kYieldComp;
+        if (l.bound) {
+          auto* const f = dyield_host ? (comp ? dark::k_bound_yield<true, true> : dark::k_bound_yield<true, false>)
+                                      : (comp ? dark::k_bound_yield<false, true> : dark::k_bound_yield<false, false>);
+          hipLaunchKernelGGL(f, grid, dim3(256), 0, s, (const quad::BoundSlot*)c->bnd_slots,
+                             (const dark::BoundRow*)c->bnd_rows, nv, c->dev.min_calc[2], list_of(l.species), P, part);
+        } else {
+          auto* const f = dyield_host ? (comp ? dark::k_dark_yield<true, true> : dark::k_dark_yield<true, false>)
+                                      : (comp ? dark::k_dark_yield<false, true> : dark::k_dark_yield<false, false>);
+          hipLaunchKernelGGL(f, grid, dim3(256), 0, s, (const dark::YieldTables*)c->ytab_dev, l.fam,
+                             list_of(l.species), P, part);
+        }
+        HIP_TRY(hipGetLastError());
+        rows += bx;
+      }
+      hipLaunchKernelGGL(dark::k_yield_sum, dim3((unsigned)(2 * P.n)), dim3(256), 0, s, (const double*)c->ypart, rows,
+                         c->yacc + pass * 2 * dark::kYieldBatch);
+      HIP_TRY(hipGetLastError());
     }
-    double h[2 * dark::kYieldBatch];
-    HIP_TRY(hipMemcpyAsync(h, c->yacc, sizeof(h), hipMemcpyDeviceToHost, s));
-    int bad = 0;
-    if (Bv.slot) HIP_TRY(hipMemcpyAsync(&bad, c->bnd_bad, sizeof(int), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    if (bad) return fail(PETITE_ERR_INTERNAL, "petite_dark_yield: a bound-electron weight needs more than 512 panel edges");
-    for (int k = 0; k < P.n; ++k) {
-      yield_host[order[k0 + k]] = h[2 * k];
-      if (dyield_host) dyield_host[order[k0 + k]] = h[2 * k + 1];
-    }
-    k0 += P.n;
+  }
+  std::vector<double> h((size_t)sums);
+  HIP_TRY(hipMemcpyAsync(h.data(), c->yacc, sums * sizeof(double), hipMemcpyDeviceToHost, s));
+  int bad = 0;
+  if (use_bound) HIP_TRY(hipMemcpyAsync(&bad, c->bnd_bad, sizeof(int), hipMemcpyDeviceToHost, s));
+  HIP_TRY(hipStreamSynchronize(s));
+  if (bad) return fail(PETITE_ERR_INTERNAL, "petite_dark_yield: a bound-electron weight needs more than 512 panel edges");
+  for (int k = 0; k < n_points; ++k) {
+    yield_host[order[k]] = h[2 * (size_t)k];
+    if (dyield_host) dyield_host[order[k]] = h[2 * (size_t)k + 1];
   }
   return PETITE_OK;
 }

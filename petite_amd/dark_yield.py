@@ -15,8 +15,8 @@ petite_yield_bound), and their dY/dm_V is the central difference of tables
 at m_V (1 +- 1e-5).  The trained masses are the
 shipped ones and those of the generated mass pack
 (petite_amd.tablegen.dark_masses); a mass outside [lightest, heaviest] raises
-PetiteError (petite_dark_yield rejects it: nothing to interpolate).  One float64 pass of the
-k_dark_yield kernel returns Y and dY/dm_V for up to 16 masses at a time;
+PetiteError (petite_dark_yield rejects it: nothing to interpolate).  A float64
+pass returns Y and dY/dm_V for up to 32 masses at a time;
 dY/d(eps^2) = Y.  ``DarkYield.__call__`` wraps it in a torch.autograd.Function.
 """
 import ctypes as C
