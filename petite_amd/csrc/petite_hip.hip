@@ -61,14 +61,16 @@ enum CounterIdx {
   C_LONG = 25,                // draws handed to k_draw_long
   C_YIELD_OUT = 26,           // particles the current sweep's transport handed on to the next sweep
   C_RPARITY = 27,             // which half of the resume buffer the current sweep reads
-  C_SPILL = 28,               // [2] depth-first walk: entries in each spill list
   C_TAIL_STEPS = 30,          // particle-steps taken in depth-first walks
   C_STATS = 32,               // [ST_N] run statistics
   C_PTRIALS = 64,             // [PETITE_NPROC] candidates per process
   C_PDRAWS = 80,              // [PETITE_NPROC] draws per process
   C_PVIOL = 96,               // [PETITE_NPROC] accepted draws above max_F per process
   C_REFILL = 112,             // [PETITE_NPROC] per-process draw refill counters, kCtrLine apart
-  C_N = C_REFILL + kCtrLine * PETITE_NPROC
+  C_SPILL = C_REFILL + kCtrLine * PETITE_NPROC,  // [2] walk: entries at the front of each spill list
+  C_MUSPILL = C_SPILL + kCtrLine,                // [2] and muons at its back
+  C_MUCLAIM = C_MUSPILL + kCtrLine,              // claims of the latter
+  C_N = C_MUCLAIM + kCtrLine
 };
 __host__ __device__ constexpr int refill_ctr(int p) { return C_REFILL + kCtrLine * p; }
 
@@ -2657,7 +2659,6 @@ int petite_run_showers(PetiteCtx* c, const PetitePrimary* prim, int64_t n, uint6
         HIP_TRY(hipMalloc(&c->tail_spill, 2 * store->capacity * sizeof(int32_t)));
         c->tail_spill_cap = store->capacity;
       }
-      const int64_t scap = c->tail_spill_cap;
       // the first walk alone (it often leaves no spill), then kTailGroup per
       // host check: a launch whose inputs are empty ends at once
       const int ng = tail_launches == 0 ? 1 : kTailGroup;
@@ -2665,9 +2666,8 @@ int petite_run_showers(PetiteCtx* c, const PetitePrimary* prim, int64_t n, uint6
         hipLaunchKernelGGL(k_tail_setup, dim3(1), dim3(64), 0, s, ctr, c->drange, store->capacity, rcap, tpar);
         HIP_TRY(hipGetLastError());
         if (c->timing) HIP_TRY(hipEventRecord(c->tev[4 * group + 2 * g], s));
-        const TailParams tp{c->tail_spill + (int64_t)tpar * scap, ctr + C_SPILL + tpar,
-                            c->tail_spill + (int64_t)(tpar ^ 1) * scap, ctr + C_SPILL + (tpar ^ 1), scap,
-                            tn.tail_depth, tail_limit(tn.tail_budget, tail_launches)};
+        const TailParams tp{c->tail_spill, c->tail_spill_cap, tpar, tn.tail_depth,
+                            tail_limit(tn.tail_budget, tail_launches)};
         hipLaunchKernelGGL(k_tail, dim3(tail_blocks), dim3(256), lds, s, c->dev, S, seed, shower_energy, ctr,
                            c->dsig_lds, (const int64_t*)c->drange, ResumeBuf{c->dresume, rcap}, tp);
         HIP_TRY(hipGetLastError());
@@ -2677,9 +2677,9 @@ int petite_run_showers(PetiteCtx* c, const PetitePrimary* prim, int64_t n, uint6
         tpar ^= 1;
         ++tail_launches;
       }
-      unsigned long long h_spill = 0;
+      unsigned long long h_spill[kCtrLine + 2] = {};  // C_SPILL.., C_MUSPILL..
       HIP_TRY(hipMemcpyAsync(&h_store, ctr + C_STORE, sizeof(h_store), hipMemcpyDeviceToHost, s));
-      HIP_TRY(hipMemcpyAsync(&h_spill, ctr + C_SPILL + tpar, sizeof(h_spill), hipMemcpyDeviceToHost, s));
+      HIP_TRY(hipMemcpyAsync(h_spill, ctr + C_SPILL, sizeof(h_spill), hipMemcpyDeviceToHost, s));
       HIP_TRY(hipStreamSynchronize(s));
       if (c->timing) {
         for (int g = 0; g < ng; ++g) {
@@ -2689,7 +2689,7 @@ int petite_run_showers(PetiteCtx* c, const PetitePrimary* prim, int64_t n, uint6
         }
       }
       if ((int64_t)h_store > store->capacity) break;
-      if (h_spill == 0) break;  // every particle walked
+      if (h_spill[tpar] == 0 && h_spill[kCtrLine + tpar] == 0) break;  // every particle walked
       if (tail_launches > 100000) return fail(PETITE_ERR_HIP, "petite_run_showers: tail launch runaway");
       continue;
     }

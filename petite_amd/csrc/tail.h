@@ -21,26 +21,37 @@
 // comes from the particle's own Philox stream, as in the sweeps, so the records
 // are the sweeps' records, bit for bit.
 //
+// A muon's vertices follow one another, 13 substeps and a draw phase each, and
+// the longest muon sets the run's length.  A wave with muons therefore keeps to
+// them: their other children go straight to the spill list, muons of a list go
+// to its back, and every second wave of a launch takes its share of those
+// first, alone in its wave while there are enough waves.
+//
 // What bounds it: the latency of a substep (~600 dependent instructions) and of
-// a draw phase, at 2 waves per SIMD.  Its predecessor walked one particle per
-// wave, every lane computing the same transport, with two atomics per draw on
-// one line of per-process counters; 400 GeV beam of 2,000 in lead: 264 ms per
-// run with it (170 ms of that in the walk), 166 ms now, all of it walk.
+// a draw phase, at 2 waves per SIMD; with muons the longest of them (32,000
+// substeps and 2,400 phases, 70 ms alone).  1,000 electrons of 10 GeV in
+// graphite 5.5 ms a run, 40,000 mixed primaries in lead 76 ms.  A 400 GeV beam
+// of 2,000 in lead, half of them muons: 88 ms; 137 ms with each muon among the
+// particles of its own subtree; 264 ms (170 ms of that in the walk) with one
+// particle per wave, every lane computing the same transport, and two atomics
+// per draw on one line of per-process counters.
 #pragma once
 
 constexpr int kTailMaxDepth = 128;  // stack entries per wave
 constexpr int kTailGroup = 4;       // walk launches queued per host check after the first
 constexpr int kTailStepsPerParticle = 8;  // iterations of a wave per particle of its lanes' budget
 constexpr int kTailPhaseSteps = 4;        // iterations a draw phase counts for
+// A launch with muons: at most kMuonIters iterations of a wave that holds some,
+// and a quarter of that of the others, whose iterations (64 lanes instead of a
+// few) take about three times as long.
+constexpr int kMuonIters = 2048;
 
 struct TailParams {
-  const int32_t* spill_in;            // slots left by the previous launch
-  const unsigned long long* n_spill_in;
-  int32_t* spill_out;                 // slots past a full stack or the launch's share
-  unsigned long long* n_spill_out;
-  int64_t spill_cap;  // the store's capacity: a list holds every particle there is room for
-  int32_t depth;   // stack entries per wave (1..kTailMaxDepth)
-  int64_t limit;   // iterations after which a wave starts no more particles
+  int32_t* spill;   // [2][cap]: slots left for the next launch, muons from a list's end
+  int64_t cap;      // the store's capacity: a list holds every particle there is room for
+  int32_t par;      // list this launch reads (counted at C_SPILL + par, C_MUSPILL + par)
+  int32_t depth;    // stack entries per wave (1..kTailMaxDepth)
+  int32_t limit;    // iterations after which a wave starts no more particles
 };
 
 // A wave's buffers in LDS.
@@ -50,6 +61,30 @@ struct WalkLds {
   float4 xs[64];     //   the 4-D point as the draw kernels store it,
   int32_t tr[64];    //   the candidate count (negative: none in max_trials)
 };
+__device__ inline bool is_muon(int pid) { return pid == 13 || pid == -13; }
+
+// The slots v (>= 0) of the calling lanes at the end of the next launch's list,
+// muons from its back; 1 where there is no room (reported by the run as an
+// internal error).
+__device__ __noinline__ int walk_hand_on(int32_t* list, int64_t cap, unsigned long long* count, int32_t v, bool muon) {
+  const int lane = threadIdx.x & 63;
+  const unsigned long long below = (1ull << lane) - 1ull;
+  int lost = 0;
+  for (int m = 0; m < 2; ++m) {
+    const bool mine = v >= 0 && muon == (m == 1);
+    const unsigned long long om = __ballot(mine);
+    if (!om) continue;
+    unsigned long long o = 0;
+    if (lane == 0) o = atomicAdd(count + (m ? C_MUSPILL - C_SPILL : 0), (unsigned long long)__popcll(om));
+    o = shfl_u64(o, 0) + (unsigned long long)__popcll(om & below);
+    if (mine) {
+      if ((int64_t)o < cap) list[m ? cap - 1 - (int64_t)o : (int64_t)o] = v;
+      else lost = 1;
+    }
+  }
+  return lost;
+}
+
 // Per-process draw statistics of a block.
 struct WalkStats {
   unsigned long long trials[8], draws[8], viol[8];
@@ -139,12 +174,16 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
   const ResumeRec* rin = RB.rec ? RB.rec + (int64_t)(counters[C_RPARITY] & 1ull) * RB.cap : nullptr;
   // a count past the list (children that did not fit, an internal error the
   // run reports) is cut to the list
-  const int64_t n_in = (int64_t)*TPm.n_spill_in;
-  const int64_t total = nres + n + (n_in < TPm.spill_cap ? n_in : TPm.spill_cap);
-  // items per claim: an even share of every wave of the launch, at most a lane's each
+  const int32_t* const spill_in = TPm.spill + TPm.par * TPm.cap;
+  const int64_t total = nres + n + min((int64_t)counters[C_SPILL + TPm.par], TPm.cap);
+  const int64_t n_mu = min((int64_t)counters[C_MUSPILL + TPm.par], TPm.cap);
+  // items per claim: an even share of every wave of the launch (of every second
+  // one for muons), at most a lane's each
   const int64_t waves = (int64_t)gridDim.x * kWalkWaves;
   const int share = (int)min((int64_t)64, max((int64_t)1, (total + waves - 1) / waves));
-  if ((int64_t)blockIdx.x * kWalkWaves * share >= total) return;
+  const int share_mu = (int)min((int64_t)64, max((int64_t)1, (2 * n_mu + waves - 1) / waves));
+  if ((int64_t)blockIdx.x * kWalkWaves >= (total + share - 1) / share + (n_mu + share_mu - 1) / share_mu) return;
+  const int limit_mu = min(TPm.limit, kMuonIters), limit = n_mu > 0 ? min(TPm.limit, kMuonIters / 4) : TPm.limit;
   HIP_DYNAMIC_SHARED(double, s_sig)
   __shared__ WalkLds s_walk[kWalkWaves];
   __shared__ WalkStats s_stat;
@@ -161,38 +200,47 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
   enum { EMPTY = 0, STEP = 1, PARKED = 2, GIVEN = 3 };
   int mode = EMPTY;
   int sp = 0;              // stack entries (wave-uniform, as the next four)
-  int64_t iters = 0;
-  bool exhausted = false, fresh = true;
+  int iters = 0;
+  bool exhausted = total <= 0, mu_exhausted = n_mu <= 0, fresh = true;
+  bool muons = false;      // the wave holds muons, and keeps to them (see the head of the file)
   int32_t slot = 0;
   int pid = 0, shower = 0, gen = 0;
   uint32_t ch = 0xFFFu;
   uint64_t sid = 0;
-  double m = 0.0, pme = 0.0, E = 0.0, p = 0.0, dep = 0.0, dz = 0.0;
+  double m = 0.0, pme = 0.0, E = 0.0, dep = 0.0;
+  double dz = 0.0;  // substep length; |p| of a particle that does not move
   float nx = 0.0f, ny = 0.0f, nz = 0.0f, rx = 0.0f, ry = 0.0f, rz = 0.0f, wgt = 0.0f;
   uint32_t k = 0;
   bool closing = false;
-  unsigned long long steps = 0, n_fail = 0, n_drop = 0, n_ovf = 0, n_lost = 0;
+  unsigned int steps = 0, n_fail = 0, n_drop = 0, n_ovf = 0, n_lost = 0;  // of this lane in this launch
   while (true) {
-    // past its share the wave starts no more: the next launch spreads what it
-    // leaves.  A wave whose particles all have lanes and include a muon goes on:
-    // a muon's chain of thousands of vertices sets the run's length, and
-    // would go slower among a spread's other particles
-    const bool stop = iters >= TPm.limit && (sp > 0 || __ballot(mode != EMPTY && (pid == 13 || pid == -13)) == 0ull);
+    // past its share the wave starts no more: the next launch spreads what it leaves
+    if (muons) muons = __ballot(mode != EMPTY && is_muon(pid)) != 0ull;
+    const bool stop = iters >= (muons ? limit_mu : limit);
     // ---- free lanes take from the stack, then claim items (after a draw
     // phase, or when no lane is stepping)
     const unsigned long long im = __ballot(mode == EMPTY);
     int64_t rr = -1;
-    if (im && !stop && (fresh || __ballot(mode == STEP) == 0ull)) {
+    if (im && !stop && !muons && (fresh || __ballot(mode == STEP) == 0ull)) {
       const int rank = __popcll(im & below);
       const int take = min(__popcll(im), sp);
-      bool got = false;
+      bool got = false, got_mu = false;
+      if (!mu_exhausted && sp == 0 && im == ~0ull) {
+        unsigned long long c = 0;
+        if (lane == 0) c = atomicAdd(counters + C_MUCLAIM, (unsigned long long)share_mu);
+        c = shfl_u64(c, 0);
+        got = lane < share_mu && (int64_t)c + lane < n_mu;
+        if (got) slot = spill_in[TPm.cap - 1 - ((int64_t)c + lane)];
+        got_mu = (int64_t)c < n_mu;
+        mu_exhausted = (int64_t)c + share_mu >= n_mu;
+      }
       if (mode == EMPTY && rank < take) {
         slot = W.stack[sp - 1 - rank];
         got = true;
       }
       sp -= take;
       const int need = min(__popcll(im) - take, share);
-      if (need > 0 && !exhausted) {
+      if (need > 0 && !exhausted && !got_mu) {
         unsigned long long c = 0;
         if (lane == 0) c = atomicAdd(counters + C_TRANSPORT, (unsigned long long)need);
         c = shfl_u64(c, 0);
@@ -200,7 +248,7 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
           rr = (int64_t)c + (rank - take);
           got = rr < total;
           if (got) slot = rr < nres ? rin[rr].slot
-                                    : (rr < nres + n ? (int32_t)(first + (rr - nres)) : TPm.spill_in[rr - nres - n]);
+                                    : (rr < nres + n ? (int32_t)(first + (rr - nres)) : spill_in[rr - nres - n]);
         }
         exhausted = (int64_t)c + need >= total;
       }
@@ -220,6 +268,7 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
         wgt = r0.w;
         mode = GIVEN;
       }
+      muons = __ballot(mode == GIVEN && is_muon(pid)) != 0ull;
     }
     // ---- the given particles' starts (k_transport's refill)
     if (mode == GIVEN) {
@@ -234,7 +283,7 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
         nz *= inv;
       }
       const bool still = ch == 0xFFFu && pid != 22;
-      p = still ? sqrt((double)pn2) : 0.0;  // the others' |p| is formed when they finish
+      if (still) dz = sqrt((double)pn2);  // the others' |p| is formed when they finish
       dep = 0.0;
       k = 0;
       closing = false;
@@ -345,7 +394,7 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
     float4 pf = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     if (mode == PARKED) {
       steps += k;
-      if (!(ch == 0xFFFu && pid != 22)) p = momentum(E, m);
+      const double p = ch == 0xFFFu && pid != 22 ? dz : momentum(E, m);
       pf = make_float4((float)E, (float)(p * nx), (float)(p * ny), (float)(p * nz));
       S.pf[slot] = pf;
       S.rf[slot] = make_float4(rx, ry, rz, (float)k);
@@ -456,28 +505,32 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
     }
     // the stores above are read by other lanes of the wave
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    // the lane goes on with its higher-energy child, unless the wave stops
-    const int lower = (cslot[0] >= 0 && cslot[1] >= 0) ? (lab[1].e < lab[0].e ? 1 : 0) : (cslot[0] >= 0 ? 1 : 0);
-    const int higher = 1 - lower;
+    // the lane goes on with its higher-energy child, unless the wave stops; in
+    // a wave with muons with its muon, and the others are handed on
+    int higher = cslot[0] >= 0 && (cslot[1] < 0 || lab[1].e < lab[0].e) ? 0 : 1;
+    bool hmu = false, lmu = false;
+    if (muons) {
+      hmu = is_muon(cpid[higher]);
+      lmu = cslot[1 - higher] >= 0 && is_muon(cpid[1 - higher]);
+      if (lmu && !hmu) {
+        higher = 1 - higher;
+        hmu = true;
+        lmu = false;
+      }
+    }
     const int32_t hs = higher ? cslot[1] : cslot[0], ls = higher ? cslot[0] : cslot[1];
-    const bool go_on = hs >= 0 && !stop;
+    const bool go_on = hs >= 0 && !stop && (hmu || !muons);
     for (int t = 0; t < 2; ++t) {
       const int32_t v = t == 0 ? (go_on ? -1 : hs) : ls;
       const unsigned long long pm = __ballot(v >= 0);
       if (!pm) continue;
-      const int at = sp + __popcll(pm & below);
+      const int at = muons ? depth : sp + __popcll(pm & below);
       if (v >= 0 && at < depth) W.stack[at] = v;
-      const unsigned long long om = __ballot(v >= 0 && at >= depth);
-      if (om) {
-        unsigned long long o = 0;
-        if (lane == 0) o = atomicAdd(TPm.n_spill_out, (unsigned long long)__popcll(om));
-        o = shfl_u64(o, 0) + (unsigned long long)__popcll(om & below);
-        if (v >= 0 && at >= depth) {
-          if ((int64_t)o < TPm.spill_cap) TPm.spill_out[o] = v;
-          else ++n_lost;  // reported by the run as an internal error
-        }
-      }
-      sp = min(depth, sp + __popcll(pm));
+      const int32_t out = at >= depth ? v : -1;
+      if (__ballot(out >= 0))
+        n_lost += walk_hand_on(TPm.spill + (TPm.par ^ 1) * TPm.cap, TPm.cap, counters + C_SPILL + (TPm.par ^ 1), out,
+                               t == 0 ? hmu : lmu);
+      if (!muons) sp = min(depth, sp + __popcll(pm));
     }
     if (go_on) {
       const float4 c = higher ? cp[1] : cp[0];
@@ -495,33 +548,30 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
   // ---- what the wave did not start goes to the next launch, and so do the
   // items no wave claimed (a handed-on one starts over there: its random
   // numbers are indexed by its substeps, so it ends the same)
+  int32_t* const spill_out = TPm.spill + (TPm.par ^ 1) * TPm.cap;
+  unsigned long long* const n_out = counters + C_SPILL + (TPm.par ^ 1);
   while (!exhausted) {
     unsigned long long c = 0;
     if (lane == 0) c = atomicAdd(counters + C_TRANSPORT, 64ull);
     c = shfl_u64(c, 0);
     exhausted = (int64_t)c + 64 >= total;
-    const int64_t have = min((int64_t)64, max((int64_t)0, total - (int64_t)c));
-    if (have == 0) break;
-    unsigned long long o = 0;
-    if (lane == 0) o = atomicAdd(TPm.n_spill_out, (unsigned long long)have);
-    o = shfl_u64(o, 0);
-    if (lane < have) {
-      const int64_t rr = (int64_t)c + lane;
-      const int32_t v = rr < nres ? rin[rr].slot
-                                  : (rr < nres + n ? (int32_t)(first + (rr - nres)) : TPm.spill_in[rr - nres - n]);
-      if ((int64_t)(o + lane) < TPm.spill_cap) TPm.spill_out[o + lane] = v;
-      else ++n_lost;
-    }
+    const int64_t rr = (int64_t)c + lane;
+    int32_t v = -1;
+    if (rr < total)
+      v = rr < nres ? rin[rr].slot
+                    : (rr < nres + n ? (int32_t)(first + (rr - nres)) : spill_in[rr - nres - n]);
+    n_lost += walk_hand_on(spill_out, TPm.cap, n_out, v, v >= 0 && is_muon(S.pid[v]));
   }
-  if (sp > 0) {
-    unsigned long long o = 0;
-    if (lane == 0) o = atomicAdd(TPm.n_spill_out, (unsigned long long)sp);
-    o = shfl_u64(o, 0);
-    for (int e = lane; e < sp; e += 64) {
-      if ((int64_t)(o + e) < TPm.spill_cap) TPm.spill_out[o + e] = W.stack[e];
-      else ++n_lost;
-    }
+  while (!mu_exhausted) {
+    unsigned long long c = 0;
+    if (lane == 0) c = atomicAdd(counters + C_MUCLAIM, 64ull);
+    c = shfl_u64(c, 0);
+    mu_exhausted = (int64_t)c + 64 >= n_mu;
+    const int64_t rr = (int64_t)c + lane;
+    n_lost += walk_hand_on(spill_out, TPm.cap, n_out, rr < n_mu ? spill_in[TPm.cap - 1 - rr] : -1, true);
   }
+  for (int e0 = 0; e0 < sp; e0 += 64)
+    n_lost += walk_hand_on(spill_out, TPm.cap, n_out, e0 + lane < sp ? W.stack[e0 + lane] : -1, false);
   {
     unsigned long long* const st = counters + C_STATS;
     const unsigned long long v[7] = {steps, steps, n_fail, n_drop, n_ovf, n_lost, 0ull};
@@ -549,9 +599,10 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
 // spread often while their number grows and seldom once a few long chains
 // remain (a spread costs a launch, and leaves a chain among other particles);
 // budgets above 2^30 never stop a wave.
-static int64_t tail_limit(int32_t budget, int64_t i) {
-  if (budget > (1 << 30)) return (int64_t)1 << 62;
-  return (int64_t)std::max(budget, 1) * kTailStepsPerParticle << std::min<int64_t>(i, 20);
+static int32_t tail_limit(int32_t budget, int64_t i) {
+  if (budget > (1 << 30)) return INT32_MAX;
+  return (int32_t)std::min<int64_t>((int64_t)std::max(budget, 1) * kTailStepsPerParticle << std::min<int64_t>(i, 20),
+                                    INT32_MAX);
 }
 
 // Start of a tail launch: the items are the particles handed on by the last
@@ -571,7 +622,9 @@ __global__ void k_tail_setup(unsigned long long* ctr, int64_t* range, int64_t ca
     ctr[C_RPARITY] ^= 1ull;
     ctr[C_TRANSPORT] = 0ull;
     ctr[C_SPILL + (par ^ 1)] = 0ull;
-    if (sr.n > 0 || sr.nres > 0 || ctr[C_SPILL + par] > 0ull) ctr[C_SWEEPS] += 1ull;
+    ctr[C_MUSPILL + (par ^ 1)] = 0ull;
+    ctr[C_MUCLAIM] = 0ull;
+    if (sr.n > 0 || sr.nres > 0 || ctr[C_SPILL + par] > 0ull || ctr[C_MUSPILL + par] > 0ull) ctr[C_SWEEPS] += 1ull;
   }
 }
 

@@ -76,3 +76,24 @@ def test_walk_leaves_the_sweeps_records(lead, batch):
         for k in ("n_particles", "n_steps", "n_draws", "n_trials", "n_dropped", "n_maxf_viol", "n_draws_proc",
                   "n_trials_proc", "n_viol_proc"):
             assert st[k] == s[k], (batch, name, k)
+
+
+# muons have waves and a list of their own: one muon; one of them and other
+# particles in a wave; more than a lane each in every second wave of a launch
+MUONS = {"one": (1, 60.0, 60.0, [13]), "mixed": (1500, 0.02, 20.0, [13, -13, 11, 22]), "many": (9001, 0.2, 1.5, [13, -13])}
+
+
+@pytest.mark.parametrize("batch", MUONS)
+def test_muons_walk_apart(lead, batch):
+    prim = _primaries(*MUONS[batch], seed=6)
+    ref, energy, st = _run(lead, prim, {"tail_sweep": 1})
+    for name, tuning in WALKS.items():
+        if name == "handed on":
+            tuning = dict(tuning, tail_sweep=len(prim) + 1)
+        got, e, s = _run(lead, prim, dict(tuning, tail_waves=1))
+        for k in ref:
+            # the bits: a muon below its rest mass has no momentum
+            assert ref[k].tobytes() == got[k].tobytes(), (batch, name, k)
+        assert np.allclose(energy, e, rtol=1e-12, atol=1e-12), (batch, name)
+        for k in ("n_particles", "n_steps", "n_draws", "n_trials", "n_dropped", "n_maxf_viol"):
+            assert st[k] == s[k], (batch, name, k)
