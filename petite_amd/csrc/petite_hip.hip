@@ -42,7 +42,7 @@ int fail(int code, const std::string& msg) {
 // ST_OVERFLOW: children past the store capacity; ST_REQ_OVERFLOW: draw requests
 // past their process's region (impossible while a sweep holds at most as many
 // particles as a region holds requests; counted as a backstop).
-enum StatIdx { ST_STEPS = 0, ST_DRAWS, ST_TRIALS, ST_VIOL, ST_NOSAMPLE, ST_DROPPED, ST_OVERFLOW, ST_REQ_OVERFLOW, ST_N = 8 };
+enum StatIdx { ST_STEPS = 0, ST_NOSAMPLE, ST_DROPPED, ST_OVERFLOW, ST_REQ_OVERFLOW, ST_N = 8 };
 
 // Layout of the context's counter block (unsigned long long).  Atomics on one
 // 128-byte line are served one after another, also on different addresses:
@@ -106,6 +106,7 @@ struct DrawLaunch {
   float* w_out;
   unsigned long long* counters;
   const unsigned int* dcount;  // non-null: counts on the device, plan made by each block
+  int32_t half_runs;           // a wave starts with half of its share instead of a chunk (draw_loop)
   int32_t full_blocks;         // blocks of a whole-GPU launch (device plan)
   int32_t min_lg;              // log2 of the fewest lanes per request
   int32_t group_requests;      // requests a lane group is sized to serve (small counts)
@@ -186,18 +187,23 @@ __device__ inline void block_stat_add(const unsigned long long (&v)[N], unsigned
 
 // Hands out request indices to the lanes in ``need`` from wave-private
 // chunks of ``chunk`` consecutive indices (one atomic per chunk); a take asks
-// for at most ``chunk`` of them.
+// for at most ``chunk`` of them.  [cur, end) may start as a run of the wave's
+// own: the indices below ``first`` are dealt out that way, and the counter
+// counts from there (none are asked of it past ``count``).
 struct WaveQueue {
   int chunk = 64;
-  int64_t cur = 0, end = 0;
+  int64_t cur = 0, end = 0, first = 0, count = INT64_MAX;
   __device__ inline int64_t take(unsigned long long need_mask, bool need, unsigned long long* counter) {
     const int lane = threadIdx.x & 63;
     const int n = __popcll(need_mask);
     const int64_t avail = end - cur;
     unsigned long long nb = 0;
     if (avail < n) {
-      if (lane == 0) nb = atomicAdd(counter, (unsigned long long)chunk);
-      nb = shfl_u64(nb, 0);
+      nb = (unsigned long long)first;
+      if (first < count) {
+        if (lane == 0) nb += atomicAdd(counter, (unsigned long long)chunk);
+        nb = shfl_u64(nb, 0);
+      }
     }
     int64_t r = -1;
     if (need) {
@@ -287,7 +293,8 @@ __device__ inline double candidate_w(const DevTables& T, double E, const float* 
 // refills less often than a single lane, and larger G cuts the latency of
 // sweeps with fewer requests than lanes.
 template <int p>
-__device__ void draw_loop(const DevTables& T, const DrawLaunch& io, uint64_t seed, const int64_t count, int lgG, int blocks) {
+__device__ void draw_loop(const DevTables& T, const DrawLaunch& io, uint64_t seed, const int64_t count, int lgG, int block,
+                          int blocks) {
   constexpr int ND = proc_ndim<p>();
   const int lane = threadIdx.x & 63;
   int G = 1 << lgG;
@@ -302,6 +309,21 @@ __device__ void draw_loop(const DevTables& T, const DrawLaunch& io, uint64_t see
   // first wave: 130 us for a handful of one-candidate draws.
   WaveQueue q;
   q.chunk = (int)min((int64_t)64, max((int64_t)(64 >> lgG), count / (16 * (int64_t)blocks)));
+  // The first run of a wave is dealt out: the queue's accesses are served one
+  // after another (10 ns each), and the first and last ones of 4,096 waves took
+  // half of a call of 10,000 one-candidate draws (160 -> 112 us).  A chunk in a
+  // run's sweeps, where the processes' launches overlap and waves start late
+  // (100,000 primaries 164 ms, 172 with half a share); half of the share in
+  // k_draw_small for a call (1e6 mixed draws 481 us, 528 with a chunk).
+  {
+    const int64_t wave = (int64_t)block * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    const int64_t waves = (int64_t)blocks * (blockDim.x >> 6);
+    const int64_t run = io.half_runs ? max((int64_t)(64 >> lgG), count / (2 * waves)) : q.chunk;
+    q.first = waves * run;
+    q.count = count;
+    q.cur = min(wave * run, count);
+    q.end = min(q.cur + run, count);
+  }
   bool have = false, done = false;
   bool drained = false;  // wave-uniform: the request queue is empty
   int late = 0;          // rounds since
@@ -441,11 +463,10 @@ __device__ void draw_loop(const DevTables& T, const DrawLaunch& io, uint64_t see
   // every block of a draw launch calls draw_loop (a block-uniform choice), so
   // the whole block reaches this point
   unsigned long long* const ctr = io.counters;
-  const unsigned long long v[7] = {n_trials, n_draw, n_viol, n_fail, n_trials, n_draw, n_viol};
-  unsigned long long* const dst[7] = {ctr + C_STATS + ST_TRIALS, ctr + C_STATS + ST_DRAWS, ctr + C_STATS + ST_VIOL,
-                                      ctr + C_STATS + ST_NOSAMPLE, ctr + C_PTRIALS + p, ctr + C_PDRAWS + p,
+  const unsigned long long v[4] = {n_fail, n_trials, n_draw, n_viol};
+  unsigned long long* const dst[4] = {ctr + C_STATS + ST_NOSAMPLE, ctr + C_PTRIALS + p, ctr + C_PDRAWS + p,
                                       ctr + C_PVIOL + p};
-  block_stat_add<7>(v, dst);
+  block_stat_add<4>(v, dst);
 }
 
 // One kernel per process: the integrand, the map dimension and the
@@ -454,8 +475,6 @@ __device__ void draw_loop(const DevTables& T, const DrawLaunch& io, uint64_t see
 // The 4-D draws need 129-132 VGPRs unconstrained (3 waves per SIMD); held to
 // 128 (4 waves, no spills) they hide more of their map gathers' latency: the
 // Brem draw stage is 4 % faster.  Five waves (96 VGPRs) spill and are slower.
-// (k_draw_small, which holds every process's draw, spills at 128: it keeps
-// its 132.)
 template <int P>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_draw(DevTables T, DrawLaunch io, uint64_t seed) {
   if (io.dcount) {
@@ -465,10 +484,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     int lg, blocks;
     draw_plan((double)cnt, io.full_blocks, io.min_lg, io.group_requests, lg, blocks);
     if ((int)blockIdx.x >= blocks) return;
-    draw_loop<P>(T, io, seed, cnt, lg, blocks);
+    draw_loop<P>(T, io, seed, cnt, lg, (int)blockIdx.x, blocks);
   } else {
     if (io.count[P] <= 0) return;
-    draw_loop<P>(T, io, seed, io.count[P], io.lgG[P], (int)gridDim.x);
+    draw_loop<P>(T, io, seed, io.count[P], io.lgG[P], (int)blockIdx.x, (int)gridDim.x);
   }
 }
 
@@ -567,11 +586,10 @@ __global__ __launch_bounds__(256) void k_draw_long_finish(DevTables T, DrawLaunc
     }
   }
   unsigned long long* const ctr = io.counters;
-  const unsigned long long v[7] = {n_trials, n_draw, n_viol, n_fail, n_trials, n_draw, n_viol};
-  unsigned long long* const dst[7] = {ctr + C_STATS + ST_TRIALS, ctr + C_STATS + ST_DRAWS, ctr + C_STATS + ST_VIOL,
-                                      ctr + C_STATS + ST_NOSAMPLE, ctr + C_PTRIALS + P, ctr + C_PDRAWS + P,
+  const unsigned long long v[4] = {n_fail, n_trials, n_draw, n_viol};
+  unsigned long long* const dst[4] = {ctr + C_STATS + ST_NOSAMPLE, ctr + C_PTRIALS + P, ctr + C_PDRAWS + P,
                                       ctr + C_PVIOL + P};
-  block_stat_add<7>(v, dst);
+  block_stat_add<4>(v, dst);
 }
 
 typedef void (*DrawKernel)(DevTables, DrawLaunch, uint64_t);
@@ -621,14 +639,9 @@ __device__ void draw_block_one(const DevTables& T, const DrawLaunch& io, uint64_
         xo[3] = (float)x[3];
         io.trials_out[oidx] = (int32_t)(jc + 1);
         io.w_out[oidx] = (float)w;
-        atomicAdd(io.counters + C_STATS + ST_TRIALS, (unsigned long long)(jc + 1));
-        atomicAdd(io.counters + C_STATS + ST_DRAWS, 1ull);
         atomicAdd(io.counters + C_PTRIALS + p, (unsigned long long)(jc + 1));
         atomicAdd(io.counters + C_PDRAWS + p, 1ull);
-        if (w > mf) {
-          atomicAdd(io.counters + C_STATS + ST_VIOL, 1ull);
-          atomicAdd(io.counters + C_PVIOL + p, 1ull);
-        }
+        if (w > mf) atomicAdd(io.counters + C_PVIOL + p, 1ull);
       }
       return;
     }
@@ -637,25 +650,39 @@ __device__ void draw_block_one(const DevTables& T, const DrawLaunch& io, uint64_
   if (threadIdx.x == 0) {
     io.trials_out[oidx] = -(int32_t)max_trials;
     io.w_out[oidx] = 0.0f;
-    atomicAdd(io.counters + C_STATS + ST_TRIALS, (unsigned long long)max_trials);
-    atomicAdd(io.counters + C_STATS + ST_DRAWS, 1ull);
     atomicAdd(io.counters + C_STATS + ST_NOSAMPLE, 1ull);
     atomicAdd(io.counters + C_PTRIALS + p, (unsigned long long)max_trials);
     atomicAdd(io.counters + C_PDRAWS + p, 1ull);
   }
 }
 
-// The draws of a small sweep: every SM process in one launch on the
-// caller's stream, blocks [p * per, (p + 1) * per) for process p (bit p of
-// `procs` set); a process with at most `per` requests takes one block per
-// request (draw_block_one).  In the last sweeps of a run, where a handful of requests
-// remain, the per-process launches on their own streams cost more in
-// launches, forks and joins than the draws themselves.  Same draw loop, so
-// the same results.
-__global__ __launch_bounds__(256) void k_draw_small(DevTables T, DrawLaunch io, uint64_t seed, int per, uint32_t procs) {
-  const int p = (int)blockIdx.x / per;
-  const int b = (int)blockIdx.x - p * per;
-  if (p >= 8 || !((procs >> p) & 1u)) return;
+// The draws of a small sweep, or of a call: every SM
+// process in one launch of 8 share blocks on the caller's stream (bit p of
+// `procs`: the process is among them).  The processes that hold a sixteenth of
+// the requests or more split six shares of blocks evenly (at most
+// io.full_blocks each: a process alone fills the chip), the others get a
+// quarter of a share; a process with at most as many requests as blocks takes
+// one block per request (draw_block_one).  In the last sweeps of a run, where
+// a handful of requests remain, the per-process launches on their own streams
+// cost more in launches, forks and joins than the draws themselves.  Same draw
+// loop, so the same results.
+__global__ __launch_bounds__(256) void k_draw_small(DevTables T, DrawLaunch io, uint64_t seed, int share, uint32_t procs) {
+  int64_t total = 0;
+  for (int q = 0; q < 8; ++q)
+    if ((procs >> q) & 1u) total += io.dcount[q];
+  uint32_t big = 0u;
+  for (int q = 0; q < 8; ++q)
+    if (((procs >> q) & 1u) && io.dcount[q] > 0 && 16 * (int64_t)io.dcount[q] >= total) big |= 1u << q;
+  if (!big) return;
+  const int per_big = min(io.full_blocks, 6 * share / __popc(big));
+  int p = 0, b = (int)blockIdx.x, per = 0;
+  for (; p < 8; ++p) {
+    const bool used = ((procs >> p) & 1u) && io.dcount[p] > 0;
+    per = used ? (((big >> p) & 1u) ? per_big : max(1, share / 4)) : 0;
+    if (b < per) break;
+    b -= per;
+  }
+  if (p >= 8) return;
   const int64_t cnt = min((int64_t)io.dcount[p], io.req_cap);
   if (cnt <= (int64_t)per) {
     if (b >= cnt) return;
@@ -675,14 +702,14 @@ __global__ __launch_bounds__(256) void k_draw_small(DevTables T, DrawLaunch io, 
   draw_plan((double)cnt, per, io.min_lg, io.group_requests, lg, blocks);
   if (b >= blocks) return;
   switch (p) {
-    case 0: draw_loop<0>(T, io, seed, cnt, lg, blocks); break;
-    case 1: draw_loop<1>(T, io, seed, cnt, lg, blocks); break;
-    case 2: draw_loop<2>(T, io, seed, cnt, lg, blocks); break;
-    case 3: draw_loop<3>(T, io, seed, cnt, lg, blocks); break;
-    case 4: draw_loop<4>(T, io, seed, cnt, lg, blocks); break;
-    case 5: draw_loop<5>(T, io, seed, cnt, lg, blocks); break;
-    case 6: draw_loop<6>(T, io, seed, cnt, lg, blocks); break;
-    default: draw_loop<7>(T, io, seed, cnt, lg, blocks); break;
+    case 0: draw_loop<0>(T, io, seed, cnt, lg, b, blocks); break;
+    case 1: draw_loop<1>(T, io, seed, cnt, lg, b, blocks); break;
+    case 2: draw_loop<2>(T, io, seed, cnt, lg, b, blocks); break;
+    case 3: draw_loop<3>(T, io, seed, cnt, lg, b, blocks); break;
+    case 4: draw_loop<4>(T, io, seed, cnt, lg, b, blocks); break;
+    case 5: draw_loop<5>(T, io, seed, cnt, lg, b, blocks); break;
+    case 6: draw_loop<6>(T, io, seed, cnt, lg, b, blocks); break;
+    default: draw_loop<7>(T, io, seed, cnt, lg, b, blocks); break;
   }
 }
 
@@ -2086,6 +2113,36 @@ static int launch_draws_device(PetiteCtx* c, const DrawLaunch& io, uint64_t seed
   return PETITE_OK;
 }
 
+// Explicit draws in one launch (k_draw_small) with the counts left on the
+// device: no count readback before it, no streams to fork and join, and the
+// next process' blocks take a process' last waves.  Its share of blocks by the
+// number of requests n, few where a wave would end after a draw or two (us a
+// call of mixed draws on 256 CUs with shares of 128, 192, 256 and 384, then
+// with a launch per process): 16,384 80, 113, 129, 142, 323; 262,144 197, 195,
+// 215, 288, 611; 1e6 508, 455, 429, 481, 905; 16e6 6980, 5860, 5900, 5580,
+// 6030.  0: contexts with dark processes, which k_draw_small does not hold.
+static int draw_mixed_blocks(const PetiteCtx* c, int64_t n) {
+  for (int p = 8; p < PETITE_NPROC; ++p)
+    if (c->desc.grid[p].n_E > 0) return 0;
+  const int quarters = n <= (1 << 16) ? 2 : (n <= (1 << 19) ? 3 : (n <= (1 << 21) ? 4 : 6));
+  return std::max(16, c->n_cu * quarters / 4);
+}
+
+static int launch_draws_mixed(PetiteCtx* c, DrawLaunch io, int per, const unsigned int* counts, uint64_t seed,
+                              hipStream_t s) {
+  uint32_t procs = 0;
+  for (int p = 0; p < 8; ++p)
+    if (c->desc.grid[p].n_E > 0) procs |= 1u << p;
+  io.dcount = counts;
+  io.half_runs = 1;
+  io.full_blocks = c->n_cu * 4;
+  io.min_lg = lanes_log2(c->tune.min_group_lanes);
+  io.group_requests = c->tune.group_requests;
+  hipLaunchKernelGGL(k_draw_small, dim3((unsigned)(8 * per)), dim3(256), 0, s, c->dev, io, seed, per, procs);
+  HIP_TRY(hipGetLastError());
+  return PETITE_OK;
+}
+
 // Device address of `scratch` on each device, looked up once per device with
 // that device current (the array's host-side name is not a device address).
 static std::mutex g_noalloc_mu;
@@ -2418,9 +2475,6 @@ int petite_vegas_draw(PetiteCtx* c, const int32_t* proc, const double* E, const 
   hipLaunchKernelGGL(k_bucket, dim3(request_blocks(n)), dim3(256), 0, s, c->dev, proc, E, n, c->req_slot, c->req_E,
                      c->req_cap, c->req_count, trials_out, w_out);
   HIP_TRY(hipGetLastError());
-  unsigned int rq[PETITE_NPROC];
-  HIP_TRY(hipMemcpyAsync(rq, c->req_count, sizeof(rq), hipMemcpyDeviceToHost, s));
-  HIP_TRY(hipStreamSynchronize(s));
   DrawLaunch io{};
   io.req_slot = c->req_slot;
   io.req_E = c->req_E;
@@ -2431,10 +2485,17 @@ int petite_vegas_draw(PetiteCtx* c, const int32_t* proc, const double* E, const 
   io.trials_out = trials_out;
   io.w_out = w_out;
   io.counters = c->counters;
-  io.longs = c->longs;
-  int64_t blocks = 0;
-  plan_draw(c, rq, io, blocks);
-  rc = launch_draws(c, io, seed, s);
+  if (const int per = draw_mixed_blocks(c, n)) {
+    rc = launch_draws_mixed(c, io, per, c->req_count, seed, s);
+  } else {
+    unsigned int rq[PETITE_NPROC];
+    HIP_TRY(hipMemcpyAsync(rq, c->req_count, sizeof(rq), hipMemcpyDeviceToHost, s));
+    HIP_TRY(hipStreamSynchronize(s));
+    io.longs = c->longs;
+    int64_t blocks = 0;
+    plan_draw(c, rq, io, blocks);
+    rc = launch_draws(c, io, seed, s);
+  }
   if (rc) return rc;
   unsigned long long st[ST_N];
   HIP_TRY(hipMemcpyAsync(st, c->counters + C_STATS, sizeof(st), hipMemcpyDeviceToHost, s));
@@ -2462,9 +2523,6 @@ int petite_vegas_draw_noalloc(PetiteCtx* c, const int32_t* proc, const double* E
   hipLaunchKernelGGL(k_bucket, dim3(request_blocks(n)), dim3(256), 0, s, c->dev, proc, E, n, req_slot, req_E,
                      kNoAllocCap, counts, trials_out, w_out);
   HIP_TRY(hipGetLastError());
-  unsigned int rq[PETITE_NPROC];
-  HIP_TRY(hipMemcpyAsync(rq, counts, sizeof(rq), hipMemcpyDeviceToHost, s));
-  HIP_TRY(hipStreamSynchronize(s));
   DrawLaunch io{};
   io.req_slot = req_slot;
   io.req_E = req_E;
@@ -2475,9 +2533,17 @@ int petite_vegas_draw_noalloc(PetiteCtx* c, const int32_t* proc, const double* E
   io.trials_out = trials_out;
   io.w_out = w_out;
   io.counters = ctr;
-  int64_t blocks = 0;
-  plan_draw(c, rq, io, blocks);
-  int rc = launch_draws_serial(c, io, seed, s);
+  int rc;
+  if (const int per = draw_mixed_blocks(c, n)) {
+    rc = launch_draws_mixed(c, io, per, counts, seed, s);
+  } else {
+    unsigned int rq[PETITE_NPROC];
+    HIP_TRY(hipMemcpyAsync(rq, counts, sizeof(rq), hipMemcpyDeviceToHost, s));
+    HIP_TRY(hipStreamSynchronize(s));
+    int64_t blocks = 0;
+    plan_draw(c, rq, io, blocks);
+    rc = launch_draws_serial(c, io, seed, s);
+  }
   if (rc) return rc;
   unsigned long long st[ST_N];
   HIP_TRY(hipMemcpyAsync(st, ctr + C_STATS, sizeof(st), hipMemcpyDeviceToHost, s));
@@ -2553,7 +2619,7 @@ int petite_run_showers(PetiteCtx* c, const PetitePrimary* prim, int64_t n, uint6
   io.w_out = c->res_w;
   io.counters = ctr;
   io.dcount = c->req_count;
-  io.full_blocks = 0;  // per process, set by launch_draws_device
+  io.full_blocks = c->n_cu * 4;  // of k_draw_small; launch_draws_device sets each process'
   EmitLaunch em{};
   em.req_slot = c->req_slot;
   em.req_E = c->req_E;
@@ -2746,7 +2812,7 @@ int petite_run_showers(PetiteCtx* c, const PetitePrimary* prim, int64_t n, uint6
       const int64_t lanes_blocks = (last + 255) / 256;
       small_tr = (unsigned)std::min<int64_t>(tr_blocks, std::max<int64_t>(c->n_cu, lanes_blocks));
       small_em = (unsigned)std::min<int64_t>(em_blocks, std::max<int64_t>(c->n_cu, lanes_blocks));
-      small_per = (int)std::min<int64_t>(std::max(64, draw_blocks(c, BREM)), std::max<int64_t>(64, (last + 31) / 32));
+      small_per = (int)std::min<int64_t>(std::max(64, c->n_cu * 3 / 2), std::max<int64_t>(64, (last + 31) / 32));
     }
     if ((int64_t)h_store > store->capacity) break;  // children were dropped: report the size reached
     if (h_range[1] == 0 && h_range[3] == 0 && (int64_t)h_store == h_range[2]) break;  // the last sweep found nothing to do
@@ -2764,33 +2830,24 @@ int petite_run_showers(PetiteCtx* c, const PetitePrimary* prim, int64_t n, uint6
     }
   }
   drop_graph();
-  unsigned long long hs[ST_N], sweeps = 0;
-  HIP_TRY(hipMemcpyAsync(hs, ctr + C_STATS, sizeof(hs), hipMemcpyDeviceToHost, s));
-  HIP_TRY(hipMemcpyAsync(&sweeps, ctr + C_SWEEPS, sizeof(sweeps), hipMemcpyDeviceToHost, s));
+  unsigned long long h_ctr[C_REFILL];  // every counter that is read
+  HIP_TRY(hipMemcpyAsync(h_ctr, ctr, sizeof(h_ctr), hipMemcpyDeviceToHost, s));
   HIP_TRY(hipStreamSynchronize(s));
+  const unsigned long long* const hs = h_ctr + C_STATS;
   const int64_t written = (int64_t)h_store;
   stats->n_particles = written;
   stats->n_steps = (int64_t)hs[ST_STEPS];
-  stats->n_draws = (int64_t)hs[ST_DRAWS];
-  stats->n_trials = (int64_t)hs[ST_TRIALS];
-  stats->n_maxf_viol = (int64_t)hs[ST_VIOL];
   stats->n_no_sample = (int64_t)hs[ST_NOSAMPLE];
-  stats->n_iterations = (int64_t)sweeps;
+  stats->n_iterations = (int64_t)h_ctr[C_SWEEPS];
   stats->n_dropped = (int64_t)hs[ST_DROPPED];
-  {
-    unsigned long long pt[PETITE_NPROC], pd[PETITE_NPROC], pv[PETITE_NPROC];
-    HIP_TRY(hipMemcpyAsync(pt, ctr + C_PTRIALS, sizeof(pt), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipMemcpyAsync(pd, ctr + C_PDRAWS, sizeof(pd), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipMemcpyAsync(pv, ctr + C_PVIOL, sizeof(pv), hipMemcpyDeviceToHost, s));
-    unsigned long long ts = 0;
-    HIP_TRY(hipMemcpyAsync(&ts, ctr + C_TAIL_STEPS, sizeof(ts), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    stats->n_steps_tail = (int64_t)ts;
-    for (int p = 0; p < PETITE_NPROC; ++p) {
-      stats->n_viol_proc[p] = (int64_t)pv[p];
-      stats->n_trials_proc[p] = (int64_t)pt[p];
-      stats->n_draws_proc[p] = (int64_t)pd[p];
-    }
+  stats->n_steps_tail = (int64_t)h_ctr[C_TAIL_STEPS];
+  for (int p = 0; p < PETITE_NPROC; ++p) {
+    stats->n_viol_proc[p] = (int64_t)h_ctr[C_PVIOL + p];
+    stats->n_trials_proc[p] = (int64_t)h_ctr[C_PTRIALS + p];
+    stats->n_draws_proc[p] = (int64_t)h_ctr[C_PDRAWS + p];
+    stats->n_maxf_viol += stats->n_viol_proc[p];
+    stats->n_trials += stats->n_trials_proc[p];
+    stats->n_draws += stats->n_draws_proc[p];
   }
   stats->ms_transport = t_tr;
   stats->ms_draw = t_dr;
@@ -3179,17 +3236,18 @@ int petite_dark_reweight(PetiteCtx* c, const PetiteStore* sm, int64_t n_sm, uint
       out_base += (int64_t)n_m;
     }
   }
-  unsigned long long hs[ST_N], dst[3];
-  HIP_TRY(hipMemcpyAsync(hs, ctr + C_STATS, sizeof(hs), hipMemcpyDeviceToHost, s));
-  HIP_TRY(hipMemcpyAsync(dst, ctr + C_DARK_STATS, sizeof(dst), hipMemcpyDeviceToHost, s));
+  unsigned long long h_ctr[C_REFILL];
+  HIP_TRY(hipMemcpyAsync(h_ctr, ctr, sizeof(h_ctr), hipMemcpyDeviceToHost, s));
   HIP_TRY(hipMemcpyAsync(stats->yield, c->dyield, 5 * sizeof(double), hipMemcpyDeviceToHost, s));
   HIP_TRY(hipStreamSynchronize(s));
-  stats->n_vectors = (int64_t)dst[1];
-  stats->n_zero_rate = (int64_t)dst[0];
-  stats->n_pe_fail = (int64_t)dst[2];
-  stats->n_draws = (int64_t)hs[ST_DRAWS];
-  stats->n_trials = (int64_t)hs[ST_TRIALS];
-  stats->n_no_sample = (int64_t)hs[ST_NOSAMPLE];
+  stats->n_vectors = (int64_t)h_ctr[C_DARK_STATS + 1];
+  stats->n_zero_rate = (int64_t)h_ctr[C_DARK_STATS];
+  stats->n_pe_fail = (int64_t)h_ctr[C_DARK_STATS + 2];
+  for (int p = 0; p < PETITE_NPROC; ++p) {
+    stats->n_draws += (int64_t)h_ctr[C_PDRAWS + p];
+    stats->n_trials += (int64_t)h_ctr[C_PTRIALS + p];
+  }
+  stats->n_no_sample = (int64_t)h_ctr[C_STATS + ST_NOSAMPLE];
   stats->ms_select = t_sel;
   stats->ms_meson = t_me;
   stats->ms_draw = t_dr;

@@ -582,14 +582,9 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
   if (threadIdx.x < 8) {
     const int q = threadIdx.x;
     if (s_stat.draws[q]) {
-      atomicAdd(counters + C_STATS + ST_TRIALS, s_stat.trials[q]);
-      atomicAdd(counters + C_STATS + ST_DRAWS, s_stat.draws[q]);
       atomicAdd(counters + C_PTRIALS + q, s_stat.trials[q]);
       atomicAdd(counters + C_PDRAWS + q, s_stat.draws[q]);
-      if (s_stat.viol[q]) {
-        atomicAdd(counters + C_STATS + ST_VIOL, s_stat.viol[q]);
-        atomicAdd(counters + C_PVIOL + q, s_stat.viol[q]);
-      }
+      if (s_stat.viol[q]) atomicAdd(counters + C_PVIOL + q, s_stat.viol[q]);
     }
   }
 }

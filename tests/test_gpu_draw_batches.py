@@ -68,3 +68,21 @@ def test_groups_that_grow(ctx, P, E, n):
         assert np.array_equal(t[s], ts)
         assert np.array_equal(w[s], ws)
         assert np.array_equal(x[s], xs)
+
+
+# one launch for all processes, its blocks shared by their counts: processes
+# that hold almost nothing, one that holds everything, the edges of the rule's
+# ranges and of a block per request
+@pytest.mark.parametrize("shares", [{"Brem": 1.0}, {"Brem": 0.5, "PairProd": 0.3, "Ann": 0.2},
+                                    {"Comp": 0.98, "Brem": 0.01, "Ann": 0.005, "MuonBrem": 0.005}], ids=["one", "three", "few"])
+@pytest.mark.parametrize("n", [1, 127, 129, 1 << 16, (1 << 16) + 1, (1 << 19) + 1, (1 << 21) + 1])
+def test_processes_in_one_launch(ctx, n, shares):
+    rng = np.random.default_rng(n)
+    proc = rng.choice([all_process_code[P] for P in shares], size=n, p=list(shares.values())).astype(np.int32)
+    E = np.exp(rng.uniform(np.log(0.2), np.log(80.0), n))
+    sid = rng.integers(0, 2 ** 62, n)
+    x, t, w = _draw(ctx, proc, E, sid)
+    assert np.all(t > 0)
+    some = np.unique(np.concatenate([np.arange(min(n, 300)), rng.integers(0, n, 1500)]))
+    xs, ts, ws = _pieces(ctx, proc[some], E[some], sid[some], 61)
+    assert np.array_equal(t[some], ts) and np.array_equal(w[some], ws) and np.array_equal(x[some], xs)
