@@ -1716,9 +1716,30 @@ __global__ void k_draw_pe(const uint64_t* sid, int64_t n, uint64_t seed, double 
 struct DetectorPlanes {
   int32_t n;
   int32_t has_ecut;
-  double radius, inner, emin, emax;
+  double s_out, s_in, emin, emax;  // squared radii (radius_square_limits)
   double z[PETITE_MAX_DETECTORS];
 };
+
+// s_out, s_in with sqrt(s) < radius exactly where s < s_out and sqrt(s) >
+// inner exactly where s > s_in: the smallest and the largest double on the
+// other side (the root, rounded correctly, never decreases).
+static void radius_square_limits(double radius, double inner, double& s_out, double& s_in) {
+  const double inf = (double)INFINITY;
+  s_out = radius;  // none below a radius of 0, -inf or NaN
+  if (radius > 0.0) {
+    double s = radius * radius;
+    while (s > 0.0 && std::sqrt(s) >= radius) s = std::nextafter(s, 0.0);
+    while (std::sqrt(s) < radius) s = std::nextafter(s, inf);
+    s_out = s;
+  }
+  s_in = inner;  // every s >= 0 above a negative one, none above NaN
+  if (inner >= 0.0) {
+    double s = inner * inner;
+    while (s > 0.0 && std::sqrt(s) > inner) s = std::nextafter(s, 0.0);
+    while (s < inf && std::sqrt(std::nextafter(s, inf)) <= inner) s = std::nextafter(s, inf);
+    s_in = s;
+  }
+}
 
 __device__ inline double wave_sum_f64(double v) {
   for (int off = 32; off > 0; off >>= 1) v += shfl_f64(v, (threadIdx.x & 63) ^ off);
@@ -1726,22 +1747,24 @@ __device__ inline double wave_sum_f64(double v) {
 }
 
 // Pass bits of one record for planes [0, n_planes): T = (z - z0) / pz,
-// r_T = |(x0 + T px, y0 + T py)|, inner < r_T < radius.
+// r_T = |(x0 + T px, y0 + T py)|, inner < r_T < radius (on r_T^2).
 __device__ inline bool plane_pass(const DetectorPlanes& D, int d, double x0, double y0, double z0, double px, double py,
                                   double pz) {
 #pragma clang fp contract(off)
   const double T = (D.z[d] - z0) / pz;
   const double xf = x0 + T * px, yf = y0 + T * py;
-  const double rT = sqrt(xf * xf + yf * yf);
-  return rT > D.inner && rT < D.radius;
+  const double s = xf * xf + yf * yf;
+  return s > D.s_in && s < D.s_out;
 }
 
-// Grid-stride over the records.  With at most kRegPlanes planes every thread
-// keeps its weight sums in registers and they are reduced once per wave at
-// the end; otherwise each block pass reduces them per wave.  Per block the
-// wave sums meet in LDS, then one float64 atomic per block and plane.
-constexpr int kRegPlanes = 8;
-template <bool REG>
+// Grid-stride over the records.  With at most REG planes every thread keeps
+// its weight sums in registers and they are reduced once per wave at the end;
+// REG = 0 reduces them per wave in each pass.  Per block the wave sums meet in
+// LDS, then one float64 atomic per block and plane.  1e6 records at 12 planes:
+// 27 us with sums in registers, 66 with a reduction per pass, a root per plane
+// and four times the blocks.
+constexpr int kRegPlanes[2] = {8, 16};
+template <int REG>
 __global__ __launch_bounds__(256) void k_detector_cut(const float4* __restrict__ p, const float4* __restrict__ r,
                                                       int64_t n, DetectorPlanes D, uint64_t* __restrict__ mask,
                                                       double* __restrict__ wsum) {
@@ -1749,9 +1772,9 @@ __global__ __launch_bounds__(256) void k_detector_cut(const float4* __restrict__
   for (int d = threadIdx.x; d <= D.n; d += blockDim.x) s_w[d] = 0.0;
   __syncthreads();
   const int lane = threadIdx.x & 63;
-  double acc[kRegPlanes + 1];
+  double acc[REG + 1];
 #pragma unroll
-  for (int d = 0; d <= kRegPlanes; ++d) acc[d] = 0.0;
+  for (int d = 0; d <= REG; ++d) acc[d] = 0.0;
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t i0 = (int64_t)blockIdx.x * blockDim.x; i0 < n; i0 += stride) {
     const int64_t i = i0 + threadIdx.x;
@@ -1770,16 +1793,16 @@ __global__ __launch_bounds__(256) void k_detector_cut(const float4* __restrict__
       pz = (double)pi.w;
     }
     uint64_t bits = 0;
-    if (REG) {
+    if (REG > 0) {
 #pragma unroll
-      for (int d = 0; d < kRegPlanes; ++d) {
+      for (int d = 0; d < REG; ++d) {
         if (d < D.n) {
           const bool pass = inwin && plane_pass(D, d, x0, y0, z0, px, py, pz);
           bits |= (uint64_t)pass << d;
           acc[d] += pass ? w : 0.0;
         }
       }
-      acc[kRegPlanes] += inwin ? w : 0.0;
+      acc[REG] += inwin ? w : 0.0;
     } else {
       for (int d = 0; d < D.n; ++d) {
         const bool pass = inwin && plane_pass(D, d, x0, y0, z0, px, py, pz);
@@ -1792,11 +1815,11 @@ __global__ __launch_bounds__(256) void k_detector_cut(const float4* __restrict__
     }
     if (mask && i < n) mask[i] = bits;
   }
-  if (REG) {
+  if (REG > 0) {
 #pragma unroll
-    for (int d = 0; d <= kRegPlanes; ++d) {
-      const int slot = d == kRegPlanes ? D.n : d;
-      if (d < D.n || d == kRegPlanes) {
+    for (int d = 0; d <= REG; ++d) {
+      const int slot = d == REG ? D.n : d;
+      if (d < D.n || d == REG) {
         const double v = wave_sum_f64(acc[d]);
         if (lane == 0 && v != 0.0) atomicAdd(&s_w[slot], v);
       }
@@ -3645,20 +3668,21 @@ int petite_detector_cut(const float* p, const float* r, int64_t n, const double*
   DetectorPlanes D{};
   D.n = n_det;
   D.has_ecut = has_ecut ? 1 : 0;
-  D.radius = radius;
-  D.inner = inner_radius;
+  radius_square_limits(radius, inner_radius, D.s_out, D.s_in);
   D.emin = emin;
   D.emax = emax;
   for (int d = 0; d < n_det; ++d) D.z[d] = det_z[d];
   if (wsum) HIP_TRY(hipMemsetAsync(wsum, 0, (size_t)(n_det + 1) * sizeof(double), s));
   if (n > 0) {
-    const int64_t blocks = std::min<int64_t>((n + 255) / 256, 4096);
-    if (n_det <= kRegPlanes)
-      hipLaunchKernelGGL(k_detector_cut<true>, dim3((unsigned)blocks), dim3(256), 0, s, (const float4*)p,
-                         (const float4*)r, n, D, mask, wsum);
-    else
-      hipLaunchKernelGGL(k_detector_cut<false>, dim3((unsigned)blocks), dim3(256), 0, s, (const float4*)p,
-                         (const float4*)r, n, D, mask, wsum);
+    // Eight records a thread where that leaves 256 blocks, at most 1,024
+    // blocks: their sums are added one after another, planes + 1 atomics each
+    // (1e6 records at 12 planes 53, 56, 69 and 93 us a call with 512 to 4,096
+    // blocks; 3e7 at 3 planes 308, 253, 275 and 273).
+    const int64_t blocks =
+        std::min<int64_t>(std::min<int64_t>((n + 255) / 256, 1024), std::max<int64_t>(256, (n + 2047) / 2048));
+    auto* const f = n_det <= kRegPlanes[0] ? k_detector_cut<kRegPlanes[0]>
+                                           : (n_det <= kRegPlanes[1] ? k_detector_cut<kRegPlanes[1]> : k_detector_cut<0>);
+    hipLaunchKernelGGL(f, dim3((unsigned)blocks), dim3(256), 0, s, (const float4*)p, (const float4*)r, n, D, mask, wsum);
     HIP_TRY(hipGetLastError());
   }
   return PETITE_OK;
