@@ -186,8 +186,9 @@ __device__ inline bool drate_energy(const PetiteDarkDesc& D, const double* b, in
 // A block's share of a counter: thread-wise `want`, the thread's slot returned
 // (meaningless where !want), one atomic per block.  Per wave, the two counters'
 // atomics of 1.4e6 records x 3 processes, served one after another, held the
-// selection at 0.80 ms (0.33 ms with one per block).  Every thread of a
-// block of 256 calls it; two calls in a row use different LDS.
+// selection at 0.80 ms (0.33 ms with one per block; blocks of 1,024 threads
+// spill and gain nothing).  Every thread of a block of 256 calls it; two calls
+// in a row use different LDS.
 template <typename C>
 __device__ inline C block_slot(bool want, C* counter) {
   __shared__ unsigned int s_n[4];
@@ -381,10 +382,10 @@ __global__ __launch_bounds__(256) void k_dark_emit(DevTables T, PetiteDarkDesc D
                                                    const float* x_res, const int32_t* trials_res, EmitOut O,
                                                    int64_t out_base, uint64_t seed, double* yield,
                                                    unsigned long long* stats) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   double wsum[4] = {0.0, 0.0, 0.0, 0.0};
   unsigned long long n_vec = 0, n_pe_fail = 0;
-  if (e < n_e) {
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n_e; e += stride) {
     const int flag = Q.flag[e];
     const int code = flag & 0xFF;
     const int state = flag >> 8;
@@ -446,7 +447,8 @@ __global__ __launch_bounds__(256) void k_dark_emit(DevTables T, PetiteDarkDesc D
       const float4 rf = S.rf[slot];
       rv = make_float4(rf.x, rf.y, rf.z, (float)w);
       ++n_vec;
-      wsum[code - DARKBREM] = w;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) wsum[k] += code - DARKBREM == k ? w : 0.0;
     }
     const int64_t o = out_base + e;
     O.p[o] = pv;
@@ -455,7 +457,7 @@ __global__ __launch_bounds__(256) void k_dark_emit(DevTables T, PetiteDarkDesc D
     O.meta[o] = code | (ok ? 0x100 : 0);
   }
   // the yields and counts: one atomic per block and process (per wave they took
-  // five sixths of the kernel: 0.42 ms, now 0.07, for 1.1e6 entries)
+  // five sixths of the kernel: 0.42 ms, now 0.06, for 1.1e6 entries)
   __shared__ double s_y[4][4];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   for (int k = 0; k < 4; ++k) {

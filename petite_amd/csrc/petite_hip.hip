@@ -3217,7 +3217,8 @@ int petite_dark_reweight(PetiteCtx* c, const PetiteStore* sm, int64_t n_sm, uint
       if (c->timing) HIP_TRY(hipEventRecord(c->ev[3], s));
       if (n_e > 0) {
         dark::EmitOut O{(float4*)out->p, (float4*)out->r, out->parent, out->meta};
-        hipLaunchKernelGGL(dark::k_dark_emit, dim3((unsigned)((n_e + 255) / 256)), dim3(256), 0, s, c->dev, c->dark, S,
+        hipLaunchKernelGGL(dark::k_dark_emit, dim3((unsigned)std::min<int64_t>((n_e + 255) / 256, (int64_t)c->n_cu * 8)),
+                           dim3(256), 0, s, c->dev, c->dark, S,
                            c->ent, (int64_t)n_e, (const float*)c->dres_x, (const int32_t*)c->dres_trials, O, out_base,
                            seed, c->dyield, ctr + C_DARK_STATS);
         HIP_TRY(hipGetLastError());

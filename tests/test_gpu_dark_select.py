@@ -31,7 +31,7 @@ def _entries(ds, store, n):
 
 
 # less than a wave, than a block; a block; one and four blocks and a particle
-@pytest.mark.parametrize("n", [1, 63, 64, 65, 255, 256, 257, 1025, -1])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 255, 256, 257, 1023, 1024, 1025, -1])
 def test_entries_of_the_first_records(record, n):
     ds, store, total = record
     n = total if n < 0 else n
