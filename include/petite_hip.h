@@ -118,9 +118,9 @@ typedef struct {
   int64_t n_viol_proc[PETITE_NPROC];   /* accepted draws with J*f above max_F per process code (the
                                         * accept probability min(1, J*f / max_F) clips them, as the
                                         * reference's test does) */
-  double ms_tail;          /* depth-first walk time (HIP events, with timing enabled) */
-  int64_t launches_tail;   /* depth-first walk launches */
-  int64_t n_steps_tail;    /* the particle-steps of n_steps taken in depth-first walks */
+  double ms_tail;          /* walk time (HIP events, with timing enabled) */
+  int64_t launches_tail;   /* walk launches */
+  int64_t n_steps_tail;    /* the particle-steps of n_steps taken in walks */
 } PetiteStats;
 
 /* Create a context: copies the table blobs (host pointers) to the device. */

@@ -61,7 +61,7 @@ enum CounterIdx {
   C_LONG = 25,                // draws handed to k_draw_long
   C_YIELD_OUT = 26,           // particles the current sweep's transport handed on to the next sweep
   C_RPARITY = 27,             // which half of the resume buffer the current sweep reads
-  C_TAIL_STEPS = 30,          // particle-steps taken in depth-first walks
+  C_TAIL_STEPS = 30,          // particle-steps taken in walks
   C_STATS = 32,               // [ST_N] run statistics
   C_PTRIALS = 64,             // [PETITE_NPROC] candidates per process
   C_PDRAWS = 80,              // [PETITE_NPROC] draws per process
@@ -1886,7 +1886,7 @@ struct PetiteCtx {
   int64_t* drange = nullptr;
   ResumeRec* dresume = nullptr;  // [2][resume_cap]
   int64_t resume_cap = 0;
-  int32_t* tail_spill = nullptr;  // [2][tail_spill_cap]: depth-first walk spill lists
+  int32_t* tail_spill = nullptr;  // [2][tail_spill_cap]: walk spill lists, each as large as the store
   int64_t tail_spill_cap = 0;
   LongDraw* longs = nullptr;      // [kLongCap], contexts with a DarkAnn map
   std::vector<hipEvent_t> tev;
@@ -2676,8 +2676,8 @@ int petite_run_showers(PetiteCtx* c, const PetitePrimary* prim, int64_t n, uint6
   // a host check, the primaries included, then launched until no spill is
   // left.  Small batches are all walk: every sweep costs 0.3-0.4 ms whatever it
   // holds, and a run needs one per generation (measured, sweeps first / walk
-  // only: 1,000 x 10 GeV graphite 14.7 / 6.6 ms, 10,000 primaries of 0.1-100 GeV
-  // in lead 61 / 27 ms)
+  // only: 1,000 x 10 GeV graphite 14.7 / 5.5 ms, 40,000 primaries of 0.1-100 GeV
+  // in lead 94 / 73 ms)
   bool tail = n < (int64_t)tn.tail_sweep;
   int tpar = 0;  // spill list the next walk reads
   int64_t tail_launches = 0;

@@ -30,8 +30,8 @@
 // What bounds it: the latency of a substep (~600 dependent instructions) and of
 // a draw phase, at 2 waves per SIMD; with muons the longest of them (32,000
 // substeps and 2,400 phases, 70 ms alone).  1,000 electrons of 10 GeV in
-// graphite 5.5 ms a run, 40,000 mixed primaries in lead 76 ms.  A 400 GeV beam
-// of 2,000 in lead, half of them muons: 88 ms; 137 ms with each muon among the
+// graphite 5.4 ms a run, 40,000 mixed primaries in lead 73 ms.  A 400 GeV beam
+// of 2,000 in lead, half of them muons: 84 ms; 137 ms with each muon among the
 // particles of its own subtree; 264 ms (170 ms of that in the walk) with one
 // particle per wave, every lane computing the same transport, and two atomics
 // per draw on one line of per-process counters.
