@@ -2682,7 +2682,14 @@ int petite_run_showers(PetiteCtx* c, const PetitePrimary* prim, int64_t n, uint6
   int tpar = 0;  // spill list the next walk reads
   int64_t tail_launches = 0;
   double t_tail = 0.0;
-  const unsigned tail_blocks = blocks_for(c, tn.tail_waves);
+  // Three waves per SIMD instead of two where the walk is long enough to be
+  // bound by its instructions rather than by its longest chain (ms with two /
+  // three; a store has room for about 1.7 times the records of lead, 4 times
+  // graphite's): lead, 10,000 mixed primaries (36e6 places) 22.3 / 23.6, 20,000
+  // 40 / 38, 40,000 73 / 69, 60,000 106 / 92; 8.5e6 records of graphite (34e6)
+  // 8.2 / 8.2; with muons 72 / 80
+  const bool wide = tail && !muons && store->capacity >= ((int64_t)1 << 26);
+  const unsigned tail_blocks = blocks_for(c, wide ? tn.tail_waves * 3 / 2 : tn.tail_waves);
   if (c->timing) {
     while ((int)c->tev.size() < 4 * group + 2 * kTailGroup) {
       hipEvent_t e;
@@ -2757,7 +2764,8 @@ int petite_run_showers(PetiteCtx* c, const PetitePrimary* prim, int64_t n, uint6
         if (c->timing) HIP_TRY(hipEventRecord(c->tev[4 * group + 2 * g], s));
         const TailParams tp{c->tail_spill, c->tail_spill_cap, tpar, tn.tail_depth,
                             tail_limit(tn.tail_budget, tail_launches)};
-        hipLaunchKernelGGL(k_tail, dim3(tail_blocks), dim3(256), lds, s, c->dev, S, seed, shower_energy, ctr,
+        hipLaunchKernelGGL(wide ? k_tail<3> : k_tail<2>, dim3(tail_blocks), dim3(256), lds, s, c->dev, S, seed,
+                           shower_energy, ctr,
                            c->dsig_lds, (const int64_t*)c->drange, ResumeBuf{c->dresume, rcap}, tp);
         HIP_TRY(hipGetLastError());
         if (c->timing) HIP_TRY(hipEventRecord(c->tev[4 * group + 2 * g + 1], s));

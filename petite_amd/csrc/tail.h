@@ -165,10 +165,13 @@ __device__ inline void walk_draws(const DevTables& T, uint64_t seed, bool mine, 
 // sweep handed on (live state in its resume records), the store slots
 // [first, first + n), then the previous launch's spills.  range: the tail
 // setup's {first, n, end, nres}.
+// EU: waves per SIMD the registers are held to (168 of them and 25 spills for
+// three; the run chooses).
 constexpr int kWalkWaves = 4;  // waves per block
-__global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu(2))) void k_tail(DevTables T, DevStore S, uint64_t seed, double* shower_energy,
-                                                          unsigned long long* counters, const double* sig_lds_src,
-                                                          const int64_t* range, ResumeBuf RB, TailParams TPm) {
+template <int EU>
+__global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu(EU))) void k_tail(
+    DevTables T, DevStore S, uint64_t seed, double* shower_energy, unsigned long long* counters,
+    const double* sig_lds_src, const int64_t* range, ResumeBuf RB, TailParams TPm) {
   const int64_t first = range[0], n = range[1];
   const int64_t nres = RB.rec ? range[3] : 0;
   const ResumeRec* rin = RB.rec ? RB.rec + (int64_t)(counters[C_RPARITY] & 1ull) * RB.cap : nullptr;

@@ -27,12 +27,12 @@ def _primaries(n, e_lo, e_hi, pids, seed):
     return prim
 
 
-def _run(sh, prim, tuning):
+def _run(sh, prim, tuning, capacity=None):
     ctx = sh.device_context()
     base = ctx.get_tuning()
     ctx.set_tuning(dict(base, **tuning))
     try:
-        b = sh.generate_showers(prim, seed=9)
+        b = sh.generate_showers(prim, seed=9, capacity=capacity)
     finally:
         ctx.set_tuning(base)
     a = b.to_numpy()
@@ -93,6 +93,20 @@ def test_muons_walk_apart(lead, batch):
         got, e, s = _run(lead, prim, dict(tuning, tail_waves=1))
         for k in ref:
             # the bits: a muon below its rest mass has no momentum
+            assert ref[k].tobytes() == got[k].tobytes(), (batch, name, k)
+        assert np.allclose(energy, e, rtol=1e-12, atol=1e-12), (batch, name)
+        for k in ("n_particles", "n_steps", "n_draws", "n_trials", "n_dropped", "n_maxf_viol"):
+            assert st[k] == s[k], (batch, name, k)
+
+
+# a store with room for 2^26 records: the walk that is held to three waves' registers
+@pytest.mark.parametrize("batch", ["one", "wave", "many", "low"])
+def test_walk_of_a_large_store(lead, batch):
+    prim = _primaries(*BATCHES[batch], seed=8)
+    ref, energy, st = _run(lead, prim, {"tail_sweep": 1})
+    for name in ("start", "smallest"):
+        got, e, s = _run(lead, prim, WALKS[name], capacity=1 << 26)
+        for k in ref:
             assert ref[k].tobytes() == got[k].tobytes(), (batch, name, k)
         assert np.allclose(energy, e, rtol=1e-12, atol=1e-12), (batch, name)
         for k in ("n_particles", "n_steps", "n_draws", "n_trials", "n_dropped", "n_maxf_viol"):
