@@ -303,7 +303,7 @@ def main():
     totals = {"steps": 0, "particles": 0, "draws": 0, "trials": 0, "tail_steps": 0}
     # stage times from HIP events on the run's stream: the transport kernel,
     # the draws with their emissions (per-process streams, fork to join), and
-    # the depth-first walk of the last particles
+    # the walk (of the last particles, or of the whole batch)
     kern = {"transport": [0.0, 0], "draw_emit": [0.0, 0], "tail": [0.0, 0]}
     t0 = time.perf_counter()
     for k in range(args.steps):
@@ -330,17 +330,19 @@ def main():
     steps_per_s = totals["steps"] / dt
     showers_per_s = K * len(prim) / dt
 
-    # roofline of the dominant kernel, k_transport (the largest single kernel in
-    # the rocprofv3 summary; the draw kernels of the six processes run side by side)
-    t_dom = kern["transport"][0] / 1e3
-    alg = B_STEP * (totals["steps"] - totals["tail_steps"])  # the steps k_transport took
+    # roofline of the kernel that advances the particles: k_transport, or the
+    # walk where it takes the batch whole (the draw kernels of the six
+    # processes run side by side; a walk draws and emits as well)
+    dom, dom_kernel = ("transport", "k_transport") if kern["transport"][1] else ("tail", "k_tail")
+    t_dom = kern[dom][0] / 1e3
+    alg = B_STEP * (totals["tail_steps"] if dom == "tail" else totals["steps"] - totals["tail_steps"])
     ach = alg / t_dom / 1e9
     roof = {"bound": "hbm", "achieved": ach, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": ach / HBM_PEAK_GBS,
-            "traffic": None, "kernel": "k_transport", "per_unit": "128 B per particle-step"}
-    roof["avg_launch_ms"] = kern["transport"][0] / max(kern["transport"][1], 1)
-    roof["traffic"] = measured_traffic(roof["kernel"], alg / max(kern["transport"][1], 1))
-    # the bound that holds: k_transport is VALU-issue bound (its HBM traffic is
-    # a fifth of the algorithmic bytes: a particle stays in registers)
+            "traffic": None, "kernel": dom_kernel, "per_unit": "128 B per particle-step"}
+    roof["avg_launch_ms"] = kern[dom][0] / max(kern[dom][1], 1)
+    roof["traffic"] = measured_traffic(roof["kernel"], alg / max(kern[dom][1], 1))
+    # the bound that holds is VALU issue (HBM traffic is a fifth of the
+    # algorithmic bytes: a particle stays in registers)
     roof["valu"] = measured_valu(roof["kernel"])
     kernels = {k: {"ms_total": v[0] / K, "launches": v[1] // K} for k, v in kern.items()}
 

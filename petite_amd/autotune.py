@@ -44,7 +44,7 @@ SPACE = {
     "small_sweep": [1, 4096, 16384, 65536, 262144],
     "small_yield_steps": [24, 32, 40, 160, 1 << 30],
     "graph": [1, 2],
-    "tail_sweep": [1, 1024, 4096, 16384, 65536],
+    "tail_sweep": [1, 1024, 4096, 16384, 65536, 262144],
     "tail_waves": [4, 8, 16],
     "tail_budget": [8, 16, 64, 1 << 30],
 }
