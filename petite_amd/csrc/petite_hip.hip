@@ -232,7 +232,7 @@ __device__ inline double integrand_p(const DevTables& T, double E, const double*
   if (P == MUONE) return f_muone(E, T.Ee_min, x[0]);
   if (P == DARKBREM) return f_dark_brem(E, kMe, T.mV, T.mT, T.Z, T.A, x);
   if (P == DARKMUONBREM) return f_dark_brem(E, kMmu, T.mV, T.mT, T.Z, T.A, x);
-  if (P == DARKANN) return (double)f_dark_ann_f32(E, T.mV, x[0]);
+  if (P == DARKANN) return (double)f_dark_ann_f32(E, T.mV, x[0], T.ann_c);
   if (P == DARKCOMP) return f_compton(E, T.mV, x[0]);
   return 0.0;
 }
@@ -2260,6 +2260,7 @@ int petite_ctx_create(const PetiteTableDesc* desc, const double* blob64, int64_t
   for (int i = 0; i < 5; ++i) T.min_calc[i] = desc->min_calc[i];
   T.rescale_MCS = desc->rescale_MCS;
   T.MS = desc->MS;
+  T.ann_c = desc->mV > 2.0 * kMe ? (float)ann_prefactor(desc->mV) : 0.0f;  // (draw_possible)
   T.max_trials = (uint32_t)std::min<int64_t>(std::max<int64_t>(desc->max_trials, 1), 0x7FFFFFF0);
   const double Z = desc->Z;
   const double a0 = 184.15 * pow(2.718, -0.5) * pow(Z, -1.0 / 3.0) / kMe;

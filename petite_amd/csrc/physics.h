@@ -50,6 +50,7 @@ struct DevTables {
   double rescale_MCS;
   int32_t MS;
   uint32_t max_trials; // 1 .. 0x7FFFFFF0
+  float ann_c;         // f_dark_ann_f32's factor of m_V alone, formed in float64 (ann_prefactor)
   const PetiteTableDesc* d;  // device copy of the descriptor: its grids and tables
 };
 
@@ -500,11 +501,17 @@ __device__ __noinline__ double f_dark_ann_ref(double Ee, double mV, double u0) {
 // With L = (2/beta) ln u0, Q = e^L, y = m_V^2/s and d = 1 - y the powers of umax
 // drop out: 1 - x1 = d Q, x1 = y + d (1 - Q) and 1 - x2 = d (1 - Q) / x1, which
 // float32 holds without cancellation; the powers are hardware logarithms and
-// exponentials (base 2).  Its error against the float64 formula stays below
-// 5e-5 (m_V 1.2 MeV to 0.3 GeV, E to 400 GeV), and it takes about 90
+// exponentials (base 2).  beta_f^2 = 1 - 4 m_e^2 / m_V^2 does cancel just above
+// m_V = 2 m_e (in float32 0.7 % of J f is lost at 1.022 MeV, 10 % at 1.021998):
+// it comes in `c`, formed in float64 once per context.  It takes about 90
 // instructions against 1,500.
 __device__ inline float log1p_f32(float y);
-__device__ inline float f_dark_ann_f32(double Ee, double mV, double u0) {
+// (4 pi^2 alpha / 64) beta_f (3 - beta_f^2) / 2, beta_f as f_dark_ann forms it.
+__host__ inline double ann_prefactor(double mV) {
+  const double betaf = sqrt(1.0 - 4.0 * kMe * kMe / (mV * mV));
+  return 4.0 * kPi * kPi * kAlpha / 64.0 * betaf * (1.5 - betaf * betaf / 2.0);
+}
+__device__ inline float f_dark_ann_f32(double Ee, double mV, double u0, float c) {
   const double s = 2.0 * kMe * (Ee + kMe);
   const double y = mV * mV / s;
   const float d = (float)(1.0 - y);
@@ -528,9 +535,6 @@ __device__ inline float f_dark_ann_f32(double Ee, double mV, double u0) {
   const float k = 8.0f + 3.0f * beta;
   const float a = k * __builtin_amdgcn_exp2f((hb - 1.0f) * __log2f(t)) - 4.0f * (2.0f - t);
   const float b = k - 4.0f * (1.0f + xx) * __builtin_amdgcn_exp2f((1.0f - hb) * __log2f(q));
-  const float r = (float)(kMe / mV);
-  const float bf2 = 1.0f - 4.0f * r * r;
-  const float c = (float)(4.0 * kPi * kPi * kAlpha / 64.0) * sqrtf(bf2) * (1.5f - 0.5f * bf2);
   return c * __builtin_amdgcn_rcpf((float)s) * umax * beta * a * b * rx;
 }
 
