@@ -265,7 +265,7 @@ __device__ inline double integrand_ref(const DevTables& T, double E, const doubl
 // Relative band around the accept threshold max_F * u in which a float32
 // J*f of a 4-D process or of DarkAnn is re-evaluated in float64: the float32
 // bodies agree with the float64 reference formula to 5e-6 (99th percentile) and
-// 2e-5 (99.9th; DarkAnn 5e-5 at most), so outside the band the two make the
+// 2e-5 (99.9th; DarkAnn 7e-6 at most), so outside the band the two make the
 // same decision.
 constexpr double kRefBand = 4.0e-4;
 

@@ -497,7 +497,11 @@ __device__ __noinline__ double f_dark_ann_ref(double Ee, double mV, double u0) {
 
 // The same integrand in float32 for the draws, which take it for a candidate
 // well away from the accept threshold and f_dark_ann near it; NaN where
-// float64 rounding decides (u0 within 1e-7 of 1) or for u0 <= 0.
+// float64 rounding decides (u0 within 1e-7 of 1, or x1 - y below 1e-10: s
+// within that of m_V^2, where f_dark_ann is 0 or off by its whole value) or for
+// u0 <= 0.  Elsewhere the two agree to 7e-6 (this body restated in numpy with
+// an ulp of error in each hardware function, 4e6 points, m_V from 2 m_e to
+// 1 GeV, E from the threshold to 5 TeV).
 // With L = (2/beta) ln u0, Q = e^L, y = m_V^2/s and d = 1 - y the powers of umax
 // drop out: 1 - x1 = d Q, x1 = y + d (1 - Q) and 1 - x2 = d (1 - Q) / x1, which
 // float32 holds without cancellation; the powers are hardware logarithms and
@@ -526,11 +530,12 @@ __device__ inline float f_dark_ann_f32(double Ee, double mV, double u0, float c)
   const float L = L2 * 0.693147181f;
   const float om = L > -0.1f ? -L * (1.0f + L * (0.5f + L * (1.0f / 6.0f + L * (1.0f / 24.0f + L * (1.0f / 120.0f)))))
                              : 1.0f - Q;  // 1 - Q
-  if (!(om > 1.0e-6f && uf > 0.0f)) return __builtin_nanf("");
+  const float dm = d * om;              // x1 - y
+  if (!(om > 1.0e-6f && dm > 1.0e-10f && uf > 0.0f)) return __builtin_nanf("");
   const float q = d * Q;                // 1 - x1
-  const float xx = (float)y + d * om;   // x1
+  const float xx = (float)y + dm;       // x1
   const float rx = __builtin_amdgcn_rcpf(xx);
-  const float t = d * om * rx;          // 1 - x2
+  const float t = dm * rx;              // 1 - x2
   const float umax = __builtin_amdgcn_exp2f(hb * __log2f(d));
   const float k = 8.0f + 3.0f * beta;
   const float a = k * __builtin_amdgcn_exp2f((hb - 1.0f) * __log2f(t)) - 4.0f * (2.0f - t);
