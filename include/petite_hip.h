@@ -168,7 +168,8 @@ typedef struct {
                               * the next launch [128] */
   int32_t tail_budget;       /* walk: particles per lane after which a wave leaves the rest of its stack
                               * to the next launch, in the first launch; twice as many in each later one
-                              * [16]; a value above 2^30 never leaves it */
+                              * [16], and in launches with muons at most 2,048 substeps and phases of a
+                              * wave with some, 512 of the others; a value above 2^30 never leaves it */
 } PetiteTuning;
 
 /* Set (tuning != NULL) or reset to the defaults (NULL) the context's launch

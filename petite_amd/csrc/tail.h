@@ -24,8 +24,9 @@
 // A muon's vertices follow one another, 13 substeps and a draw phase each, and
 // the longest muon sets the run's length.  A wave with muons therefore keeps to
 // them: their other children go straight to the spill list, muons of a list go
-// to its back, and every second wave of a launch takes its share of those
-// first, alone in its wave while there are enough waves.
+// to its back, and an empty wave takes from there first: an even share of
+// every second wave of the launch, so that the other half of them take the
+// list's front; alone in its wave while there are fewer muons than that.
 //
 // What bounds it: the latency of a substep (~600 dependent instructions) and of
 // a draw phase, at 2 waves per SIMD; with muons the longest of them (32,000
@@ -41,9 +42,10 @@ constexpr int kTailMaxDepth = 128;  // stack entries per wave
 constexpr int kTailGroup = 4;       // walk launches queued per host check after the first
 constexpr int kTailStepsPerParticle = 8;  // iterations of a wave per particle of its lanes' budget
 constexpr int kTailPhaseSteps = 4;        // iterations a draw phase counts for
-// A launch with muons: at most kMuonIters iterations of a wave that holds some,
-// and a quarter of that of the others, whose iterations (64 lanes instead of a
-// few) take about three times as long.
+// Iterations after which a wave that holds muons starts no more particles, and,
+// in a launch with muons on its list, a quarter of that for the others, whose
+// iterations (64 lanes instead of a few) take about three times as long: caps
+// on the budget's limit, but for a budget that never stops a wave.
 constexpr int kMuonIters = 2048;
 
 struct TailParams {
@@ -180,13 +182,16 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
   const int32_t* const spill_in = TPm.spill + TPm.par * TPm.cap;
   const int64_t total = nres + n + min((int64_t)counters[C_SPILL + TPm.par], TPm.cap);
   const int64_t n_mu = min((int64_t)counters[C_MUSPILL + TPm.par], TPm.cap);
-  // items per claim: an even share of every wave of the launch (of every second
-  // one for muons), at most a lane's each
+  // items per claim: an even share of every wave of the launch (of half of them
+  // for muons), at most a lane's each
   const int64_t waves = (int64_t)gridDim.x * kWalkWaves;
   const int share = (int)min((int64_t)64, max((int64_t)1, (total + waves - 1) / waves));
   const int share_mu = (int)min((int64_t)64, max((int64_t)1, (2 * n_mu + waves - 1) / waves));
   if ((int64_t)blockIdx.x * kWalkWaves >= (total + share - 1) / share + (n_mu + share_mu - 1) / share_mu) return;
-  const int limit_mu = min(TPm.limit, kMuonIters), limit = n_mu > 0 ? min(TPm.limit, kMuonIters / 4) : TPm.limit;
+  // INT32_MAX: no wave stops (tail_limit), one with muons as little as the others
+  const bool capped = TPm.limit != INT32_MAX;
+  const int limit_mu = capped ? min(TPm.limit, kMuonIters) : TPm.limit;
+  const int limit = capped && n_mu > 0 ? min(TPm.limit, kMuonIters / 4) : TPm.limit;
   HIP_DYNAMIC_SHARED(double, s_sig)
   __shared__ WalkLds s_walk[kWalkWaves];
   __shared__ WalkStats s_stat;
@@ -596,7 +601,8 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
 // lane in the first, twice as many in each later one, so that particles are
 // spread often while their number grows and seldom once a few long chains
 // remain (a spread costs a launch, and leaves a chain among other particles);
-// budgets above 2^30 never stop a wave.
+// budgets above 2^30 never stop a wave.  (kMuonIters caps the others' limits in
+// launches with muons.)
 static int32_t tail_limit(int32_t budget, int64_t i) {
   if (budget > (1 << 30)) return INT32_MAX;
   return (int32_t)std::min<int64_t>((int64_t)std::max(budget, 1) * kTailStepsPerParticle << std::min<int64_t>(i, 20),
