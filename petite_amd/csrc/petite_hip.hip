@@ -68,6 +68,8 @@ enum CounterIdx {
   C_PVIOL = 96,               // [PETITE_NPROC] accepted draws above max_F per process
   C_REFILL = 112,             // [PETITE_NPROC] per-process draw refill counters, kCtrLine apart
   C_SPILL = C_REFILL + kCtrLine * PETITE_NPROC,  // [2] walk: entries at the front of each spill list
+  C_MARKED = C_SPILL + 2,                        // particles past a list's end, marked in the store
+  C_GATHER = C_SPILL + 3,                        // of them, before the current launch lists any
   C_MUSPILL = C_SPILL + kCtrLine,                // [2] and muons at its back
   C_MUCLAIM = C_MUSPILL + kCtrLine,              // claims of the latter
   C_N = C_MUCLAIM + kCtrLine
@@ -1886,7 +1888,7 @@ struct PetiteCtx {
   int64_t* drange = nullptr;
   ResumeRec* dresume = nullptr;  // [2][resume_cap]
   int64_t resume_cap = 0;
-  int32_t* tail_spill = nullptr;  // [2][tail_spill_cap]: walk spill lists, each as large as the store
+  int32_t* tail_spill = nullptr;  // [2][tail_spill_cap]: walk spill lists (at most 32 MB)
   int64_t tail_spill_cap = 0;
   LongDraw* longs = nullptr;      // [kLongCap], contexts with a DarkAnn map
   std::vector<hipEvent_t> tev;
@@ -2749,22 +2751,28 @@ int petite_run_showers(PetiteCtx* c, const PetitePrimary* prim, int64_t n, uint6
   }
   while (true) {
     if (tail) {
-      if (c->tail_spill_cap < store->capacity) {
+      // (a muon's vertex leaves one muon: there are never more than primaries)
+      const int64_t front = std::min(store->capacity, kListFront), back = std::min((int64_t)n_muons, kListMuons);
+      const bool may_mark = front < store->capacity || back < (int64_t)n_muons;
+      if (c->tail_spill_cap < front + back) {
         if (c->tail_spill) HIP_TRY(hipFree(c->tail_spill));
         c->tail_spill = nullptr;
         c->tail_spill_cap = 0;
-        HIP_TRY(hipMalloc(&c->tail_spill, 2 * store->capacity * sizeof(int32_t)));
-        c->tail_spill_cap = store->capacity;
+        HIP_TRY(hipMalloc(&c->tail_spill, 2 * (front + back) * sizeof(int32_t)));
+        c->tail_spill_cap = front + back;
       }
       // the first walk alone (it often leaves no spill), then kTailGroup per
       // host check: a launch whose inputs are empty ends at once
       const int ng = tail_launches == 0 ? 1 : kTailGroup;
       for (int g = 0; g < ng; ++g) {
-        hipLaunchKernelGGL(k_tail_setup, dim3(1), dim3(64), 0, s, ctr, c->drange, store->capacity, rcap, tpar);
+        const TailParams tp{c->tail_spill, front, back, tpar, tn.tail_depth, tail_limit(tn.tail_budget, tail_launches)};
+        hipLaunchKernelGGL(k_tail_setup, dim3(1), dim3(64), 0, s, ctr, c->drange, store->capacity, rcap, tp);
         HIP_TRY(hipGetLastError());
         if (c->timing) HIP_TRY(hipEventRecord(c->tev[4 * group + 2 * g], s));
-        const TailParams tp{c->tail_spill, c->tail_spill_cap, tpar, tn.tail_depth,
-                            tail_limit(tn.tail_budget, tail_launches)};
+        if (may_mark && tail_launches > 0) {
+          hipLaunchKernelGGL(k_tail_gather, dim3((unsigned)c->n_cu * 4), dim3(256), 0, s, S, ctr, tp);
+          HIP_TRY(hipGetLastError());
+        }
         hipLaunchKernelGGL(wide ? k_tail<3> : k_tail<2>, dim3(tail_blocks), dim3(256), lds, s, c->dev, S, seed,
                            shower_energy, ctr,
                            c->dsig_lds, (const int64_t*)c->drange, ResumeBuf{c->dresume, rcap}, tp);
@@ -2787,7 +2795,10 @@ int petite_run_showers(PetiteCtx* c, const PetitePrimary* prim, int64_t n, uint6
         }
       }
       if ((int64_t)h_store > store->capacity) break;
-      if (h_spill[tpar] == 0 && h_spill[kCtrLine + tpar] == 0) break;  // every particle walked
+      if (h_spill[tpar] == 0 && h_spill[kCtrLine + tpar] == 0) {  // every particle walked
+        if (h_spill[C_MARKED - C_SPILL]) return fail(PETITE_ERR_INTERNAL, "petite_run_showers: unlisted particles left");
+        break;
+      }
       if (tail_launches > 100000) return fail(PETITE_ERR_HIP, "petite_run_showers: tail launch runaway");
       continue;
     }

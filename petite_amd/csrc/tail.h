@@ -17,7 +17,9 @@
 // lower-energy one goes on the wave's stack, from which free lanes take.  A
 // full stack passes children to a spill list, and after its share of
 // iterations a wave starts nothing more and leaves its stack there, so the
-// next launch spreads the particles over all waves again.  Every random number
+// next launch spreads the particles over all waves again.  (Particles past a
+// list's end are marked in the store, and k_tail_gather lists them as lists
+// empty.)  Every random number
 // comes from the particle's own Philox stream, as in the sweeps, so the records
 // are the sweeps' records, bit for bit.
 //
@@ -48,9 +50,15 @@ constexpr int kTailPhaseSteps = 4;        // iterations a draw phase counts for
 // on the budget's limit, but for a budget that never stops a wave.
 constexpr int kMuonIters = 2048;
 
+// Entries of a spill list: kListFront from its front, kListMuons muons from its
+// end (a store with less room needs no more than that).  Lists as large as any
+// store took 8 bytes a place beside it, gigabytes for large batches.
+constexpr int64_t kListFront = 3 << 20, kListMuons = 1 << 20;
+constexpr int32_t kMarked = (int32_t)0x80000000;  // bit of a particle's meta: waits, but is on no list
+
 struct TailParams {
-  int32_t* spill;   // [2][cap]: slots left for the next launch, muons from a list's end
-  int64_t cap;      // the store's capacity: a list holds every particle there is room for
+  int32_t* spill;   // [2][front + muons]: slots left for the next launch, muons from a list's end
+  int64_t front, muons;
   int32_t par;      // list this launch reads (counted at C_SPILL + par, C_MUSPILL + par)
   int32_t depth;    // stack entries per wave (1..kTailMaxDepth)
   int32_t limit;    // iterations after which a wave starts no more particles
@@ -66,12 +74,12 @@ struct WalkLds {
 __device__ inline bool is_muon(int pid) { return pid == 13 || pid == -13; }
 
 // The slots v (>= 0) of the calling lanes at the end of the next launch's list,
-// muons from its back; 1 where there is no room (reported by the run as an
-// internal error).
-__device__ __noinline__ int walk_hand_on(int32_t* list, int64_t cap, unsigned long long* count, int32_t v, bool muon) {
+// muons from its back; those there is no room for are marked in the store (1).
+__device__ __noinline__ int walk_hand_on(int32_t* list, int64_t front, int64_t muons, unsigned long long* count,
+                                         int32_t* meta, int32_t v, bool muon) {
   const int lane = threadIdx.x & 63;
   const unsigned long long below = (1ull << lane) - 1ull;
-  int lost = 0;
+  int marked = 0;
   for (int m = 0; m < 2; ++m) {
     const bool mine = v >= 0 && muon == (m == 1);
     const unsigned long long om = __ballot(mine);
@@ -80,11 +88,15 @@ __device__ __noinline__ int walk_hand_on(int32_t* list, int64_t cap, unsigned lo
     if (lane == 0) o = atomicAdd(count + (m ? C_MUSPILL - C_SPILL : 0), (unsigned long long)__popcll(om));
     o = shfl_u64(o, 0) + (unsigned long long)__popcll(om & below);
     if (mine) {
-      if ((int64_t)o < cap) list[m ? cap - 1 - (int64_t)o : (int64_t)o] = v;
-      else lost = 1;
+      if ((int64_t)o < (m ? muons : front)) {
+        list[m ? front + muons - 1 - (int64_t)o : (int64_t)o] = v;
+      } else {
+        atomicOr(meta + v, kMarked);
+        marked = 1;
+      }
     }
   }
-  return lost;
+  return marked;
 }
 
 // Per-process draw statistics of a block.
@@ -177,11 +189,11 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
   const int64_t first = range[0], n = range[1];
   const int64_t nres = RB.rec ? range[3] : 0;
   const ResumeRec* rin = RB.rec ? RB.rec + (int64_t)(counters[C_RPARITY] & 1ull) * RB.cap : nullptr;
-  // a count past the list (children that did not fit, an internal error the
-  // run reports) is cut to the list
-  const int32_t* const spill_in = TPm.spill + TPm.par * TPm.cap;
-  const int64_t total = nres + n + min((int64_t)counters[C_SPILL + TPm.par], TPm.cap);
-  const int64_t n_mu = min((int64_t)counters[C_MUSPILL + TPm.par], TPm.cap);
+  // a count past the list is cut to the list (the others are marked)
+  const int64_t list_cap = TPm.front + TPm.muons;
+  const int32_t* const spill_in = TPm.spill + TPm.par * list_cap;
+  const int64_t total = nres + n + min((int64_t)counters[C_SPILL + TPm.par], TPm.front);
+  const int64_t n_mu = min((int64_t)counters[C_MUSPILL + TPm.par], TPm.muons);
   // items per claim: an even share of every wave of the launch (of half of them
   // for muons), at most a lane's each
   const int64_t waves = (int64_t)gridDim.x * kWalkWaves;
@@ -220,7 +232,7 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
   float nx = 0.0f, ny = 0.0f, nz = 0.0f, rx = 0.0f, ry = 0.0f, rz = 0.0f, wgt = 0.0f;
   uint32_t k = 0;
   bool closing = false;
-  unsigned int steps = 0, n_fail = 0, n_drop = 0, n_ovf = 0, n_lost = 0;  // of this lane in this launch
+  unsigned int steps = 0, n_fail = 0, n_drop = 0, n_ovf = 0, n_marked = 0;  // of this lane in this launch
   while (true) {
     // past its share the wave starts no more: the next launch spreads what it leaves
     if (muons) muons = __ballot(mode != EMPTY && is_muon(pid)) != 0ull;
@@ -238,7 +250,7 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
         if (lane == 0) c = atomicAdd(counters + C_MUCLAIM, (unsigned long long)share_mu);
         c = shfl_u64(c, 0);
         got = lane < share_mu && (int64_t)c + lane < n_mu;
-        if (got) slot = spill_in[TPm.cap - 1 - ((int64_t)c + lane)];
+        if (got) slot = spill_in[list_cap - 1 - ((int64_t)c + lane)];
         got_mu = (int64_t)c < n_mu;
         mu_exhausted = (int64_t)c + share_mu >= n_mu;
       }
@@ -536,8 +548,8 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
       if (v >= 0 && at < depth) W.stack[at] = v;
       const int32_t out = at >= depth ? v : -1;
       if (__ballot(out >= 0))
-        n_lost += walk_hand_on(TPm.spill + (TPm.par ^ 1) * TPm.cap, TPm.cap, counters + C_SPILL + (TPm.par ^ 1), out,
-                               t == 0 ? hmu : lmu);
+        n_marked += walk_hand_on(TPm.spill + (TPm.par ^ 1) * list_cap, TPm.front, TPm.muons,
+                                 counters + C_SPILL + (TPm.par ^ 1), S.meta, out, t == 0 ? hmu : lmu);
       if (!muons) sp = min(depth, sp + __popcll(pm));
     }
     if (go_on) {
@@ -556,7 +568,7 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
   // ---- what the wave did not start goes to the next launch, and so do the
   // items no wave claimed (a handed-on one starts over there: its random
   // numbers are indexed by its substeps, so it ends the same)
-  int32_t* const spill_out = TPm.spill + (TPm.par ^ 1) * TPm.cap;
+  int32_t* const spill_out = TPm.spill + (TPm.par ^ 1) * list_cap;
   unsigned long long* const n_out = counters + C_SPILL + (TPm.par ^ 1);
   while (!exhausted) {
     unsigned long long c = 0;
@@ -568,7 +580,7 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
     if (rr < total)
       v = rr < nres ? rin[rr].slot
                     : (rr < nres + n ? (int32_t)(first + (rr - nres)) : spill_in[rr - nres - n]);
-    n_lost += walk_hand_on(spill_out, TPm.cap, n_out, v, v >= 0 && is_muon(S.pid[v]));
+    n_marked += walk_hand_on(spill_out, TPm.front, TPm.muons, n_out, S.meta, v, v >= 0 && is_muon(S.pid[v]));
   }
   while (!mu_exhausted) {
     unsigned long long c = 0;
@@ -576,15 +588,15 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
     c = shfl_u64(c, 0);
     mu_exhausted = (int64_t)c + 64 >= n_mu;
     const int64_t rr = (int64_t)c + lane;
-    n_lost += walk_hand_on(spill_out, TPm.cap, n_out, rr < n_mu ? spill_in[TPm.cap - 1 - rr] : -1, true);
+    n_marked += walk_hand_on(spill_out, TPm.front, TPm.muons, n_out, S.meta, rr < n_mu ? spill_in[list_cap - 1 - rr] : -1, true);
   }
   for (int e0 = 0; e0 < sp; e0 += 64)
-    n_lost += walk_hand_on(spill_out, TPm.cap, n_out, e0 + lane < sp ? W.stack[e0 + lane] : -1, false);
+    n_marked += walk_hand_on(spill_out, TPm.front, TPm.muons, n_out, S.meta, e0 + lane < sp ? W.stack[e0 + lane] : -1, false);
   {
     unsigned long long* const st = counters + C_STATS;
-    const unsigned long long v[7] = {steps, steps, n_fail, n_drop, n_ovf, n_lost, 0ull};
+    const unsigned long long v[7] = {steps, steps, n_fail, n_drop, n_ovf, n_marked, 0ull};
     unsigned long long* const dst[7] = {st + ST_STEPS, counters + C_TAIL_STEPS, st + ST_NOSAMPLE, st + ST_DROPPED,
-                                        st + ST_OVERFLOW, st + ST_REQ_OVERFLOW, st};
+                                        st + ST_OVERFLOW, counters + C_MARKED, st};
     block_stat_add<7>(v, dst);
   }
   if (threadIdx.x < 8) {
@@ -612,8 +624,10 @@ static int32_t tail_limit(int32_t budget, int64_t i) {
 // Start of a tail launch: the items are the particles handed on by the last
 // sweep, every store entry appended since the last sweep or tail launch (no
 // bound: the walk files no draw requests), and the previous launch's spills
-// (in the list of parity `par`; the other list is cleared for this launch's).
-__global__ void k_tail_setup(unsigned long long* ctr, int64_t* range, int64_t capacity, int64_t resume_cap, int par) {
+// (in the list of parity `par`, whose counts are cut to it; the other list is
+// cleared for this launch's).
+__global__ void k_tail_setup(unsigned long long* ctr, int64_t* range, int64_t capacity, int64_t resume_cap,
+                             TailParams P) {
   if (threadIdx.x == 0) {
     const int64_t big = (int64_t)1 << 62;
     const SweepRange sr = sweep_range(range[2], (int64_t)ctr[C_STORE], capacity, big, (int64_t)ctr[C_YIELD_OUT],
@@ -625,11 +639,81 @@ __global__ void k_tail_setup(unsigned long long* ctr, int64_t* range, int64_t ca
     ctr[C_YIELD_OUT] = 0ull;
     ctr[C_RPARITY] ^= 1ull;
     ctr[C_TRANSPORT] = 0ull;
-    ctr[C_SPILL + (par ^ 1)] = 0ull;
-    ctr[C_MUSPILL + (par ^ 1)] = 0ull;
+    ctr[C_SPILL + P.par] = min(ctr[C_SPILL + P.par], (unsigned long long)P.front);
+    ctr[C_MUSPILL + P.par] = min(ctr[C_MUSPILL + P.par], (unsigned long long)P.muons);
+    ctr[C_SPILL + (P.par ^ 1)] = 0ull;
+    ctr[C_MUSPILL + (P.par ^ 1)] = 0ull;
     ctr[C_MUCLAIM] = 0ull;
-    if (sr.n > 0 || sr.nres > 0 || ctr[C_SPILL + par] > 0ull || ctr[C_MUSPILL + par] > 0ull) ctr[C_SWEEPS] += 1ull;
+    ctr[C_GATHER] = ctr[C_MARKED];
+    if (sr.n > 0 || sr.nres > 0 || ctr[C_SPILL + P.par] > 0ull || ctr[C_MUSPILL + P.par] > 0ull) ctr[C_SWEEPS] += 1ull;
   }
+}
+
+// The marked particles onto the coming launch's list, as many as it has room
+// for: one atomic per block, list and 4,096 store entries.  A launch that finds
+// none marked ends at once.
+constexpr int kGatherRun = 16;
+__global__ __launch_bounds__(256) void k_tail_gather(DevStore S, unsigned long long* ctr, TailParams P) {
+  if (ctr[C_GATHER] == 0ull) return;
+  __shared__ unsigned int s_n[2][4];
+  __shared__ unsigned long long s_base[2];
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const unsigned long long below = (1ull << lane) - 1ull;
+  const int64_t cap = P.front + P.muons, n = min((int64_t)ctr[C_STORE], S.capacity);
+  int32_t* const list = P.spill + P.par * cap;
+  constexpr int64_t kWaveRun = 64 * kGatherRun, kBlockRun = 4 * kWaveRun;
+  unsigned long long listed = 0ull;
+  for (int64_t b0 = (int64_t)blockIdx.x * kBlockRun; b0 < n; b0 += (int64_t)gridDim.x * kBlockRun) {
+    const int64_t w0 = b0 + wid * kWaveRun;
+    unsigned int c[2] = {0u, 0u};
+    for (int j = 0; j < kGatherRun; ++j) {
+      const int64_t i = w0 + j * 64 + lane;
+      const bool marked = i < n && S.meta[i] < 0;
+      const unsigned long long m = __ballot(marked);
+      if (!m) continue;
+      const unsigned int mu = (unsigned int)__popcll(__ballot(marked && is_muon(S.pid[i])));
+      c[0] += (unsigned int)__popcll(m) - mu;
+      c[1] += mu;
+    }
+    if (lane == 0) {
+      s_n[0][wid] = c[0];
+      s_n[1][wid] = c[1];
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+      const unsigned int t = s_n[threadIdx.x][0] + s_n[threadIdx.x][1] + s_n[threadIdx.x][2] + s_n[threadIdx.x][3];
+      s_base[threadIdx.x] =
+          t ? atomicAdd(ctr + (threadIdx.x ? C_MUSPILL : C_SPILL) + P.par, (unsigned long long)t) : 0ull;
+    }
+    __syncthreads();
+    unsigned long long o[2] = {s_base[0], s_base[1]};
+    for (int w = 0; w < wid; ++w) {
+      o[0] += s_n[0][w];
+      o[1] += s_n[1][w];
+    }
+    for (int j = 0; j < kGatherRun; ++j) {
+      const int64_t i = w0 + j * 64 + lane;
+      const bool marked = i < n && S.meta[i] < 0;
+      if (!__ballot(marked)) continue;
+      const bool muon = marked && is_muon(S.pid[i]);
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const bool mine = marked && muon == (q == 1);
+        const unsigned long long m = __ballot(mine);
+        const int64_t at = (int64_t)(o[q] + __popcll(m & below));
+        if (mine && at < (q ? P.muons : P.front)) {
+          list[q ? cap - 1 - at : at] = (int32_t)i;
+          S.meta[i] &= ~kMarked;
+          ++listed;
+        }
+        o[q] += (unsigned long long)__popcll(m);
+      }
+    }
+    __syncthreads();  // s_n and s_base are read before the next run writes them
+  }
+  const unsigned long long v[1] = {0ull - listed};
+  unsigned long long* const dst[1] = {ctr + C_MARKED};
+  block_stat_add<1>(v, dst);
 }
 
 // After a tail launch: everything it appended was walked or spilled, so the
