@@ -61,6 +61,7 @@ enum CounterIdx {
   C_LONG = 25,                // draws handed to k_draw_long
   C_YIELD_OUT = 26,           // particles the current sweep's transport handed on to the next sweep
   C_RPARITY = 27,             // which half of the resume buffer the current sweep reads
+  C_WORK = 28,                // sum of E / cutoff over the primary electrons, positrons and photons
   C_TAIL_STEPS = 30,          // particle-steps taken in walks
   C_STATS = 32,               // [ST_N] run statistics
   C_PTRIALS = 64,             // [PETITE_NPROC] candidates per process
@@ -873,11 +874,16 @@ struct DevStore {
   int64_t capacity;
 };
 
-__global__ void k_init_primaries(DevStore S, const PetitePrimary* prim, int64_t n, unsigned long long* n_muons) {
+__global__ __launch_bounds__(256) void k_init_primaries(DevStore S, const PetitePrimary* prim, int64_t n,
+                                                        double inv_cutoff, unsigned long long* counters) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const PetitePrimary p = i < n ? prim[i] : PetitePrimary{};
+  const bool muon = p.pid == 13 || p.pid == -13, em = p.pid == 11 || p.pid == -11 || p.pid == 22;
+  const unsigned long long v[2] = {muon ? 1ull : 0ull,
+                                   em ? (unsigned long long)fmin(fmax(p.E * inv_cutoff, 0.0), 1.0e9) : 0ull};
+  unsigned long long* const dst[2] = {counters + C_MUONS, counters + C_WORK};
+  block_stat_add<2>(v, dst);
   if (i >= n) return;
-  const PetitePrimary p = prim[i];
-  if ((p.pid == 13 || p.pid == -13) && n_muons) atomicAdd(n_muons, 1ull);
   S.p0[i] = make_float4((float)p.E, (float)p.px, (float)p.py, (float)p.pz);
   S.r0[i] = make_float4((float)p.x, (float)p.y, (float)p.z, (float)p.weight);
   S.pf[i] = S.p0[i];
@@ -2625,12 +2631,14 @@ int petite_run_showers(PetiteCtx* c, const PetitePrimary* prim, int64_t n, uint6
   HIP_TRY(hipMemsetAsync(c->drange, 0, 4 * sizeof(int64_t), s));
   const unsigned long long n0 = (unsigned long long)n;
   HIP_TRY(hipMemcpyAsync(ctr + C_STORE, &n0, sizeof(n0), hipMemcpyHostToDevice, s));
-  hipLaunchKernelGGL(k_init_primaries, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, S, prim, n, ctr + C_MUONS);
+  hipLaunchKernelGGL(k_init_primaries, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, S, prim, n,
+                     1.0 / std::max(c->dev.min_energy, 1.0e-3), ctr);
   HIP_TRY(hipGetLastError());
   // muon processes can only be requested when a primary is a muon
-  unsigned long long n_muons = 0;
-  HIP_TRY(hipMemcpyAsync(&n_muons, ctr + C_MUONS, sizeof(n_muons), hipMemcpyDeviceToHost, s));
+  unsigned long long h_prim[C_WORK - C_MUONS + 1];
+  HIP_TRY(hipMemcpyAsync(h_prim, ctr + C_MUONS, sizeof(h_prim), hipMemcpyDeviceToHost, s));
   HIP_TRY(hipStreamSynchronize(s));
+  const unsigned long long n_muons = h_prim[0], work = h_prim[C_WORK - C_MUONS];
   const bool muons = n_muons > 0;
   Requests R{c->req_slot, c->req_E, c->req_cap, c->req_count};
   DrawLaunch io{};
@@ -2686,12 +2694,14 @@ int petite_run_showers(PetiteCtx* c, const PetitePrimary* prim, int64_t n, uint6
   int64_t tail_launches = 0;
   double t_tail = 0.0;
   // Three waves per SIMD instead of two where the walk is long enough to be
-  // bound by its instructions rather than by its longest chain (ms with two /
-  // three; a store has room for about 1.7 times the records of lead, 4 times
-  // graphite's): lead, 10,000 mixed primaries (36e6 places) 22.3 / 23.6, 20,000
-  // 40 / 38, 40,000 73 / 69, 60,000 106 / 92; 8.5e6 records of graphite (34e6)
-  // 8.2 / 8.2; with muons 72 / 80
-  const bool wide = tail && !muons && store->capacity >= ((int64_t)1 << 26);
+  // bound by its instructions rather than by its longest chain: by the
+  // primaries' energy in cutoffs, which the records (0.7 per cutoff in graphite,
+  // 1.5 in lead) go with.  ms with two / three: lead, mixed primaries of 0.1-100
+  // GeV, 1.4e7 cutoffs 22.7 / 22.8, 2.9e7 40.0 / 37.2, 4.4e7 57.5 / 50.3; iron,
+  // photons of 1-60 GeV, 2.5e6 9.8 / 10.7, 1.4e7 22.5 / 21.7, 2.9e7 40.9 / 37.8;
+  // graphite, 10 GeV, 1e7 8.6 / 9.6, 2e7 12.7 / 13.1, 5e7 26.7 / 24.0; 90 GeV,
+  // 9e6 13.0 / 14.8, 3.6e7 23.4 / 24.3; a beam with muons 72 / 80
+  const bool wide = tail && !muons && work >= 25000000ull;
   const unsigned tail_blocks = blocks_for(c, wide ? tn.tail_waves * 3 / 2 : tn.tail_waves);
   if (c->timing) {
     while ((int)c->tev.size() < 4 * group + 2 * kTailGroup) {
