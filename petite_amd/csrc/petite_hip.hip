@@ -2775,8 +2775,13 @@ int petite_run_showers(PetiteCtx* c, const PetitePrimary* prim, int64_t n, uint6
       // host check: a launch whose inputs are empty ends at once
       const int ng = tail_launches == 0 ? 1 : kTailGroup;
       for (int g = 0; g < ng; ++g) {
-        const TailParams tp{c->tail_spill, front, back, tpar, tn.tail_depth, tail_limit(tn.tail_budget, tail_launches)};
-        hipLaunchKernelGGL(k_tail_setup, dim3(1), dim3(64), 0, s, ctr, c->drange, store->capacity, rcap, tp);
+        auto list = [&](int par) {
+          int32_t* const l = c->tail_spill + par * (front + back);
+          return WalkList{l, l + (front + back - 1), front, back};
+        };
+        const TailParams tp{list(tpar), list(tpar ^ 1), tpar, tn.tail_depth, tail_limit(tn.tail_budget, tail_launches)};
+        hipLaunchKernelGGL(k_tail_setup, dim3(1), dim3(64), 0, s, ctr, c->drange, store->capacity, rcap, tp,
+                           tail_launches == 0);
         HIP_TRY(hipGetLastError());
         if (c->timing) HIP_TRY(hipEventRecord(c->tev[4 * group + 2 * g], s));
         if (may_mark && tail_launches > 0) {
@@ -2788,8 +2793,6 @@ int petite_run_showers(PetiteCtx* c, const PetitePrimary* prim, int64_t n, uint6
                            c->dsig_lds, (const int64_t*)c->drange, ResumeBuf{c->dresume, rcap}, tp);
         HIP_TRY(hipGetLastError());
         if (c->timing) HIP_TRY(hipEventRecord(c->tev[4 * group + 2 * g + 1], s));
-        hipLaunchKernelGGL(k_tail_finish, dim3(1), dim3(64), 0, s, ctr, c->drange, store->capacity);
-        HIP_TRY(hipGetLastError());
         tpar ^= 1;
         ++tail_launches;
       }

@@ -56,10 +56,14 @@ constexpr int kMuonIters = 2048;
 constexpr int64_t kListFront = 3 << 20, kListMuons = 1 << 20;
 constexpr int32_t kMarked = (int32_t)0x80000000;  // bit of a particle's meta: waits, but is on no list
 
+// A spill list: its entries, muons from `end` down.
+struct WalkList {
+  int32_t *list, *end;
+  int64_t front, muons;  // room
+};
 struct TailParams {
-  int32_t* spill;   // [2][front + muons]: slots left for the next launch, muons from a list's end
-  int64_t front, muons;
-  int32_t par;      // list this launch reads (counted at C_SPILL + par, C_MUSPILL + par)
+  WalkList in, out;
+  int32_t par;      // list `in` (counted at C_SPILL + par, C_MUSPILL + par)
   int32_t depth;    // stack entries per wave (1..kTailMaxDepth)
   int32_t limit;    // iterations after which a wave starts no more particles
 };
@@ -73,10 +77,17 @@ struct WalkLds {
 };
 __device__ inline bool is_muon(int pid) { return pid == 13 || pid == -13; }
 
+// What walk_hand_on writes to, in LDS (its arguments held in scalar registers
+// throughout the walk cost 1 % of it).
+struct WalkOut {
+  WalkList to;
+  unsigned long long* count;
+  int32_t* meta;
+};
+
 // The slots v (>= 0) of the calling lanes at the end of the next launch's list,
 // muons from its back; those there is no room for are marked in the store (1).
-__device__ __noinline__ int walk_hand_on(int32_t* list, int64_t front, int64_t muons, unsigned long long* count,
-                                         int32_t* meta, int32_t v, bool muon) {
+__device__ __noinline__ int walk_hand_on(const WalkOut* out, int32_t v, bool muon) {
   const int lane = threadIdx.x & 63;
   const unsigned long long below = (1ull << lane) - 1ull;
   int marked = 0;
@@ -85,13 +96,14 @@ __device__ __noinline__ int walk_hand_on(int32_t* list, int64_t front, int64_t m
     const unsigned long long om = __ballot(mine);
     if (!om) continue;
     unsigned long long o = 0;
-    if (lane == 0) o = atomicAdd(count + (m ? C_MUSPILL - C_SPILL : 0), (unsigned long long)__popcll(om));
+    if (lane == 0) o = atomicAdd(out->count + (m ? C_MUSPILL - C_SPILL : 0), (unsigned long long)__popcll(om));
     o = shfl_u64(o, 0) + (unsigned long long)__popcll(om & below);
     if (mine) {
-      if ((int64_t)o < (m ? muons : front)) {
-        list[m ? front + muons - 1 - (int64_t)o : (int64_t)o] = v;
+      if ((int64_t)o < (m ? out->to.muons : out->to.front)) {
+        if (m) out->to.end[-(int64_t)o] = v;
+        else out->to.list[o] = v;
       } else {
-        atomicOr(meta + v, kMarked);
+        atomicOr(out->meta + v, kMarked);
         marked = 1;
       }
     }
@@ -190,10 +202,9 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
   const int64_t nres = RB.rec ? range[3] : 0;
   const ResumeRec* rin = RB.rec ? RB.rec + (int64_t)(counters[C_RPARITY] & 1ull) * RB.cap : nullptr;
   // a count past the list is cut to the list (the others are marked)
-  const int64_t list_cap = TPm.front + TPm.muons;
-  const int32_t* const spill_in = TPm.spill + TPm.par * list_cap;
-  const int64_t total = nres + n + min((int64_t)counters[C_SPILL + TPm.par], TPm.front);
-  const int64_t n_mu = min((int64_t)counters[C_MUSPILL + TPm.par], TPm.muons);
+  const int32_t* const spill_in = TPm.in.list;
+  const int64_t total = nres + n + min((int64_t)counters[C_SPILL + TPm.par], TPm.in.front);
+  const int64_t n_mu = min((int64_t)counters[C_MUSPILL + TPm.par], TPm.in.muons);
   // items per claim: an even share of every wave of the launch (of half of them
   // for muons), at most a lane's each
   const int64_t waves = (int64_t)gridDim.x * kWalkWaves;
@@ -207,7 +218,9 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
   HIP_DYNAMIC_SHARED(double, s_sig)
   __shared__ WalkLds s_walk[kWalkWaves];
   __shared__ WalkStats s_stat;
+  __shared__ WalkOut s_out;
   for (int i = threadIdx.x; i < T.lds_doubles; i += blockDim.x) s_sig[i] = sig_lds_src[i];
+  if (threadIdx.x == 0) s_out = WalkOut{TPm.out, counters + C_SPILL + (TPm.par ^ 1), S.meta};
   if (threadIdx.x < 8) s_stat.trials[threadIdx.x] = s_stat.draws[threadIdx.x] = s_stat.viol[threadIdx.x] = 0ull;
   __syncthreads();
   const LdsSigma L{s_sig};
@@ -250,7 +263,7 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
         if (lane == 0) c = atomicAdd(counters + C_MUCLAIM, (unsigned long long)share_mu);
         c = shfl_u64(c, 0);
         got = lane < share_mu && (int64_t)c + lane < n_mu;
-        if (got) slot = spill_in[list_cap - 1 - ((int64_t)c + lane)];
+        if (got) slot = TPm.in.end[-((int64_t)c + lane)];
         got_mu = (int64_t)c < n_mu;
         mu_exhausted = (int64_t)c + share_mu >= n_mu;
       }
@@ -548,8 +561,7 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
       if (v >= 0 && at < depth) W.stack[at] = v;
       const int32_t out = at >= depth ? v : -1;
       if (__ballot(out >= 0))
-        n_marked += walk_hand_on(TPm.spill + (TPm.par ^ 1) * list_cap, TPm.front, TPm.muons,
-                                 counters + C_SPILL + (TPm.par ^ 1), S.meta, out, t == 0 ? hmu : lmu);
+        n_marked += walk_hand_on(&s_out, out, t == 0 ? hmu : lmu);
       if (!muons) sp = min(depth, sp + __popcll(pm));
     }
     if (go_on) {
@@ -568,8 +580,6 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
   // ---- what the wave did not start goes to the next launch, and so do the
   // items no wave claimed (a handed-on one starts over there: its random
   // numbers are indexed by its substeps, so it ends the same)
-  int32_t* const spill_out = TPm.spill + (TPm.par ^ 1) * list_cap;
-  unsigned long long* const n_out = counters + C_SPILL + (TPm.par ^ 1);
   while (!exhausted) {
     unsigned long long c = 0;
     if (lane == 0) c = atomicAdd(counters + C_TRANSPORT, 64ull);
@@ -580,7 +590,7 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
     if (rr < total)
       v = rr < nres ? rin[rr].slot
                     : (rr < nres + n ? (int32_t)(first + (rr - nres)) : spill_in[rr - nres - n]);
-    n_marked += walk_hand_on(spill_out, TPm.front, TPm.muons, n_out, S.meta, v, v >= 0 && is_muon(S.pid[v]));
+    n_marked += walk_hand_on(&s_out, v, v >= 0 && is_muon(S.pid[v]));
   }
   while (!mu_exhausted) {
     unsigned long long c = 0;
@@ -588,10 +598,10 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
     c = shfl_u64(c, 0);
     mu_exhausted = (int64_t)c + 64 >= n_mu;
     const int64_t rr = (int64_t)c + lane;
-    n_marked += walk_hand_on(spill_out, TPm.front, TPm.muons, n_out, S.meta, rr < n_mu ? spill_in[list_cap - 1 - rr] : -1, true);
+    n_marked += walk_hand_on(&s_out, rr < n_mu ? TPm.in.end[-rr] : -1, true);
   }
   for (int e0 = 0; e0 < sp; e0 += 64)
-    n_marked += walk_hand_on(spill_out, TPm.front, TPm.muons, n_out, S.meta, e0 + lane < sp ? W.stack[e0 + lane] : -1, false);
+    n_marked += walk_hand_on(&s_out, e0 + lane < sp ? W.stack[e0 + lane] : -1, false);
   {
     unsigned long long* const st = counters + C_STATS;
     const unsigned long long v[7] = {steps, steps, n_fail, n_drop, n_ovf, n_marked, 0ull};
@@ -625,12 +635,14 @@ static int32_t tail_limit(int32_t budget, int64_t i) {
 // sweep, every store entry appended since the last sweep or tail launch (no
 // bound: the walk files no draw requests), and the previous launch's spills
 // (in the list of parity `par`, whose counts are cut to it; the other list is
-// cleared for this launch's).
+// cleared for this launch's).  Everything a tail launch appended was walked or
+// spilled, so the launches after the first start past it.
 __global__ void k_tail_setup(unsigned long long* ctr, int64_t* range, int64_t capacity, int64_t resume_cap,
-                             TailParams P) {
+                             TailParams P, bool first) {
   if (threadIdx.x == 0) {
     const int64_t big = (int64_t)1 << 62;
-    const SweepRange sr = sweep_range(range[2], (int64_t)ctr[C_STORE], capacity, big, (int64_t)ctr[C_YIELD_OUT],
+    const int64_t now = min((int64_t)ctr[C_STORE], capacity);
+    const SweepRange sr = sweep_range(first ? range[2] : now, now, capacity, big, (int64_t)ctr[C_YIELD_OUT],
                                       resume_cap);
     range[0] = sr.first;
     range[1] = sr.n;
@@ -639,8 +651,8 @@ __global__ void k_tail_setup(unsigned long long* ctr, int64_t* range, int64_t ca
     ctr[C_YIELD_OUT] = 0ull;
     ctr[C_RPARITY] ^= 1ull;
     ctr[C_TRANSPORT] = 0ull;
-    ctr[C_SPILL + P.par] = min(ctr[C_SPILL + P.par], (unsigned long long)P.front);
-    ctr[C_MUSPILL + P.par] = min(ctr[C_MUSPILL + P.par], (unsigned long long)P.muons);
+    ctr[C_SPILL + P.par] = min(ctr[C_SPILL + P.par], (unsigned long long)P.in.front);
+    ctr[C_MUSPILL + P.par] = min(ctr[C_MUSPILL + P.par], (unsigned long long)P.in.muons);
     ctr[C_SPILL + (P.par ^ 1)] = 0ull;
     ctr[C_MUSPILL + (P.par ^ 1)] = 0ull;
     ctr[C_MUCLAIM] = 0ull;
@@ -659,8 +671,7 @@ __global__ __launch_bounds__(256) void k_tail_gather(DevStore S, unsigned long l
   __shared__ unsigned long long s_base[2];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const unsigned long long below = (1ull << lane) - 1ull;
-  const int64_t cap = P.front + P.muons, n = min((int64_t)ctr[C_STORE], S.capacity);
-  int32_t* const list = P.spill + P.par * cap;
+  const int64_t n = min((int64_t)ctr[C_STORE], S.capacity);
   constexpr int64_t kWaveRun = 64 * kGatherRun, kBlockRun = 4 * kWaveRun;
   unsigned long long listed = 0ull;
   for (int64_t b0 = (int64_t)blockIdx.x * kBlockRun; b0 < n; b0 += (int64_t)gridDim.x * kBlockRun) {
@@ -701,8 +712,8 @@ __global__ __launch_bounds__(256) void k_tail_gather(DevStore S, unsigned long l
         const bool mine = marked && muon == (q == 1);
         const unsigned long long m = __ballot(mine);
         const int64_t at = (int64_t)(o[q] + __popcll(m & below));
-        if (mine && at < (q ? P.muons : P.front)) {
-          list[q ? cap - 1 - at : at] = (int32_t)i;
+        if (mine && at < (q ? P.in.muons : P.in.front)) {
+          *(q ? P.in.end - at : P.in.list + at) = (int32_t)i;
           S.meta[i] &= ~kMarked;
           ++listed;
         }
@@ -714,13 +725,4 @@ __global__ __launch_bounds__(256) void k_tail_gather(DevStore S, unsigned long l
   const unsigned long long v[1] = {0ull - listed};
   unsigned long long* const dst[1] = {ctr + C_MARKED};
   block_stat_add<1>(v, dst);
-}
-
-// After a tail launch: everything it appended was walked or spilled, so the
-// next launch (or sweep) starts past it.
-__global__ void k_tail_finish(unsigned long long* ctr, int64_t* range, int64_t capacity) {
-  if (threadIdx.x == 0) {
-    const int64_t now = (int64_t)ctr[C_STORE];
-    range[2] = now < capacity ? now : capacity;
-  }
 }
