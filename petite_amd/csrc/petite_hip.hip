@@ -2808,10 +2808,10 @@ int petite_run_showers(PetiteCtx* c, const PetitePrimary* prim, int64_t n, uint6
         }
       }
       if ((int64_t)h_store > store->capacity) break;
-      if (h_spill[tpar] == 0 && h_spill[kCtrLine + tpar] == 0) {  // every particle walked
-        if (h_spill[C_MARKED - C_SPILL]) return fail(PETITE_ERR_INTERNAL, "petite_run_showers: unlisted particles left");
-        break;
-      }
+      // (a launch may end all of a full list, and leave marked particles)
+      const bool marked = h_spill[C_MARKED - C_SPILL] != 0;
+      if (marked && !may_mark) return fail(PETITE_ERR_INTERNAL, "petite_run_showers: unlisted particles left");
+      if (h_spill[tpar] == 0 && h_spill[kCtrLine + tpar] == 0 && !marked) break;  // every particle walked
       if (tail_launches > 100000) return fail(PETITE_ERR_HIP, "petite_run_showers: tail launch runaway");
       continue;
     }

@@ -657,7 +657,8 @@ __global__ void k_tail_setup(unsigned long long* ctr, int64_t* range, int64_t ca
     ctr[C_MUSPILL + (P.par ^ 1)] = 0ull;
     ctr[C_MUCLAIM] = 0ull;
     ctr[C_GATHER] = ctr[C_MARKED];
-    if (sr.n > 0 || sr.nres > 0 || ctr[C_SPILL + P.par] > 0ull || ctr[C_MUSPILL + P.par] > 0ull) ctr[C_SWEEPS] += 1ull;
+    if (sr.n > 0 || sr.nres > 0 || (ctr[C_SPILL + P.par] | ctr[C_MUSPILL + P.par] | ctr[C_MARKED]) != 0ull)
+      ctr[C_SWEEPS] += 1ull;
   }
 }
 

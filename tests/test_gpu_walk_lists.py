@@ -98,6 +98,18 @@ def test_particles_past_a_lists_end(lead, name, parts):
     assert s["launches_transport"] == 0 and s["n_iterations"] > 2
 
 
+def test_marked_particles_beside_empty_lists(lead):
+    """Limits double: by the fifth launch, the last of a host check, a launch
+    ends a full list's photons below the cutoff, 131,072 lanes' at a time, and
+    the marked ones beside it are still to come."""
+    n = 9500000
+    prim = np.zeros(n, dtype=PRIMARY_DTYPE)
+    prim["pid"], prim["E"], prim["pz"], prim["weight"] = 22, 0.005, 0.005, 1.0
+    prim["sid"] = np.arange(n)
+    st, s = _same(lead, prim, dict(WALK, tail_budget=2), n)
+    assert s["n_particles"] == n and s["launches_tail"] > 5
+
+
 def test_restart_of_handed_on_particles(lead):
     """More handed-on particles than the launch has lanes: those that no wave
     claims go to the list and start over from their records."""
