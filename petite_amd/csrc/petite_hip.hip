@@ -1894,7 +1894,7 @@ struct PetiteCtx {
   int64_t* drange = nullptr;
   ResumeRec* dresume = nullptr;  // [2][resume_cap]
   int64_t resume_cap = 0;
-  int32_t* tail_spill = nullptr;  // [2][tail_spill_cap]: walk spill lists (at most 32 MB)
+  int32_t* tail_spill = nullptr;  // [2][tail_spill_cap]: walk spill lists (at most 72 MB)
   int64_t tail_spill_cap = 0;
   LongDraw* longs = nullptr;      // [kLongCap], contexts with a DarkAnn map
   std::vector<hipEvent_t> tev;
