@@ -3708,12 +3708,17 @@ int petite_detector_cut(const float* p, const float* r, int64_t n, const double*
   for (int d = 0; d < n_det; ++d) D.z[d] = det_z[d];
   if (wsum) HIP_TRY(hipMemsetAsync(wsum, 0, (size_t)(n_det + 1) * sizeof(double), s));
   if (n > 0) {
-    // Eight records a thread where that leaves 256 blocks, at most 1,024
-    // blocks: their sums are added one after another, planes + 1 atomics each
-    // (1e6 records at 12 planes 53, 56, 69 and 93 us a call with 512 to 4,096
-    // blocks; 3e7 at 3 planes 308, 253, 275 and 273).
-    const int64_t blocks =
-        std::min<int64_t>(std::min<int64_t>((n + 255) / 256, 1024), std::max<int64_t>(256, (n + 2047) / 2048));
+    // With sums in registers, eight records a thread where that leaves 256
+    // blocks, at most 1,024 blocks: their sums are added one after another,
+    // planes + 1 atomics each (host-timed with the call, alone: 1e6 records at 12
+    // planes 53, 56, 69 and 93 us with 512 to 4,096 blocks; 3e7 at 3 planes 308,
+    // 253, 275 and 273).  A thread's passes with a reduction each want more
+    // blocks (40 planes, with the blocks of the other kernels / up to 4,096:
+    // 1e5 records 61 / 47 us, 5e7 4.55 / 4.11 ms).
+    const int64_t most = (n + 255) / 256;
+    const int64_t blocks = n_det <= kRegPlanes[1]
+                               ? std::min<int64_t>(std::min<int64_t>(most, 1024), std::max<int64_t>(256, (n + 2047) / 2048))
+                               : std::min<int64_t>(most, 4096);
     auto* const f = n_det <= kRegPlanes[0] ? k_detector_cut<kRegPlanes[0]>
                                            : (n_det <= kRegPlanes[1] ? k_detector_cut<kRegPlanes[1]> : k_detector_cut<0>);
     hipLaunchKernelGGL(f, dim3((unsigned)blocks), dim3(256), 0, s, (const float4*)p, (const float4*)r, n, D, mask, wsum);
