@@ -55,18 +55,20 @@ def measured_valu(kernel):
     return dict(t, source="profiles/valu.json")
 
 
-def measured_traffic(kernel, alg_bytes_per_launch):
-    """HBM bytes per launch of `kernel` from the committed rocprofv3 FETCH_SIZE /
+def measured_traffic(kernel, alg_bytes_per_launch, alg_bytes_per_step):
+    """HBM bytes of `kernel` per launch (per step of the walk, whose launches
+    are as uneven as their count) from the committed rocprofv3 FETCH_SIZE /
     WRITE_SIZE measurement of this workload (profiles/traffic.json, made by the
-    command it records), with the algorithmic bytes per launch beside it."""
+    command it records), with the algorithmic bytes beside it."""
     path = os.path.join(ROOT, "profiles", "traffic.json")
     try:
         with open(path) as f:
             t = json.load(f)[kernel]
     except (OSError, KeyError, ValueError):
         return None
-    return {"bytes_per_launch": t["bytes_per_launch"], "fetch_bytes": t["fetch_bytes"],
-            "write_bytes": t["write_bytes"], "over_algorithmic": t["bytes_per_launch"] / alg_bytes_per_launch,
+    per = "bytes_per_step" if "bytes_per_step" in t else "bytes_per_launch"
+    return {per: t[per], "fetch_bytes": t["fetch_bytes"], "write_bytes": t["write_bytes"],
+            "over_algorithmic": t[per] / (alg_bytes_per_step if per == "bytes_per_step" else alg_bytes_per_launch),
             "source": "profiles/traffic.json"}
 
 
@@ -297,7 +299,7 @@ def main():
     print(f"bench: {len(prim)} primaries, lead, cutoff {CUTOFF}", file=sys.stderr, flush=True)
     for w in range(args.warmup):
         b = sh.generate_showers(prim, seed=SEED)
-        print(f"warmup {w}: {b.n} particles, {b.stats['n_iterations']} sweeps", file=sys.stderr, flush=True)
+        print(f"warmup {w}: {b.n} particles, {b.stats['n_iterations']} sweeps and walk launches", file=sys.stderr, flush=True)
         del b
     torch.cuda.synchronize()
     totals = {"steps": 0, "particles": 0, "draws": 0, "trials": 0, "tail_steps": 0}
@@ -332,7 +334,8 @@ def main():
 
     # roofline of the kernel that advances the particles: k_transport, or the
     # walk where it takes the batch whole (the draw kernels of the six
-    # processes run side by side; a walk draws and emits as well)
+    # processes run side by side; a walk draws and emits as well, in the time
+    # that its particle-steps are divided by)
     dom, dom_kernel = ("transport", "k_transport") if kern["transport"][1] else ("tail", "k_tail")
     t_dom = kern[dom][0] / 1e3
     alg = B_STEP * (totals["tail_steps"] if dom == "tail" else totals["steps"] - totals["tail_steps"])
@@ -340,9 +343,10 @@ def main():
     roof = {"bound": "hbm", "achieved": ach, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": ach / HBM_PEAK_GBS,
             "traffic": None, "kernel": dom_kernel, "per_unit": "128 B per particle-step"}
     roof["avg_launch_ms"] = kern[dom][0] / max(kern[dom][1], 1)
-    roof["traffic"] = measured_traffic(roof["kernel"], alg / max(kern[dom][1], 1))
-    # the bound that holds is VALU issue (HBM traffic is a fifth of the
-    # algorithmic bytes: a particle stays in registers)
+    roof["traffic"] = measured_traffic(roof["kernel"], alg / max(kern[dom][1], 1), alg / K)
+    # the bound that holds is VALU issue (a particle stays in registers: HBM
+    # traffic is a fifth of the algorithmic bytes of k_transport, two fifths of
+    # the walk's)
     roof["valu"] = measured_valu(roof["kernel"])
     kernels = {k: {"ms_total": v[0] / K, "launches": v[1] // K} for k, v in kern.items()}
 
@@ -586,7 +590,7 @@ YIELD_N, YIELD_MAT = 50_000, "lead"
 YIELD_MASSES = np.geomspace(1e-3, 0.1, 32)
 # algorithmic bytes: the dark selection reads a 64-byte SM record and the
 # emission writes a 48-byte vector record; the yield pass reads pid, E0 and
-# the weight (12 bytes) of every record once per batch of 16 masses
+# the weight (12 bytes) of every record once per batch of 32 masses
 B_DARK_SM, B_DARK_V, B_YIELD = 64, 48, 12
 
 
@@ -698,7 +702,7 @@ def bench_yield(reps=5):
     fd = yield_finite_differences(model, rec, YIELD_MASSES)
     fd_err = float(np.max(np.abs(fd - dY) / np.maximum(np.abs(dY), 1e-300)))
     inner = YIELD_MASSES
-    passes = math.ceil(len(YIELD_MASSES) / 16)
+    passes = math.ceil(len(YIELD_MASSES) / 32)
     alg = B_YIELD * rec.n * passes
     out = {"workload": f"{YIELD_N} e- showers, E log-uniform [1,20] GeV, {YIELD_MAT}, cutoff {CUTOFF} GeV; "
                        f"32 m_V in [1,100] MeV; eps^2 enters linearly",
@@ -707,7 +711,7 @@ def bench_yield(reps=5):
            "scans_per_s": 1.0 / t_g, "grad_evals_per_s": len(YIELD_MASSES) / t_g,
            "fd_max_rel_err": fd_err, "fd_points": len(inner),
            "roofline": {"bound": "hbm", "achieved": alg / t_g / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                        "per_unit": "12 B per record per 16-mass pass (host-timed, includes launch and readback)"},
+                        "per_unit": "12 B per record per 32-mass pass (host-timed, includes launch and readback)"},
            "yield_per_eps2_at_10MeV": float(np.interp(0.01, YIELD_MASSES, Y))}
     return out, ds, rec, model
 

@@ -107,7 +107,7 @@ typedef struct {
   int64_t n_trials;     /* candidates evaluated */
   int64_t n_maxf_viol;  /* accepted candidates with J*f > max_F */
   int64_t n_no_sample;  /* draws that hit max_trials */
-  int64_t n_iterations; /* generation sweeps */
+  int64_t n_iterations; /* sweeps and walk launches that had particles to advance */
   int64_t n_dropped;    /* children below min_energy */
   /* kernel times measured with HIP events on the run's stream (0 unless
    * timing is enabled with petite_set_timing) */

@@ -18,7 +18,7 @@ FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     # float64 constants stay in the loops that use them: hoisted into scalar
     # registers they spill to vector lanes and come back by v_readlane (k_tail
-    # 341 scalar and 22 vector spills -> 118 and none, k_transport 121 -> 78
+    # 341 scalar and 22 vector spills -> 113 and none, k_transport 121 -> 78
     # vector registers; walk, draws and yields 2-5 % faster)
     "-mllvm", "-disable-machine-licm",
     "-I", os.path.join(ROOT, "include"), "-I", os.path.join(HERE, "csrc"),

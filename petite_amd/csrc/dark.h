@@ -585,8 +585,8 @@ __global__ __launch_bounds__(kMesonBlock) void k_meson_decay(DevTables T, Petite
 // and a short record still fills the chip.  The blocks' sums go to rows of
 // their own and one kernel adds those (atomics of every wave on the points'
 // sums, all in four cache lines, were served one after another).  19e6 records
-// x 32 points with gradients: 3.4 ms (interpolation 2.3, bound 0.74, lists
-// 0.32); two scans of mixed species with unpacked tables took 10.6 ms.
+// x 32 points with gradients: 3.0 ms (interpolation 1.96, bound 0.75, lists
+// 0.31); two scans of mixed species with unpacked tables took 10.6 ms.
 constexpr int kYieldBatch = 32;   // points of a pass
 constexpr int kYieldGroup = 8;     // points of a block of k_dark_yield
 constexpr int kBoundGroup = 4;    // points of a block of k_bound_yield

@@ -30,11 +30,13 @@
 // every second wave of the launch, so that the other half of them take the
 // list's front; alone in its wave while there are fewer muons than that.
 //
-// What bounds it: the latency of a substep (~600 dependent instructions) and of
-// a draw phase, at 2 waves per SIMD; with muons the longest of them (32,000
-// substeps and 2,400 phases, 70 ms alone).  1,000 electrons of 10 GeV in
-// graphite 5.4 ms a run, 40,000 mixed primaries in lead 73 ms.  A 400 GeV beam
-// of 2,000 in lead, half of them muons: 84 ms; 137 ms with each muon among the
+// What bounds it: for small batches the latency of a substep (~600 dependent
+// instructions) and of a draw phase (two waves per SIMD at most; VALU issue 30 %
+// for 1,000 electrons of 10 GeV in graphite, 5.2 ms a run); for large ones VALU
+// issue (74 % of the peak at 100,000 mixed primaries in lead, 148 ms, 40,000 in
+// 71 ms, both at three waves per SIMD at most); with muons the longest of them
+// (32,000 substeps and 2,400 phases, 70 ms alone).  A 400 GeV beam
+// of 2,000 in lead, half of them muons: 85 ms; 137 ms with each muon among the
 // particles of its own subtree; 264 ms (170 ms of that in the walk) with one
 // particle per wave, every lane computing the same transport, and two atomics
 // per draw on one line of per-process counters.
@@ -193,7 +195,7 @@ __device__ inline void walk_draws(const DevTables& T, uint64_t seed, bool mine, 
 // sweep handed on (live state in its resume records), the store slots
 // [first, first + n), then the previous launch's spills.  range: the tail
 // setup's {first, n, end, nres}.
-// EU: waves per SIMD the registers are held to (168 of them and 25 spills for
+// EU: waves per SIMD the registers are held to (168 of them and 23 spills for
 // three; the run chooses).
 constexpr int kWalkWaves = 4;  // waves per block
 template <int EU>
