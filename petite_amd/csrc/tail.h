@@ -81,17 +81,18 @@ struct WalkLds {
 };
 __device__ inline bool is_muon(int pid) { return pid == 13 || pid == -13; }
 
-// What walk_hand_on writes to, in LDS (its arguments held in scalar registers
-// throughout the walk cost 1 % of it).
+// Where walk_hand_on writes, in LDS: held in scalar registers throughout the
+// walk its arguments cost 1 % of it.  The counter's address stays an argument,
+// so that the atomic goes out at once (read from LDS first, 1 % of a muon beam).
 struct WalkOut {
   WalkList to;
-  unsigned long long* count;
   int32_t* meta;
 };
+typedef __attribute__((address_space(3))) const WalkOut LdsWalkOut;
 
 // The slots v (>= 0) of the calling lanes at the end of the next launch's list,
 // muons from its back; those there is no room for are marked in the store (1).
-__device__ __noinline__ int walk_hand_on(const WalkOut* out, int32_t v, bool muon) {
+__device__ __noinline__ int walk_hand_on(LdsWalkOut* out, unsigned long long* count, int32_t v, bool muon) {
   const int lane = threadIdx.x & 63;
   const unsigned long long below = (1ull << lane) - 1ull;
   int marked = 0;
@@ -100,12 +101,13 @@ __device__ __noinline__ int walk_hand_on(const WalkOut* out, int32_t v, bool muo
     const unsigned long long om = __ballot(mine);
     if (!om) continue;
     unsigned long long o = 0;
-    if (lane == 0) o = atomicAdd(out->count + (m ? C_MUSPILL - C_SPILL : 0), (unsigned long long)__popcll(om));
+    if (lane == 0) o = atomicAdd(count + (m ? C_MUSPILL - C_SPILL : 0), (unsigned long long)__popcll(om));
+    int32_t* const at = m ? out->to.end : out->to.list;
+    const int64_t room = m ? out->to.muons : out->to.front;
     o = shfl_u64(o, 0) + (unsigned long long)__popcll(om & below);
     if (mine) {
-      if ((int64_t)o < (m ? out->to.muons : out->to.front)) {
-        if (m) out->to.end[-(int64_t)o] = v;
-        else out->to.list[o] = v;
+      if ((int64_t)o < room) {
+        at[m ? -(int64_t)o : (int64_t)o] = v;
       } else {
         atomicOr(out->meta + v, kMarked);
         marked = 1;
@@ -224,10 +226,11 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
   __shared__ WalkStats s_stat;
   __shared__ WalkOut s_out;
   for (int i = threadIdx.x; i < T.lds_doubles; i += blockDim.x) s_sig[i] = sig_lds_src[i];
-  if (threadIdx.x == 0) s_out = WalkOut{TPm.out, counters + C_SPILL + (TPm.par ^ 1), S.meta};
+  if (threadIdx.x == 0) s_out = WalkOut{TPm.out, S.meta};
   if (threadIdx.x < 8) s_stat.trials[threadIdx.x] = s_stat.draws[threadIdx.x] = s_stat.viol[threadIdx.x] = 0ull;
   __syncthreads();
   const LdsSigma L{s_sig};
+  LdsWalkOut* const to_out = (LdsWalkOut*)&s_out;
   const int lane = threadIdx.x & 63;
   const unsigned long long below = (1ull << lane) - 1ull;
   WalkLds& W = s_walk[threadIdx.x >> 6];
@@ -565,7 +568,7 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
       if (v >= 0 && at < depth) W.stack[at] = v;
       const int32_t out = at >= depth ? v : -1;
       if (__ballot(out >= 0))
-        n_marked += walk_hand_on(&s_out, out, t == 0 ? hmu : lmu);
+        n_marked += walk_hand_on(to_out, counters + C_SPILL + (TPm.par ^ 1), out, t == 0 ? hmu : lmu);
       if (!muons) sp = min(depth, sp + __popcll(pm));
     }
     if (go_on) {
@@ -594,7 +597,7 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
     if (rr < total)
       v = rr < nres ? rin[rr].slot
                     : (rr < nres + n ? (int32_t)(first + (rr - nres)) : spill_in[rr - nres - n]);
-    n_marked += walk_hand_on(&s_out, v, v >= 0 && is_muon(S.pid[v]));
+    n_marked += walk_hand_on(to_out, counters + C_SPILL + (TPm.par ^ 1), v, v >= 0 && is_muon(S.pid[v]));
   }
   while (!mu_exhausted) {
     unsigned long long c = 0;
@@ -602,10 +605,10 @@ __global__ __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu
     c = shfl_u64(c, 0);
     mu_exhausted = (int64_t)c + 64 >= n_mu;
     const int64_t rr = (int64_t)c + lane;
-    n_marked += walk_hand_on(&s_out, rr < n_mu ? TPm.in.end[-rr] : -1, true);
+    n_marked += walk_hand_on(to_out, counters + C_SPILL + (TPm.par ^ 1), rr < n_mu ? TPm.in.end[-rr] : -1, true);
   }
   for (int e0 = 0; e0 < sp; e0 += 64)
-    n_marked += walk_hand_on(&s_out, e0 + lane < sp ? W.stack[e0 + lane] : -1, false);
+    n_marked += walk_hand_on(to_out, counters + C_SPILL + (TPm.par ^ 1), e0 + lane < sp ? W.stack[e0 + lane] : -1, false);
   {
     unsigned long long* const st = counters + C_STATS;
     const unsigned long long v[7] = {steps, steps, n_fail, n_drop, n_ovf, n_marked, 0ull};
